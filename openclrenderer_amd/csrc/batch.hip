@@ -155,7 +155,7 @@ static int ensure_entries(ocr_batch* b) {
   if (b->ent.cnt) (void)hipFree(b->ent.cnt);
   b->ent = CoverEntries{};
   hipError_t e = hipMalloc((void**)&b->ent.ent, sizeof(uint2) * (size_t)kEntCap * want);
-  if (e == hipSuccess) e = hipMalloc((void**)&b->ent.cnt, sizeof(uint32_t) * (size_t)want);
+  if (e == hipSuccess) e = hipMalloc((void**)&b->ent.cnt, sizeof(uint32_t) * (size_t)std::max(want, kEntMinCounts));
   if (e != hipSuccess) {
     (void)hipGetLastError();
     if (b->ent.ent) (void)hipFree(b->ent.ent);

@@ -174,11 +174,16 @@ constexpr uint32_t kBoxRect = 1u << 31;
 // room for the other renders' shading beside the raster passes (1080p/1M
 // frame 0.183 -> 0.178 ms, though the depth pass alone takes 84 us, not 75;
 // 512 and 4096 measured slower).
-constexpr uint32_t kChunk = 64 * 32;   // raster samples per wavefront work item
+constexpr int kChunkLog2 = 11;
+constexpr uint32_t kChunk = 1u << kChunkLog2;   // raster samples per wavefront work item, at most
 constexpr uint32_t kEntCap = kChunk / 2;
+// Passes of fewer samples use smaller chunks (chunk_log2), with room for as
+// many entries per sample: chunks * kChunk / size of them have entries, and
+// at most kEntMinCounts exist.
+constexpr uint32_t kEntMinCounts = 8192 + 64;
 struct CoverEntries {
   uint2* ent;         // chunks x kEntCap
-  uint32_t* cnt;      // per chunk
+  uint32_t* cnt;      // per chunk, at least kEntMinCounts
   uint32_t chunks;
 };
 

@@ -233,7 +233,7 @@ int frame_alloc_set(Frame* f, int b) {
       (rc = dev_alloc(&o.rgba, npix, "rgba")) || (rc = dev_alloc(&o.normals, npix, "normals")) ||
       (rc = dev_alloc(&o.counters, kCounterWords, "counters")) ||
       (rc = dev_alloc(&o.ent.ent, (size_t)chunks * kEntCap, "covered-sample entries")) ||
-      (rc = dev_alloc(&o.ent.cnt, chunks, "covered-sample counts")))
+      (rc = dev_alloc(&o.ent.cnt, std::max(chunks, kEntMinCounts), "covered-sample counts")))
     return rc;
   o.ent.chunks = chunks;
   OCR_HIP_CHECK(hipMemset(o.counters, 0, 4 * kCounterWords));

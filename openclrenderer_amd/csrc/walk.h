@@ -9,14 +9,28 @@
 namespace ocr {
 
 // ------------------------------------------------------------ wave helpers
+// Inclusive sum over the wavefront's lanes, called with every lane active.
+// Six data-parallel adds in registers: within rows of 16 lanes (row_shr 1, 2,
+// 4, 8), then the last lane of each row onto the next row (row_bcast:15 into
+// rows 1 and 3) and lane 31 onto rows 2 and 3 (row_bcast:31).  Lanes without
+// a source add 0.  A scan through the LDS crossbar (one ds_bpermute and a
+// select per step, each waiting for the last) takes 24 instructions and six
+// LDS round trips; the shadow prearrange, with four to six scans per 64
+// pieces, is bound by their issue and latency.
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
-  const int lane = threadIdx.x & (kWave - 1);
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    uint32_t t = __shfl_up(v, d, kWave);
-    if (lane >= d) v += t;
-  }
+  constexpr int kRowShr = 0x110, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kRowShr + 1, 0xF, 0xF, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kRowShr + 2, 0xF, 0xF, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kRowShr + 4, 0xF, 0xF, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kRowShr + 8, 0xF, 0xF, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kRowBcast15, 0xA, 0xF, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kRowBcast31, 0xC, 0xF, false);
   return v;
+}
+
+// The wavefront's sum, from its inclusive scan (uniform).
+__device__ __forceinline__ uint32_t wave_total(uint32_t incl) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
 }
 
 // The walk's row of sample q: floor(mad(q, 1/width, min_y)) (cl2.cl:5083).
