@@ -90,7 +90,7 @@ static PassArgs batch_pass(const ocr_batch* b) {
   a.unshadowed = 1u;
   for (const Scene* s : b->scenes)
     if (s->n_shadow) a.unshadowed = 0u;
-  a.lists = make_lists(b->cuts, b->counters, b->cap_cut);
+  a.lists = make_lists(b->cuts, b->counters, b->cap_cut, b->tune.raster_tile ? 1u : list_parts(b->tri_slots, b->cap_cut));
   a.lists.ent = b->ent;
   if (b->tune.raster_tile) a.lists.tb = b->tb;
   return a;
@@ -167,8 +167,11 @@ static int ensure_entries(ocr_batch* b) {
 }
 
 static int ensure_lists(ocr_batch* b) {
-  uint64_t want_cut = std::min<uint64_t>(b->sum_tris * 2 + 64, 0xFFFFFFF0ull);
-  if (b->cuts && b->cap_cut >= want_cut) {
+  // a batch reserved for serving keeps its list while the records fit, in
+  // fewer partitions if need be
+  const uint64_t want_cut = std::min<uint64_t>(list_capacity(b->tri_slots), 0xFFFFFFF0ull);
+  const uint64_t need = b->ent_fixed ? std::min<uint64_t>(b->sum_tris * 2 + 64, 0xFFFFFFF0ull) : want_cut;
+  if (b->cuts && b->cap_cut >= need) {
     const int rc = ensure_entries(b);
     return rc ? rc : ensure_bins_of(b);
   }
@@ -193,10 +196,14 @@ static int ensure_lists(ocr_batch* b) {
 int ocr::batch_reserve(ocr_batch* b, uint64_t sum_tris) {
   OCR_HIP_CHECK(hipSetDevice(b->ctx->device));
   const uint64_t keep = b->sum_tris;
+  const uint32_t keep_slots = b->tri_slots;
   b->sum_tris = sum_tris;
+  // every view's triangle range is rounded up to whole blocks
+  b->tri_slots = (uint32_t)std::min<uint64_t>(sum_tris + (uint64_t)kPreThreads * b->max_views, 0x7FFFFFFFull);
   b->ent_fixed = true;
   const int rc = ensure_lists(b);
   b->sum_tris = keep;
+  b->tri_slots = keep_slots;
   return rc;
 }
 
@@ -384,8 +391,8 @@ int ocr_batch_create(ocr_ctx* ctx, uint32_t max_views, ocr_batch** out) {
   b->max_views = max_views;
   hipError_t e = hipMalloc((void**)&b->d_views, sizeof(DevView) * max_views);
   if (e == hipSuccess) e = hipMalloc((void**)&b->d_scenes, sizeof(DevScene) * max_views);
-  if (e == hipSuccess) e = hipMalloc((void**)&b->counters, 4 * kCounterWords);
-  if (e == hipSuccess) e = hipMemset(b->counters, 0, 4 * kCounterWords);
+  if (e == hipSuccess) e = hipMalloc((void**)&b->counters, 4 * kListCounterWords);
+  if (e == hipSuccess) e = hipMemset(b->counters, 0, 4 * kListCounterWords);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->capture_stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipHostMalloc((void**)&b->ds_host, sizeof(DevScene) * max_views);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&b->ds_done, hipEventDisableTiming);
@@ -610,7 +617,7 @@ int ocr_batch_get_stats(ocr_batch* b, void* stream, ocr_frame_stats* out) {
     for (uint32_t k = 0; k < group_count(b); k++) {
       uint32_t g[kCounterWords];
       OCR_HIP_CHECK(hipMemcpy(g, b->subs[k]->counters, sizeof(g), hipMemcpyDeviceToHost));
-      c[kPacked + 1] += g[kPacked + 1];
+      c[kCutCount] += g[kCutCount];
       c[kFragCount] += g[kFragCount];
       c[kOverflow] |= g[kOverflow];
       // a group whose bins overflowed grows them for its next render
@@ -623,7 +630,7 @@ int ocr_batch_get_stats(ocr_batch* b, void* stream, ocr_frame_stats* out) {
       b->want_bin = (uint32_t)std::min<uint64_t>((uint64_t)c[kBinTotal] + c[kBinTotal] / 4 + 64, 0xFFFFFFF0ull);
   }
   memset(out, 0, sizeof(*out));
-  out->n_cut = c[kPacked + 1];
+  out->n_cut = c[kCutCount];
   out->n_frag = c[kFragCount];
   out->overflow = c[kOverflow] ? 1u : 0u;
   out->n_profiled = (uint32_t)b->n_profiled;

@@ -189,18 +189,21 @@ struct CoverEntries {
 
 // The cut list and counters shared by the views of one render.  One
 // allocation of 2 * cap_cut records holds the CutTri records followed by
-// their RasterTri setups.  tb.bin is null unless the render is tiled.
+// their RasterTri setups.  The list is `parts` partitions (a power of two up
+// to kListParts) of cap_cut / parts records, each with a sample space and a
+// counter of its own; prearrange block b appends to partition b mod parts.
+// tb.bin is null unless the render is tiled (one partition).
 struct Lists {
   CutTri* cuts;
   RasterTri* rast;
   uint32_t* counters;
   uint32_t cap_cut;
-  uint32_t count_frags;   // keep the reference's fragment count (statistics)
+  uint32_t parts;
   TileBins tb;
   CoverEntries ent;
 };
-inline Lists make_lists(CutTri* cuts, uint32_t* counters, uint32_t cap_cut, bool count_frags = true) {
-  return Lists{cuts, reinterpret_cast<RasterTri*>(cuts + cap_cut), counters, cap_cut, count_frags ? 1u : 0u};
+inline Lists make_lists(CutTri* cuts, uint32_t* counters, uint32_t cap_cut, uint32_t parts) {
+  return Lists{cuts, reinterpret_cast<RasterTri*>(cuts + cap_cut), counters, cap_cut, parts};
 }
 constexpr uint32_t kMaxViews = 4096;
 
@@ -224,29 +227,47 @@ __host__ __device__ inline uint32_t view_tiles(uint32_t w, uint32_t h, uint32_t 
   return ((w + tw - 1) / tw) * ((h + th - 1) / th);
 }
 
-// Device counters of one render: words 0-1 hold a u64 whose high half is the
-// cut-triangle count and low half the raster sample count.  Every block of
-// prearrange adds to it; atomics on one cache line serialise (about 12 ns
-// each), so the fragment statistic lives on a line of its own.
+// Device counters of one render.  Atomics on one cache line serialise (about
+// 12 ns each), so what every block of prearrange adds to lies on lines of its
+// own: the statistics here, the partitions' counters behind.
 enum Counter : int {
-  kPacked = 0,
   kOverflow = 2,
-  kValidEnd = 16,          // shadow passes: u64, end of the list's valid prefix, byte 64
-  kFragCount = 32,         // reference fragments (statistics), byte 128
+  kFragCount = 32,         // reference fragments and cut pieces (statistics; one u64), byte 128
+  kCutCount = 33,
   kBinTotal = 48,          // tiled path: bin entries the render needed, byte 192
   kCounterWords = 64,
 };
-// Shadow-pass lists are split into kShadowParts partitions (one per lane of
-// the raster pass's wavefronts), each with its own record range, sample
-// space, packed counter and valid-prefix word on a 128-byte line of its own
-// after the render counters: prearrange block b allocates in partition
-// b mod kShadowParts.  (One counter for the whole pass serialised the
-// prearrange's wavefront allocations on one address.)
-constexpr uint32_t kShadowParts = 64;
+// Lists are split into up to kListParts partitions (one per lane of the raster
+// passes' wavefronts), each with its own record range, sample space, packed
+// counter (records << 32 | samples; shadow lists << kShadowSampleBits) and
+// valid-prefix word (shadow lists) on a 128-byte line of its own after the
+// render counters.  With one counter for the whole pass the appends serialise
+// on its address.
+constexpr uint32_t kListParts = 64;
 constexpr int kPartLineWords = 32;
-constexpr int kShadowCounterWords = kCounterWords + (int)kShadowParts * kPartLineWords;
+constexpr int kListCounterWords = kCounterWords + (int)kListParts * kPartLineWords;
 // partition p: packed counter (u64) at word kPartWord(p), valid prefix at +2
 __host__ __device__ constexpr int kPartWord(uint32_t p) { return kCounterWords + (int)p * kPartLineWords; }
+// Triangles per prearrange block, the unit of the partitions.
+constexpr uint32_t kPreThreads = 256;
+// Partitions of a camera list of cap_cut records for tri_slots triangle
+// slots: at most one per 32 blocks (32 appends to one address take 0.4 us),
+// and only as many as leave each room for two records per slot of its
+// blocks, so that a list sized by list_capacity never overflows.  A list of
+// one partition overflows only when the records do not fit.
+inline uint32_t list_parts(uint32_t tri_slots, uint32_t cap_cut) {
+  const uint64_t blocks = ((uint64_t)tri_slots + kPreThreads - 1) / kPreThreads;
+  uint32_t p = 1;
+  while (p < kListParts && (uint64_t)p * 64 <= blocks &&
+         (blocks + 2 * p - 1) / (2 * p) * 2 * kPreThreads <= cap_cut / (2 * p))
+    p *= 2;
+  return p;
+}
+// Records that a list for tri_slots triangle slots needs at most.
+inline uint64_t list_capacity(uint64_t tri_slots) {
+  const uint64_t blocks = (tri_slots + kPreThreads - 1) / kPreThreads;
+  return (blocks + (blocks >= 64 ? kListParts : 1)) * 2 * kPreThreads;
+}
 // Bits of the overflow word: the cut list is full / the sample space is full.
 constexpr uint32_t kOverflowCuts = 1u, kOverflowSamples = 2u, kOverflowBins = 4u;
 // Raster samples per render, and per cut triangle.  Frames and shadow faces
@@ -258,8 +279,8 @@ constexpr uint32_t kMaxTriSamples = (1u << 24) - 1;
 constexpr uint64_t kMaxTargetPixels = 16000000ull;
 
 // Shadow-pass lists pack each partition's counter as (records << 40 |
-// samples): a wavefront allocates at most 2^25 samples at once (a lane's two
-// pieces hold fewer than 2^25) and only if the counter it loads first is
+// samples): a wavefront allocates at most 2^25 samples at once (a lane's
+// piece holds fewer than 2^24) and only if the counter it loads first is
 // below the limits, and at most 8192 wavefronts are resident, so the sample
 // part stays below 2^30 + 2^13 * 2^25 < 2^40 and the record part below
 // kShadowMaxRecords + 2^13 * 128 < 2^24.
@@ -438,6 +459,7 @@ struct Frame {
   static constexpr int kEvents = 7;       // pass boundaries, and the shading pass's start
   static constexpr int kRing = 1024;      // renders averaged per profiling window
   std::vector<hipEvent_t> ev;             // kRing x kEvents, created on first use
+  std::vector<uint8_t> ev_tiled;          // kRing: whether the render was tiled
   int n_profiled = 0;
   bool rendered = false;
   // A frame is written either by ocr_render or by batches, never both: a
@@ -510,7 +532,6 @@ hipError_t launch_atlas_upload(const Atlas& a, uint32_t tid, const uint8_t* src,
 hipError_t launch_mip(const Atlas& a, uint32_t src_id, uint32_t dst_id, uint32_t gw, uint32_t gh,
                       hipStream_t s);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t value, size_t n, hipStream_t s);
-hipError_t launch_zero_counters(uint32_t* counters, hipStream_t s);
 hipError_t launch_light_prep(const ocr_light* lights, uint32_t n, float* lin, hipStream_t s);
 hipError_t launch_world(Scene* sc, hipStream_t s);
 

@@ -32,73 +32,92 @@
 
 namespace ocr {
 
-// Prearrange blocks: one triangle per work item.  Cut records and sample
-// ranges are allocated once per block (one 64-bit atomicAdd on the packed
-// counter (cuts << 32 | samples) per block): every wavefront of the render
-// appending to one counter would serialise on that address (~12 ns per
-// same-address atomic).  The camera pass uses 512 work items: the next
-// render's prearrange runs beside the current render's shading, and a
-// 512-item block (8 wavefronts) fits on a CU beside shading wavefronts where
-// a 1024-item one waits for the CU to drain (measured: 4083-4094 vs
-// 4019-4024 frames/s on the 1080p, 1 M-triangle frame; 256 items pays for
-// twice the atomics, 57 vs 40 us alone).  The shadow prearrange (104 VGPRs)
-// also uses 512: two blocks per CU hide each other's loads, barriers and
-// allocation atomic (16-light shadow pass over 4 M triangles 5.09 -> 4.82 ms).
-constexpr int kPreThreads = 512;
+// Prearrange blocks: one triangle per work item, kPreThreads (256) of them.
+// Cut records and sample ranges are allocated once per block (one 64-bit
+// atomicAdd on the packed counter (cuts << 32 | samples) of the block's
+// partition).  The next render's prearrange runs beside the current render's
+// shading, whose wavefronts hold 440 of a SIMD's 512 registers: a block of four
+// wavefronts with at most 72 registers finds room on a CU at once, where a
+// block of eight with 90 waited until the CU had drained (prearrange 36 us
+// alone, 200-260 us beside shading).  With the counters zeroed by the clear
+// and pieces that cover nothing left out: 1280x719, 120,000 triangles
+// 88.8 -> 81.0 us, 1080p, 1 M triangles 194.8 -> 188.2, the 16-light 4K frame
+// 5.00 -> 4.88 ms.
+// Lists of one partition (reserved or tiled) use blocks of 512, which append
+// half as often to the one counter.
+// The shadow prearrange (104 VGPRs) uses 512: two blocks per CU hide each
+// other's loads, barriers and allocation atomic (16-light shadow pass over
+// 4 M triangles 5.09 -> 4.82 ms).
+constexpr int kPreThreadsOne = 512;
 constexpr int kShadowPreThreads = 512;
 
 template <int kWaves>
 struct BlockAllocLds {
-  uint32_t cuts[kWaves], smps[kWaves], frags[kWaves];
+  uint32_t cuts[kWaves], smps[kWaves], frags[kWaves], more[kWaves];
   unsigned long long base;
-  uint32_t ok;
+  uint32_t ok, any_more;
 };
 
-// Returns false (for the whole block) when the block's records do not fit the
-// list or the sample space; the overflow word then says which.  The block's
-// sample total is checked before its atomic, and each atomic adds less than
-// kMaxSamples, so the low half reaches the threshold and sets the flag before
-// it could carry into the record count.
+// Appends ncut (0 or 1) records holding nsmp samples per work item to the
+// block's partition; `seen` pieces of nfrag fragments count in the
+// statistics.  Returns false (for the whole block) when the block's records
+// do not fit the partition or its sample space; the overflow word then says
+// which.  The block's sample total is checked before its atomic, and each
+// atomic adds less than kMaxSamples, so the low half reaches the threshold
+// and sets the flag before it could carry into the record count.  more: in,
+// whether the work item has another piece; out, whether any of the block has.
 template <int kWaves>
 __device__ __forceinline__ bool block_alloc(const Lists& L, BlockAllocLds<kWaves>& sh, uint32_t ncut, uint32_t nsmp,
-                                            uint32_t nfrag, uint32_t& cut0, uint32_t& smp0) {
+                                            uint32_t seen, uint32_t nfrag, bool& more, uint32_t& cut0, uint32_t& smp0) {
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const uint32_t ic = wave_incl_scan(ncut), is = wave_incl_scan(nsmp), ifr = wave_incl_scan(nfrag);
+  const unsigned long long cut_lanes = __ballot(ncut != 0u);
+  const uint32_t is = wave_incl_scan(nsmp), ifr = wave_incl_scan(nfrag);
+  const uint32_t nseen = (uint32_t)__popcll(__ballot(seen != 0u));
+  const unsigned long long more_lanes = __ballot(more);
   if (lane == kWave - 1) {
-    sh.cuts[wave] = ic;
+    sh.cuts[wave] = (uint32_t)__popcll(cut_lanes) | nseen << 16;
     sh.smps[wave] = is;
     sh.frags[wave] = ifr;
+    sh.more[wave] = more_lanes != 0ull;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    uint32_t tc = 0, tf = 0;
+    uint32_t tc = 0, tn = 0, tf = 0, tm = 0;
     unsigned long long ts = 0;
     for (int w = 0; w < kWaves; w++) {
       const uint32_t c = sh.cuts[w], sm = sh.smps[w];
       sh.cuts[w] = tc;
       sh.smps[w] = (uint32_t)ts;
-      tc += c;
+      tc += c & 0xFFFFu;
+      tn += c >> 16;
       ts += sm;
       tf += sh.frags[w];
+      tm |= sh.more[w];
     }
+    const uint32_t part = blockIdx.x & (L.parts - 1u), cap = L.cap_cut / L.parts;
     uint32_t bad = ts > kMaxSamples ? kOverflowSamples : 0u;
     unsigned long long base = 0;
     if (!bad && tc) {
-      base = atomicAdd(reinterpret_cast<unsigned long long*>(L.counters + kPacked), ((unsigned long long)tc << 32) + ts);
+      base = atomicAdd(reinterpret_cast<unsigned long long*>(L.counters + kPartWord(part)),
+                       ((unsigned long long)tc << 32) + ts);
       const unsigned long long end = base + ((unsigned long long)tc << 32) + ts;
-      if ((end >> 32) > L.cap_cut) bad |= kOverflowCuts;
+      if ((end >> 32) > cap) bad |= kOverflowCuts;
       if ((uint32_t)end > kMaxSamples) bad |= kOverflowSamples;
     }
-    if (tf && L.count_frags) atomicAdd(&L.counters[kFragCount], tf);
+    // fragments stay far below 2^32 (one per piece and one per 500 samples)
+    if (tn)
+      atomicAdd(reinterpret_cast<unsigned long long*>(L.counters + kFragCount), ((unsigned long long)tn << 32) + tf);
     if (bad) atomicOr(&L.counters[kOverflow], bad);
-    sh.base = base;
+    sh.base = base + ((unsigned long long)(part * cap) << 32);
     sh.ok = bad == 0;
+    sh.any_more = tm;
   }
   __syncthreads();
   const unsigned long long base = sh.base;
-  cut0 = (uint32_t)(base >> 32) + sh.cuts[wave] + ic - ncut;
+  cut0 = (uint32_t)(base >> 32) + sh.cuts[wave] + lanes_below(cut_lanes);
   smp0 = (uint32_t)base + sh.smps[wave] + is - nsmp;
   const bool ok = sh.ok != 0;
+  more = sh.any_more != 0;
   __syncthreads();   // the LDS record is reused by the block's next allocation
   return ok;
 }
@@ -176,7 +195,6 @@ __device__ __forceinline__ uint32_t cull_count(const f3 p[3], float ew, float eh
   return n > 0.f ? (uint32_t)n : 0u;
 }
 
-template <bool kCamera>
 __device__ __forceinline__ void store_cut(CutTri* dst, const f3 p[3], float rconst, uint32_t key, uint32_t oid,
                                           uint32_t view) {
   CutTri c;
@@ -186,14 +204,11 @@ __device__ __forceinline__ void store_cut(CutTri* dst, const f3 p[3], float rcon
   c.key = key;
   c.oid = oid;
   c.view = view;
-  c.da = c.db = c.dc = 0.f;
-  if constexpr (kCamera) {
-    // the plane kernel3's get_vtdiff builds per pixel (cl2.cl:5691-5760)
-    const f3 xpv = mk3(roundf(p[0].x), roundf(p[1].x), roundf(p[2].x));
-    const f3 ypv = mk3(roundf(p[0].y), roundf(p[1].y), roundf(p[2].y));
-    const f3 depths = mk3(rcp_rn(p[0].z), rcp_rn(p[1].z), rcp_rn(p[2].z));   // z in [20, 350000]
-    plane_const(depths, xpv, ypv, rconst, c.da, c.db, c.dc);
-  }
+  // the plane kernel3's get_vtdiff builds per pixel (cl2.cl:5691-5760)
+  const f3 xpv = mk3(roundf(p[0].x), roundf(p[1].x), roundf(p[2].x));
+  const f3 ypv = mk3(roundf(p[0].y), roundf(p[1].y), roundf(p[2].y));
+  const f3 depths = mk3(rcp_rn(p[0].z), rcp_rn(p[1].z), rcp_rn(p[2].z));   // z in [20, 350000]
+  plane_const(depths, xpv, ypv, rconst, c.da, c.db, c.dc);
   *dst = c;
 }
 
@@ -234,102 +249,98 @@ hipError_t launch_world(Scene* sc, hipStream_t s) {
   return hipGetLastError();
 }
 
-// full_rotate_quat's rotation into a camera or cube face (cl2.cl:700-729),
-// near clip and projection, from world-space vertices.
-__device__ __forceinline__ int face_clip_project(const f3 w[3], f3 cpos, const SinCos& sc, float fovc, float ew,
-                                                 float eh, f3 out[2][3]) {
+// full_rotate_quat's rotation into a camera or cube face (cl2.cl:700-729) and
+// near clip, from world-space vertices: 0..2 triangles.
+__device__ __forceinline__ int face_clip(const f3 w[3], f3 cpos, const SinCos& sc, f3 tris[2][3]) {
   f3 pr[3];
 #pragma unroll
   for (int i = 0; i < 3; i++) pr[i] = rot(w[i], cpos, sc);
-  f3 tris[2][3];
-  const int n = clip_near(pr[0], pr[1], pr[2], tris);
-  // slot 1 exists only for triangles crossing the near plane with one
-  // vertex behind it; static indices keep both slots in registers
-#pragma unroll
-  for (int i = 0; i < 3; i++) out[0][i] = depth_project_clipped(tris[0][i], ew, eh, fovc);
-  if (n == 2) {
-#pragma unroll
-    for (int i = 0; i < 3; i++) out[1][i] = depth_project_clipped(tris[1][i], ew, eh, fovc);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 3; i++) out[1][i] = out[0][i];
-  }
-  return n;
+  return clip_near(pr[0], pr[1], pr[2], tris);
 }
 
-// Appends this work item's cut triangles that hold samples (0..2) with their
-// sample ranges; called by every work item of the block.  A block that would
-// pass the list capacity or the sample limit writes nothing and sets the
-// overflow word, which every later pass of the render checks before reading
-// the list.
+// Whether point_in_tri's sums are exact integers for every pixel of the box
+// up to column xe and row ye: the edge terms are integer-valued (vertex
+// coordinates are rounded), and with |s|, |t| and the area bound at most
+// 2^23 in all their partial sums nothing rounds.  Then s > -0.0001 is s >= 0,
+// and s + t < e6 is s + t <= ceil(e6) - 1.
+__device__ __forceinline__ bool span_exact(const float ek[7], float xe, float ye) {
+  const float bs = fmaf(fabsf(ek[2]), ye, fmaf(fabsf(ek[1]), xe, fabsf(ek[0])));
+  const float bt = fmaf(fabsf(ek[5]), ye, fmaf(fabsf(ek[4]), xe, fabsf(ek[3])));
+  return bs + bt <= 8388608.f && ek[6] <= 8388608.f;
+}
+
+// One cut piece: its projected vertices, raster setup (key: kKeyBoxForm or
+// 0, the caller adds the key), fragments, and samples: `seen` by the
+// reference, `ns` of them in the list.
+struct Piece {
+  f3 p[3];
+  RasterTri rt;
+  float rc, my;   // 1/det constant; max_y, the end row of the box
+  uint32_t nf, seen, ns;
+};
+
+// Project, cull, count and set up a clipped triangle.  A piece whose walk
+// visits exactly its box gets the box form: one sample per box pixel, mapped
+// without the walk's fragment arithmetic.  A piece of zero rounded area with
+// exact edge sums covers no pixel (s >= 0 and t >= 0 leave no s + t < 0): it
+// counts, but is not listed.  Of the 1080p, 1 M-triangle frame's 446,000
+// pieces 105,000 are such, of a 1024^2 cube face's small ones in that scene
+// half.
+__device__ __forceinline__ void cut_piece(const f3 tri[3], float fovc, float ew, float eh, bool two_sided, int op,
+                                          Piece& P) {
+  P.nf = P.seen = P.ns = 0u;
+#pragma unroll
+  for (int i = 0; i < 3; i++) P.p[i] = depth_project_clipped(tri[i], ew, eh, fovc);
+  P.nf = cull_count(P.p, ew, eh, two_sided, op, P.rc);
+  if (!P.nf) return;
+  raster_setup(P.p, P.rc, ew, eh, P.rt, P.my);
+  // the box holds at most 16,000,000 pixels (frames and cube faces), an exact
+  // product, 0 when the walk has no samples (w or rows 0); the closed forms
+  // of walk_is_rect settle all but tall triangles near the top row, which
+  // keep the walk's samples
+  const float area = P.rt.w * (P.my - P.rt.min_y);
+  const bool box = area >= 1.f && area <= (float)kMaxTriSamples &&
+                   walk_is_rect_closed(P.rt.min_y, P.my, P.rt.w, P.rt.iw);
+  P.rt.key = box ? kKeyBoxForm : 0u;
+  P.seen = box ? (uint32_t)area : triangle_samples(P.rt, P.my, op, P.nf);
+  const bool empty = P.rt.ek[6] == 0.f && span_exact(P.rt.ek, P.rt.min_x + P.rt.w, P.my);
+  P.ns = empty ? 0u : P.seen;
+}
+
+// Appends the work items' cut pieces that hold samples with their sample
+// ranges; called by every work item of the block.  A block that would pass
+// the list capacity or the sample limit writes nothing and sets the overflow
+// word, which every later pass of the render checks before reading the list.
 // For a tiled render (L.tb.bin set) also the records' tile boxes and their
-// tiles' entry counts.
-template <bool kCamera, int kWaves>
-__device__ __forceinline__ void append_cuts(const Lists& L, BlockAllocLds<kWaves>& sh, const f3 tp[2][3],
-                                            const float rc[2], RasterTri rt[2], const uint32_t nf[2],
-                                            const uint32_t ns[2], uint32_t key0, uint32_t key_step, uint32_t oid,
-                                            uint32_t view, const float* my = nullptr, uint32_t bin_begin = 0,
-                                            uint32_t tiles_x = 0) {
-  const uint32_t k0 = ns[0] > 0, k1 = ns[1] > 0;
+// tiles' entry counts.  more: see block_alloc.
+template <int kWaves>
+__device__ __forceinline__ void append_cut(const Lists& L, BlockAllocLds<kWaves>& sh, Piece& P, uint32_t key,
+                                           uint32_t oid, uint32_t view, uint32_t bin_begin, uint32_t tiles_x,
+                                           bool& more) {
+  const bool have = P.ns > 0u;
   uint32_t c, smp;
-  if (!block_alloc(L, sh, k0 + k1, ns[0] + ns[1], nf[0] * k0 + nf[1] * k1, c, smp)) return;
-  uint4 box[2] = {};
-#pragma unroll
-  for (int i = 0; i < 2; i++) {
-    if (!ns[i]) continue;
-    const uint32_t key = key0 + key_step * (uint32_t)i;
-    // shadow records are read only through their raster setup
-    if constexpr (kCamera) store_cut<kCamera>(&L.cuts[c], tp[i], rc[i], key, oid, view);
-    rt[i].key = key | (rt[i].key & kKeyBoxForm);
-    rt[i].sample_begin = smp;
-    L.rast[c] = rt[i];
-    if constexpr (kCamera) {
-      if (L.tb.bin) {
-        box[i] = tile_box(rt[i], my[i], L.tb, bin_begin, tiles_x);
-        L.tb.box[c] = box[i];
-      }
-    }
-    smp += ns[i];
-    c++;
-  }
-  if constexpr (kCamera) {
+  if (!block_alloc(L, sh, have ? 1u : 0u, P.ns, P.seen, P.seen ? P.nf : 0u, more, c, smp)) return;
+  uint4 box{};
+  if (have) {
+    store_cut(&L.cuts[c], P.p, P.rc, key, oid, view);
+    P.rt.key = key | (P.rt.key & kKeyBoxForm);
+    P.rt.sample_begin = smp;
+    L.rast[c] = P.rt;
     if (L.tb.bin) {
-      uint32_t* cnt = L.tb.cnt;
-      const uint32_t ntiles = L.tb.ntiles;
-      expand_tile_pairs(
-          box[0], k0 != 0, box[1], k1 != 0,
-          [cnt, ntiles](uint32_t t, uint32_t len) {
-            if (t < ntiles) atomicAdd(&cnt[t], len);
-            return 0u;
-          },
-          [](uint32_t, int, uint32_t, uint32_t) {});
+      box = tile_box(P.rt, P.my, L.tb, bin_begin, tiles_x);
+      L.tb.box[c] = box;
     }
   }
-}
-
-// Cull, count and set up the (up to 2) clipped pieces of one triangle.
-// my[i]: piece i's max_y (its box's end row).  A piece whose walk visits
-// exactly its box gets the box form (rt.key = kKeyBoxForm; the caller adds
-// the key): one sample per box pixel, mapped without the walk's fragment
-// arithmetic.
-__device__ __forceinline__ void cut_pieces(const f3 tp[2][3], int num, float ew, float eh, bool two_sided, int op,
-                                           float rc[2], RasterTri rt[2], uint32_t nf[2], uint32_t ns[2],
-                                           float my[2]) {
-#pragma unroll
-  for (int i = 0; i < 2; i++) {
-    if (i >= num) continue;
-    nf[i] = cull_count(tp[i], ew, eh, two_sided, op, rc[i]);
-    if (!nf[i]) continue;
-    raster_setup(tp[i], rc[i], ew, eh, rt[i], my[i]);
-    // the box holds at most 16,000,000 pixels (frames and cube faces), an
-    // exact product, 0 when the walk has no samples (w or rows 0); the
-    // closed forms of walk_is_rect settle all but tall triangles near the
-    // top row, which keep the walk's samples
-    const float area = rt[i].w * (my[i] - rt[i].min_y);
-    const bool box = area >= 1.f && area <= (float)kMaxTriSamples &&
-                     walk_is_rect_closed(rt[i].min_y, my[i], rt[i].w, rt[i].iw);
-    rt[i].key = box ? kKeyBoxForm : 0u;
-    ns[i] = box ? (uint32_t)area : triangle_samples(rt[i], my[i], op, nf[i]);
+  if (L.tb.bin) {
+    uint32_t* cnt = L.tb.cnt;
+    const uint32_t ntiles = L.tb.ntiles;
+    expand_tile_pairs(
+        box, have, box, false,
+        [cnt, ntiles](uint32_t t, uint32_t len) {
+          if (t < ntiles) atomicAdd(&cnt[t], len);
+          return 0u;
+        },
+        [](uint32_t, int, uint32_t, uint32_t) {});
   }
 }
 
@@ -360,8 +371,8 @@ __device__ __forceinline__ uint32_t view_of(const PassArgs& a, uint32_t slot) {
 // ------------------------------------------------------------------ clear
 __global__ void __launch_bounds__(256) k_clear(PassArgs a) {
   const uint32_t slot = blockIdx.x * 256u;
-  // (a plain render zeroes its counters on its side stream instead)
-  if (a.lists.counters && blockIdx.x == 0 && threadIdx.x < kCounterWords) a.lists.counters[threadIdx.x] = 0u;
+  if (blockIdx.x == 0)
+    for (uint32_t i = threadIdx.x; i < (uint32_t)kPartWord(a.lists.parts); i += 256u) a.lists.counters[i] = 0u;
   const DevView& V = view_at(a, view_of<Range::Pix>(a, slot));
   const uint32_t i = slot - V.pix_begin + threadIdx.x;
   if (i >= V.v.width * V.v.height) return;
@@ -393,41 +404,56 @@ hipError_t launch_fill_u32(uint32_t* p, uint32_t value, size_t n, hipStream_t s)
 }
 
 // ------------------------------------------------------------- prearrange
-__global__ void __launch_bounds__(kPreThreads) k_prearrange(PassArgs a) {
-  __shared__ BlockAllocLds<kPreThreads / kWave> sh;
+template <int kThreads>
+__global__ void __launch_bounds__(kThreads) k_prearrange(PassArgs a) {
+  __shared__ BlockAllocLds<kThreads / kWave> sh;
   // per-view triangle ranges are 256-aligned: each wavefront has one view
-  const uint32_t slot = blockIdx.x * (uint32_t)kPreThreads + (threadIdx.x & ~(uint32_t)(kWave - 1));
+  const uint32_t slot = blockIdx.x * (uint32_t)kThreads + (threadIdx.x & ~(uint32_t)(kWave - 1));
   const uint32_t vi = view_of<Range::Tri>(a, slot);
   const DevView& V = view_at(a, vi);
   const DevScene& S = scene_at(a, V.scene);
   const ViewParams& v = V.v;
   const uint32_t id = slot - V.tri_begin + (threadIdx.x & (kWave - 1));
   const float ew = (float)v.width, eh = (float)v.height;
-  f3 tp[2][3];
-  float rc[2] = {0.f, 0.f};
-  RasterTri rt[2];
-  uint32_t nf[2] = {0u, 0u}, ns[2] = {0u, 0u};
-  float my[2] = {0.f, 0.f};
+  f3 tris[2][3];
+  int num = 0;
   uint32_t oid = 0;
+  bool two_sided = false;
   if (id < S.ntri) {
     const TriPos T = S.world[id];
     oid = T.oid;
     if (oid < S.nobj) {
-      const ObjDesc G = S.objs[oid];
-      f3 cpos = mk3(v.cpos[0], v.cpos[1], v.cpos[2]);
+      const ObjDesc& G = S.objs[oid];
+      const f3 cpos = mk3(v.cpos[0], v.cpos[1], v.cpos[2]);
+      two_sided = (G.flags & OCR_FEATURE_TWO_SIDED) > 0;
       if (!(fast_length(mk3(G.wp[0], G.wp[1], G.wp[2]) - cpos) > kDepthFar)) {
         const f3 w[3] = {mk3(T.p[0], T.p[1], T.p[2]), mk3(T.p[3], T.p[4], T.p[5]), mk3(T.p[6], T.p[7], T.p[8])};
-        const int num = face_clip_project(w, cpos, v.cam, v.fov, ew, eh, tp);
-        cut_pieces(tp, num, ew, eh, (G.flags & OCR_FEATURE_TWO_SIDED) > 0, kOpSize, rc, rt, nf, ns, my);
+        num = face_clip(w, cpos, v.cam, tris);
       }
     }
   }
-  append_cuts<true>(a.lists, sh, tp, rc, rt, nf, ns, 2u * id, 1u, oid, vi, my, V.bin_begin, V.bin_tiles_x);
+  // the second piece of a triangle cut by the near plane follows in an
+  // append of its own, which a block without any skips
+  Piece P;
+  P.nf = P.seen = P.ns = 0u;
+  if (num > 0) cut_piece(tris[0], v.fov, ew, eh, two_sided, kOpSize, P);
+  bool more = num > 1;
+  append_cut(a.lists, sh, P, 2u * id, oid, vi, V.bin_begin, V.bin_tiles_x, more);
+  if (!more) return;
+  P.nf = P.seen = P.ns = 0u;
+  if (num > 1) cut_piece(tris[1], v.fov, ew, eh, two_sided, kOpSize, P);
+  more = false;
+  append_cut(a.lists, sh, P, 2u * id + 1u, oid, vi, V.bin_begin, V.bin_tiles_x, more);
 }
 
 hipError_t launch_prearrange(const PassArgs& a, hipStream_t s) {
   if (a.tri_slots == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_prearrange, dim3((a.tri_slots + kPreThreads - 1) / kPreThreads), dim3(kPreThreads), 0, s, a);
+  if (a.lists.parts == 1 && a.tri_slots > 64 * kPreThreads)
+    hipLaunchKernelGGL(k_prearrange<kPreThreadsOne>, dim3((a.tri_slots + kPreThreadsOne - 1) / kPreThreadsOne),
+                       dim3(kPreThreadsOne), 0, s, a);
+  else
+    hipLaunchKernelGGL(k_prearrange<(int)kPreThreads>, dim3((a.tri_slots + kPreThreads - 1) / kPreThreads),
+                       dim3(kPreThreads), 0, s, a);
   return hipGetLastError();
 }
 
@@ -490,9 +516,6 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-__device__ __forceinline__ uint32_t lanes_below(unsigned long long m) {
-  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
 
 // Which item owns index base + lane, for items that tile [0, n) in lane
 // order (begin: the lane's item's first index, valid: whether it has one,
@@ -533,17 +556,6 @@ __device__ __forceinline__ void edge_span(float v, float c, float& lo, float& hi
   lo = c > 0.f ? fmaxf(lo, -q) : lo;
   hi = c < 0.f ? fminf(hi, q) : hi;
   hi = c == 0.f && v < 0.f ? -1.f : hi;
-}
-
-// Whether point_in_tri's sums are exact integers for every pixel of the box
-// up to column xe and row ye: the edge terms are integer-valued (vertex
-// coordinates are rounded), and with |s|, |t| and the area bound at most
-// 2^23 in all their partial sums nothing rounds.  Then s > -0.0001 is s >= 0,
-// and s + t < e6 is s + t <= ceil(e6) - 1.
-__device__ __forceinline__ bool span_exact(const float ek[7], float xe, float ye) {
-  const float bs = fmaf(fabsf(ek[2]), ye, fmaf(fabsf(ek[1]), xe, fabsf(ek[0])));
-  const float bt = fmaf(fabsf(ek[5]), ye, fmaf(fabsf(ek[4]), xe, fabsf(ek[3])));
-  return bs + bt <= 8388608.f && ek[6] <= 8388608.f;
 }
 
 // Where a render's samples go: one view's buffers, or the shadow maps (the
@@ -820,8 +832,8 @@ __device__ __forceinline__ void id_from_entries(const PassArgs& a, const Lists& 
   }
 }
 
-// Samples per chunk (log2) of a pass over `total` samples: the smallest power
-// of two from 2^kChunkMinLog2 that leaves at most kChunkTarget chunks, one or
+// Samples per chunk (log2) of a pass, from its sample count: the smallest power
+// of two from 2^kChunkMinLog2 that leaves about kChunkTarget chunks, one or
 // two per resident wavefront, up to kChunk.  A chunk is one wavefront's serial
 // work: with 2048-sample chunks whatever the total, frames of a few hundred
 // thousand samples occupied a few hundred of the chip's 8192 wavefronts for
@@ -832,10 +844,8 @@ __device__ __forceinline__ void id_from_entries(const PassArgs& a, const Lists& 
 // us in all.
 constexpr int kChunkMinLog2 = 7;
 constexpr uint32_t kChunkTarget = 8192;
-__device__ __forceinline__ int chunk_log2(uint32_t total) {
-  const uint32_t per = (total + kChunkTarget - 1) / kChunkTarget;   // samples per chunk, at least
-  const int up = per > 1u ? 32 - __clz((int)(per - 1u)) : 0;
-  return min(max(up, kChunkMinLog2), kChunkLog2);
+__device__ __forceinline__ int chunk_log2(uint32_t units) {   // of 2^kChunkMinLog2 samples
+  return min(kChunkMinLog2 + (units > kChunkTarget ? 32 - __clz((int)((units - 1u) / kChunkTarget)) : 0), kChunkLog2);
 }
 
 template <RasterMode kMode, int kOp, bool kBatch>
@@ -844,30 +854,36 @@ __global__ void __launch_bounds__(256) k_raster(PassArgs a, ShadowTarget sh) {
   const Lists& Ls = a.lists;
   if (Ls.counters[kOverflow]) return;
   const int lane = threadIdx.x & (kWave - 1);
-  // the list's records and samples; shadow lists are kShadowParts partitions
-  // (lane p holds partition p's records, samples and inclusive chunk count)
-  uint32_t ncut = 0, total = 0, nchunks;
-  uint32_t part_ncut = 0, part_total = 0, part_chunks = 0;
-  int clog = kChunkLog2;
+  // lane p holds partition p's records, samples and inclusive chunk count
+  uint32_t part_ncut = 0, part_total = 0;
   if constexpr (kMode == RasterMode::Shadow) {
     // (records << 40 | samples), up to the valid prefix
     const unsigned long long* pc = reinterpret_cast<const unsigned long long*>(Ls.counters + kPartWord(lane));
     const unsigned long long packed = min(pc[0], pc[1]);
     part_ncut = (uint32_t)(packed >> kShadowSampleBits);
     part_total = (uint32_t)(packed & kShadowSampleMask);   // at most 2^30
-    // the pass's samples in units of 2^kChunkMinLog2 (below 2^30)
-    constexpr uint32_t kUnit = 1u << kChunkMinLog2;
-    const uint32_t units = wave_total(wave_incl_scan((part_total + kUnit - 1) >> kChunkMinLog2));
-    clog = min(kChunkMinLog2 + (units > kChunkTarget ? 32 - __clz((int)((units - 1) / kChunkTarget)) : 0), kChunkLog2);
-    part_chunks = wave_incl_scan((part_total + (1u << clog) - 1) >> clog);
-    nchunks = wave_total(part_chunks);
-  } else {
-    const unsigned long long packed = *reinterpret_cast<const unsigned long long*>(Ls.counters + kPacked);
-    ncut = (uint32_t)(packed >> 32);
-    total = (uint32_t)packed;
-    clog = chunk_log2(total);
-    nchunks = (total + (1u << clog) - 1) >> clog;
+  } else if ((uint32_t)lane < Ls.parts) {
+    const unsigned long long packed = *reinterpret_cast<const unsigned long long*>(Ls.counters + kPartWord(lane));
+    part_ncut = (uint32_t)(packed >> 32);
+    part_total = (uint32_t)packed;   // at most kMaxSamples
   }
+  // the pass's samples in units of 2^kChunkMinLog2 (at most 2^30)
+  constexpr uint32_t kUnit = 1u << kChunkMinLog2;
+  const uint32_t units = wave_total(wave_incl_scan((part_total + kUnit - 1) >> kChunkMinLog2));
+  if constexpr (kMode != RasterMode::Shadow) {
+    // the partitions together hold at most kMaxSamples, like one list
+    if (units > kMaxSamples / kUnit) {
+      const unsigned long long all = ((unsigned long long)wave_total(wave_incl_scan(part_total >> 16)) << 16) +
+                                     wave_total(wave_incl_scan(part_total & 0xFFFFu));
+      if (all > kMaxSamples) {
+        if (lane == 0) atomicOr(&Ls.counters[kOverflow], kOverflowSamples);
+        return;
+      }
+    }
+  }
+  const int clog = chunk_log2(units);
+  const uint32_t part_chunks = wave_incl_scan((part_total >> clog) + ((part_total & ((1u << clog) - 1u)) ? 1u : 0u));
+  const uint32_t nchunks = wave_total(part_chunks);
   const uint32_t csize = 1u << clog;
   const uint32_t ent_cap = csize / 2u, ent_chunks = Ls.ent.chunks << (kChunkLog2 - clog);
   TriLds<kMode, kBatch>& L = lds_all[threadIdx.x / kWave];
@@ -881,17 +897,14 @@ __global__ void __launch_bounds__(256) k_raster(PassArgs a, ShadowTarget sh) {
   RasterTarget T{kMode == RasterMode::Shadow ? sh.L : a.view0.v.width,
                  kMode == RasterMode::Shadow ? sh.map : a.view0.depth, a.view0.idkey, nullptr, ent_cap, 0u};
   for (uint32_t chunk = wave0; chunk < nchunks; chunk += nwaves) {
-    const RasterTri* rast = Ls.rast;
-    uint32_t s0 = chunk << clog;
-    if constexpr (kMode == RasterMode::Shadow) {
-      // the chunk's partition: the first whose inclusive chunk count passes it
-      const uint32_t part = (uint32_t)__popcll(__ballot(part_chunks <= chunk));
-      const uint32_t before = part ? (uint32_t)__builtin_amdgcn_readlane((int)part_chunks, (int)part - 1) : 0u;
-      ncut = (uint32_t)__builtin_amdgcn_readlane((int)part_ncut, (int)part);
-      total = (uint32_t)__builtin_amdgcn_readlane((int)part_total, (int)part);
-      rast = Ls.rast + (size_t)part * (Ls.cap_cut / kShadowParts);
-      s0 = (chunk - before) << clog;
-    }
+    // the chunk's partition: the first whose inclusive chunk count passes it
+    const uint32_t part = (uint32_t)__popcll(__ballot(part_chunks <= chunk));
+    const uint32_t before = part ? (uint32_t)__builtin_amdgcn_readlane((int)part_chunks, (int)part - 1) : 0u;
+    const uint32_t ncut = (uint32_t)__builtin_amdgcn_readlane((int)part_ncut, (int)part);
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)part_total, (int)part);
+    const uint32_t first = part * (Ls.cap_cut / (kMode == RasterMode::Shadow ? kListParts : Ls.parts));
+    const RasterTri* rast = Ls.rast + first;
+    const uint32_t s0 = (chunk - before) << clog;
     const uint32_t s1 = min(s0 + csize, total);
     // covered-sample entries of the chunk: written by the depth pass, read
     // by the id pass instead of a second sweep
@@ -935,7 +948,7 @@ __global__ void __launch_bounds__(256) k_raster(PassArgs a, ShadowTarget sh) {
         if constexpr (kMode == RasterMode::Shadow)
           dst = sh.map + (size_t)(t.key & ~kKeyBoxForm) * sh.L * sh.L;   // 6 faces of L^2 per light
         if constexpr (kBatch) {
-          const DevView& V = a.views[Ls.cuts[ci].view];
+          const DevView& V = a.views[Ls.cuts[first + ci].view];
           dst = V.depth;
           ids = V.idkey;
           pitch = V.v.width;
@@ -944,7 +957,7 @@ __global__ void __launch_bounds__(256) k_raster(PassArgs a, ShadowTarget sh) {
       }
       const uint32_t stage_end = min(s1, (uint32_t)__builtin_amdgcn_readlane((int)after, kWave - 1));
       const uint32_t b = max(s, begin), e = min(stage_end, after);
-      raster_stage<kMode, kOp, kBatch>(L, T, t, ci, b < e ? b - begin : 1u, b < e ? e - begin : 0u, dst, pitch, ids,
+      raster_stage<kMode, kOp, kBatch>(L, T, t, first + ci, b < e ? b - begin : 1u, b < e ? e - begin : 0u, dst, pitch, ids,
                                        tick);
       s = stage_end;
       c0 += kWave;
@@ -1004,7 +1017,7 @@ struct ShadowGroup {
 
 // Shadow-pass allocation for the lanes with `take` set, per wavefront: one
 // atomicAdd on the packed counter of the block's partition (records
-// [part * cap, part * cap + cap) of the list, cap = cap_cut / kShadowParts,
+// [part * cap, part * cap + cap) of the list, cap = cap_cut / kListParts,
 // and a sample space of its own).  An allocation that passes the
 // partition's capacity or kShadowMaxSamples is not written: the wavefront
 // rasterises those pieces itself and lowers the partition's valid-prefix
@@ -1014,11 +1027,13 @@ struct ShadowGroup {
 __device__ __forceinline__ bool wave_alloc_fit(const Lists& L, uint32_t ncut, uint32_t nsmp, uint32_t& cut0,
                                                uint32_t& smp0) {
   const int lane = threadIdx.x & (kWave - 1);
-  const uint32_t ic = wave_incl_scan(ncut), is = wave_incl_scan(nsmp);
-  const uint32_t tc = wave_total(ic), ts = wave_total(is);
+  // ncut is 0 or 1
+  const unsigned long long m = __ballot(ncut != 0u);
+  const uint32_t is = wave_incl_scan(nsmp);
+  const uint32_t tc = (uint32_t)__popcll(m), ts = wave_total(is);
   cut0 = smp0 = 0;
   if (tc == 0) return true;
-  const uint32_t part = blockIdx.x % kShadowParts, cap = L.cap_cut / kShadowParts;
+  const uint32_t part = blockIdx.x % kListParts, cap = L.cap_cut / kListParts;
   uint32_t base_lo = 0, base_hi = 0, ok = 0;
   if (lane == 0) {
     unsigned long long* p = reinterpret_cast<unsigned long long*>(L.counters + kPartWord(part));
@@ -1031,9 +1046,9 @@ __device__ __forceinline__ bool wave_alloc_fit(const Lists& L, uint32_t ncut, ui
       base_hi = (uint32_t)(old >> kShadowSampleBits);
     }
   }
-  ok = __shfl(ok, 0, kWave);
-  cut0 = part * cap + __shfl(base_hi, 0, kWave) + ic - ncut;
-  smp0 = __shfl(base_lo, 0, kWave) + is - nsmp;
+  ok = (uint32_t)__builtin_amdgcn_readfirstlane((int)ok);
+  cut0 = part * cap + (uint32_t)__builtin_amdgcn_readfirstlane((int)base_hi) + lanes_below(m);
+  smp0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)base_lo) + is - nsmp;
   return ok != 0;
 }
 
@@ -1111,86 +1126,72 @@ __global__ void __launch_bounds__(kShadowPreThreads) k_prearrange_shadow(const T
     // ---- phase 2: 64 work items per wavefront per round, the wavefronts
     // independent of each other
     for (uint32_t r0 = wave * kWave; r0 < n_items; r0 += kShadowPreThreads) {
-      f3 tp[2][3];
-      float rc[2] = {0.f, 0.f};
-      RasterTri rt[2];
-      uint32_t nf[2] = {0u, 0u}, ns[2] = {0u, 0u};
+      f3 tris[2][3];
+      int num = 0;
       uint32_t face = 0;
+      bool both = false;
       if (r0 + lane < n_items) {
         const uint32_t it = items[r0 + lane];
         const uint32_t lt = it >> 4;
         face = it & 7u;
+        both = ((it >> 3) & 1u) != 0u;
         f3 w[3];
 #pragma unroll
         for (int k = 0; k < 3; k++) w[k] = mk3(S.wpos[lt][3 * k], S.wpos[lt][3 * k + 1], S.wpos[lt][3 * k + 2]);
-        const int num = face_clip_project(w, lpos, ft.f[face], efov, ew, eh, tp);
-        float my[2];
-        cut_pieces(tp, num, ew, eh, ((it >> 3) & 1u) != 0u, kOpSizeLight, rc, rt, nf, ns, my);
+        num = face_clip(w, lpos, ft.f[face], tris);
       }
       const uint32_t key = key0 + face;
-      // pieces above local_max samples to the list, in allocations of at
-      // most kShadowWaveSamples samples (each takes the lanes whose running
-      // sum fits, at least the first waiting lane); pieces of the list's
-      // failed allocations and the small ones rasterised here
-      const bool big0 = ns[0] > local_max, big1 = ns[1] > local_max;
-      const uint32_t mine = (big0 ? ns[0] : 0u) + (big1 ? ns[1] : 0u);   // < 2^25
-      bool waiting = mine > 0, fit = false;
-      while (__ballot(waiting)) {
-        const uint32_t upto = wave_incl_scan(waiting ? mine : 0u);
-        const bool take = waiting && upto <= kShadowWaveSamples;
-        uint32_t c, smp;
-        const bool ok = wave_alloc_fit(lists, take ? (big0 ? 1u : 0u) + (big1 ? 1u : 0u) : 0u, take ? mine : 0u,
-                                       c, smp);
-        if (take) {
-          waiting = false;
-          fit = ok;
-          if (ok) {
-#pragma unroll
-            for (int i = 0; i < 2; i++) {
-              if (!(i == 0 ? big0 : big1)) continue;
-              rt[i].key = key | (rt[i].key & kKeyBoxForm);
-              rt[i].sample_begin = smp;
-              lists.rast[c] = rt[i];
-              smp += ns[i];
-              c++;
+      uint32_t* const dst = target.map + (size_t)key * target.L * target.L;
+      // the second piece exists only where the near plane cuts
+#pragma unroll 1
+      for (int i = 0; i < 2; i++) {
+        if (!__any(num > i)) break;
+        Piece P;
+        P.ns = 0u;
+        if (num > i) {
+          const f3 tri[3] = {i == 0 ? tris[0][0] : tris[1][0], i == 0 ? tris[0][1] : tris[1][1],
+                             i == 0 ? tris[0][2] : tris[1][2]};
+          cut_piece(tri, efov, ew, eh, both, kOpSizeLight, P);
+        }
+        // pieces above local_max samples to the list, in allocations of at
+        // most kShadowWaveSamples samples (each takes the lanes whose running
+        // sum fits, at least the first waiting lane); pieces of the list's
+        // failed allocations and the small ones rasterised here
+        const uint32_t mine = P.ns > local_max ? P.ns : 0u;   // < 2^24
+        bool waiting = mine > 0, listed = false;
+        while (__ballot(waiting)) {
+          const uint32_t upto = wave_incl_scan(waiting ? mine : 0u);
+          const bool take = waiting && upto <= kShadowWaveSamples;
+          uint32_t c, smp;
+          const bool ok = wave_alloc_fit(lists, take ? 1u : 0u, take ? mine : 0u, c, smp);
+          if (take) {
+            waiting = false;
+            listed = ok;
+            if (ok) {
+              P.rt.key = key | (P.rt.key & kKeyBoxForm);
+              P.rt.sample_begin = smp;
+              lists.rast[c] = P.rt;
             }
           }
         }
-      }
-      // The rest, straight into the maps: a map keeps the minimum depth of
-      // its samples, so the order in which they arrive does not matter.  The
-      // second piece exists only behind the near plane.
-      const uint32_t nl[2] = {fit && big0 ? 0u : ns[0], fit && big1 ? 0u : ns[1]};
-      uint32_t* const dst = target.map + (size_t)key * target.L * target.L;
-#pragma unroll 1
-      for (int i = 0; i < 2; i++) {
-        if (!__any(nl[i] != 0u)) continue;
-        const RasterTri r = i == 0 ? rt[0] : rt[1];
-        const uint32_t n = i == 0 ? nl[0] : nl[1];
-        raster_stage<RasterMode::Shadow, kOpSizeLight, false>(W, T, r, (uint32_t)lane, n ? 0u : 1u, n, dst, 0u, nullptr,
-                                                              tick);
+        // The rest, straight into the maps: a map keeps the minimum depth of
+        // its samples, so the order in which they arrive does not matter.
+        const uint32_t n = listed ? 0u : P.ns;
+        if (__any(n != 0u))
+          raster_stage<RasterMode::Shadow, kOpSizeLight, false>(W, T, P.rt, (uint32_t)lane, n ? 0u : 1u, n, dst, 0u,
+                                                                nullptr, tick);
       }
     }
   }
 }
 
-__global__ void k_zero_counters(uint32_t* c) {
-  if (threadIdx.x < kCounterWords)
-    c[threadIdx.x] = threadIdx.x == kValidEnd || threadIdx.x == kValidEnd + 1 ? 0xFFFFFFFFu : 0u;
-}
-
 // A shadow pass's counters: the render words and every partition's packed
 // counter (0) and valid prefix (all ones).
 __global__ void __launch_bounds__(256) k_zero_shadow_counters(uint32_t* c) {
-  for (uint32_t i = threadIdx.x; i < (uint32_t)kShadowCounterWords; i += blockDim.x) {
+  for (uint32_t i = threadIdx.x; i < (uint32_t)kListCounterWords; i += blockDim.x) {
     const uint32_t w = i < (uint32_t)kCounterWords ? 0u : (i - kCounterWords) % kPartLineWords;
     c[i] = i >= (uint32_t)kCounterWords && (w == 2u || w == 3u) ? 0xFFFFFFFFu : 0u;
   }
-}
-
-hipError_t launch_zero_counters(uint32_t* counters, hipStream_t s) {
-  hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, s, counters);
-  return hipGetLastError();
 }
 
 // Tuning of the shadow launches, read at every pass: pieces of at most
@@ -1222,7 +1223,7 @@ hipError_t launch_shadow_group(Scene* sc, const float (*lpos)[3], const uint32_t
   g.n = n;
   // raster setups only: shadow records have no CutTri
   Lists lists{nullptr, sc->sh_rast, sc->sh_counters,
-              std::min(sc->sh_cap_cut, env_u32("OCR_SHADOW_LIST_RECORDS", sc->sh_cap_cut)), 0u};
+              std::min(sc->sh_cap_cut, env_u32("OCR_SHADOW_LIST_RECORDS", sc->sh_cap_cut)), kListParts};
   const ShadowTarget target{maps, sc->lbuf_dim};
   hipLaunchKernelGGL(k_zero_shadow_counters, dim3(1), dim3(256), 0, s, sc->sh_counters);
   if (sc->ntri)

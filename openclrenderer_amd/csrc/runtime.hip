@@ -27,10 +27,9 @@ static thread_local std::string g_last_error;
 // GPU the library runs on holds until the process ends.  Host code reaches
 // it only through the address hipGetSymbolAddress returns for the device
 // (Ctx::noalloc_scratch); calls on one GPU share it and must not overlap.
-constexpr size_t kNoAllocScratchBytes = (size_t)64 << 20;
-constexpr size_t kNoAllocCounterBytes = 256;
-constexpr uint32_t kNoAllocCapCut =
-    (uint32_t)((kNoAllocScratchBytes - kNoAllocCounterBytes) / (sizeof(CutTri) + sizeof(RasterTri)));
+constexpr size_t kNoAllocCounterBytes = 4 * (size_t)kListCounterWords;
+constexpr uint32_t kNoAllocCapCut = 524286;   // records, 64 MiB
+constexpr size_t kNoAllocScratchBytes = kNoAllocCounterBytes + kNoAllocCapCut * (sizeof(CutTri) + sizeof(RasterTri));
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 void set_error(const std::string& msg) { g_last_error = msg; }
@@ -148,7 +147,8 @@ static PassArgs single_pass(const Scene* s, const ocr_view* view, Frame* f) {
   a.unshadowed = s->n_shadow == 0 ? 1u : 0u;
   a.tiles = view_tiles(view->width, view->height, a.tile_w_log2);
   const Frame::OutBuf& ob = f->out[f->cur];
-  a.lists = make_lists(ob.cuts, ob.counters, ob.cap_cut);
+  a.lists = make_lists(ob.cuts, ob.counters, ob.cap_cut,
+                       f->raster_mode == OCR_RASTER_TILES || f->want_cut ? 1u : list_parts(a.tri_slots, ob.cap_cut));
   a.lists.ent = ob.ent;
   if (f->raster_mode == OCR_RASTER_TILES && ob.tb.bin) {
     a.lists.tb = ob.tb;
@@ -231,12 +231,12 @@ int frame_alloc_set(Frame* f, int b) {
   int rc;
   if ((rc = dev_alloc(&o.depth, npix, "depth")) || (rc = dev_alloc(&o.idkey, npix, "id buffer")) ||
       (rc = dev_alloc(&o.rgba, npix, "rgba")) || (rc = dev_alloc(&o.normals, npix, "normals")) ||
-      (rc = dev_alloc(&o.counters, kCounterWords, "counters")) ||
+      (rc = dev_alloc(&o.counters, kListCounterWords, "counters")) ||
       (rc = dev_alloc(&o.ent.ent, (size_t)chunks * kEntCap, "covered-sample entries")) ||
       (rc = dev_alloc(&o.ent.cnt, std::max(chunks, kEntMinCounts), "covered-sample counts")))
     return rc;
   o.ent.chunks = chunks;
-  OCR_HIP_CHECK(hipMemset(o.counters, 0, 4 * kCounterWords));
+  OCR_HIP_CHECK(hipMemset(o.counters, 0, 4 * kListCounterWords));
   return OCR_OK;
 }
 
@@ -362,7 +362,7 @@ int ocr_scene_create(ocr_ctx* ctx, const ocr_triangle* tris, uint32_t ntri, cons
   if ((rc = dev_alloc(&s->tri_pos, ntri, "triangles")) || (rc = dev_alloc(&s->world, ntri, "world-space triangles")) ||
       (rc = dev_alloc(&s->tri_attr, ntri, "attributes")) ||
       (rc = dev_alloc(&s->objs, nobj, "descriptors")) || (rc = dev_alloc(&s->motion, (size_t)nobj * 16, "motion poses")) ||
-      (rc = dev_alloc(&s->sh_counters, kShadowCounterWords, "counters"))) {
+      (rc = dev_alloc(&s->sh_counters, kListCounterWords, "counters"))) {
     ocr_scene_destroy(s);
     return rc;
   }
@@ -897,6 +897,7 @@ int ocr_frame_set_profiling(ocr_frame* f, int enable) {
     OCR_HIP_CHECK(hipSetDevice(f->ctx->device));
     f->ev.assign((size_t)Frame::kRing * Frame::kEvents, nullptr);
     for (auto& e : f->ev) OCR_HIP_CHECK(hipEventCreate(&e));
+    f->ev_tiled.assign(Frame::kRing, 0);
   }
   return OCR_OK;
 }
@@ -939,10 +940,11 @@ int ocr_frame_reserve(ocr_frame* f, uint32_t max_cut_triangles) {
 }
 
 // A cut list holds at most 2 pieces per scene triangle; unless the caller
-// reserved a capacity it is sized for that, so it never overflows.
+// reserved a capacity it is sized for that in every partition, so it never
+// overflows.
 static int ensure_frame_list(ocr_frame* f, int b, uint32_t ntri) {
   Frame::OutBuf& lb = f->out[b];
-  uint64_t want = f->want_cut ? (uint64_t)f->want_cut : (uint64_t)ntri * 2 + 64;
+  uint64_t want = f->want_cut ? (uint64_t)f->want_cut : list_capacity(ntri);
   want = std::min<uint64_t>(want, 0xFFFFFFF0ull);
   if (lb.cuts && lb.cap_cut == want) return OCR_OK;
   if (lb.cuts && !f->want_cut && lb.cap_cut >= want) return OCR_OK;
@@ -985,6 +987,7 @@ int ocr_render(ocr_scene* s, const ocr_view* view, ocr_frame* f, void* stream) {
   const bool prof_shade = f->profiling && f->n_profiled < Frame::kRing;
   const bool prof = prof_shade && f->profiling == 1;
   hipEvent_t* ev = prof_shade ? &f->ev[(size_t)f->n_profiled * Frame::kEvents] : nullptr;
+  if (prof_shade) f->ev_tiled[f->n_profiled] = tiled;
   hipStream_t sb = f->ss[b];
   // Render N runs on the stream of its set once render N-kSets (same
   // buffers, same stream) and everything enqueued on the caller's stream
@@ -1004,8 +1007,6 @@ int ocr_render(ocr_scene* s, const ocr_view* view, ocr_frame* f, void* stream) {
   f->select(b);
   const Frame::OutBuf& o = f->out[b];
   const PassArgs pa = single_pass(s, view, f);
-  PassArgs pc = pa;
-  pc.lists.counters = nullptr;   // zeroed before prearrange below
   if (tiled) {
     // counters and tile counts, prearrange (+ boxes and counts), bin scan
     // and scatter, then depth and ids per tile (no clear: tiles write
@@ -1020,11 +1021,10 @@ int ocr_render(ocr_scene* s, const ocr_view* view, ocr_frame* f, void* stream) {
     if (prof) OCR_HIP_CHECK(hipEventRecord(ev[3], sb));
     if (prof) OCR_HIP_CHECK(hipEventRecord(ev[4], sb));
   } else {
-    OCR_HIP_CHECK(launch_zero_counters(o.counters, sb));
     if (prof) OCR_HIP_CHECK(hipEventRecord(ev[0], sb));
-    OCR_HIP_CHECK(launch_prearrange(pa, sb));
+    OCR_HIP_CHECK(launch_clear(pa, sb));
     if (prof) OCR_HIP_CHECK(hipEventRecord(ev[1], sb));
-    OCR_HIP_CHECK(launch_clear(pc, sb));
+    OCR_HIP_CHECK(launch_prearrange(pa, sb));
     if (prof) OCR_HIP_CHECK(hipEventRecord(ev[2], sb));
     OCR_HIP_CHECK(launch_depth(pa, kRasterBlocksPerCu, sb));
     if (prof) OCR_HIP_CHECK(hipEventRecord(ev[3], sb));
@@ -1086,13 +1086,10 @@ int ocr_render_noalloc(ocr_scene* s, const ocr_view* view, uint32_t* depth, unsi
   std::lock_guard<std::mutex> lk(s->ver_mu);
   pa.scene0 = dev_scene(s);
   pa.unshadowed = s->n_shadow == 0 ? 1u : 0u;
-  pa.lists = make_lists(cuts, counters, kNoAllocCapCut);
-  PassArgs pc = pa;
-  pc.lists.counters = nullptr;   // zeroed by their own kernel below
+  pa.lists = make_lists(cuts, counters, kNoAllocCapCut, list_parts(pa.tri_slots, kNoAllocCapCut));
   OCR_HIP_CHECK(s->wait_geometry(st));
-  OCR_HIP_CHECK(launch_zero_counters(counters, st));
+  OCR_HIP_CHECK(launch_clear(pa, st));
   OCR_HIP_CHECK(launch_prearrange(pa, st));
-  OCR_HIP_CHECK(launch_clear(pc, st));
   OCR_HIP_CHECK(launch_depth(pa, kRasterBlocksPerCu, st));
   OCR_HIP_CHECK(launch_id(pa, kRasterBlocksPerCu, st));
   OCR_HIP_CHECK(s->wait_shadow_maps(st));
@@ -1109,7 +1106,7 @@ int ocr_frame_get_stats(ocr_frame* f, void* stream, ocr_frame_stats* out) {
   uint32_t c[kCounterWords];
   OCR_HIP_CHECK(hipMemcpy(c, f->out[f->cur].counters, sizeof(c), hipMemcpyDeviceToHost));
   memset(out, 0, sizeof(*out));
-  out->n_cut = c[kPacked + 1];
+  out->n_cut = c[kCutCount];
   out->n_frag = c[kFragCount];
   out->overflow = c[kOverflow] ? 1u : 0u;
   out->n_profiled = (uint32_t)f->n_profiled;
@@ -1117,8 +1114,10 @@ int ocr_frame_get_stats(ocr_frame* f, void* stream, ocr_frame_stats* out) {
     // clear, prearrange, depth, id, shade (from the end of its wait for the
     // shadow maps), and the render's whole span
     double sum[6] = {0, 0, 0, 0, 0, 0};
-    const int from[6] = {1, 0, 2, 3, 6, 0}, to[6] = {2, 1, 3, 4, 5, 5};
     for (int r = 0; r < f->n_profiled; r++) {
+      // tiled renders count and scatter their bins (ms_clear) after prearrange
+      const bool tiled = f->ev_tiled[r];
+      const int from[6] = {tiled ? 1 : 0, tiled ? 0 : 1, 2, 3, 6, 0}, to[6] = {tiled ? 2 : 1, tiled ? 1 : 2, 3, 4, 5, 5};
       hipEvent_t* ev = &f->ev[(size_t)r * Frame::kEvents];
       float ms = 0.f;
       for (int i = 0; i < 6; i++) {
@@ -1192,7 +1191,7 @@ int ocr_frame_read(ocr_frame* f, uint32_t* depth, uint32_t* tri_id, uint8_t* rgb
   OCR_HIP_CHECK(hipSetDevice(f->ctx->device));
   hipStream_t st = (hipStream_t)stream;
   OCR_HIP_CHECK(hipStreamSynchronize(st));
-  uint32_t c[kCounterWords];
+  uint32_t c[kPartWord(1)];
   // a frame rendered by batches has no counters of its own (the batch's
   // status comes from ocr_batch_get_stats); its counters stay zero
   OCR_HIP_CHECK(hipMemcpy(c, f->out[f->cur].counters, sizeof(c), hipMemcpyDeviceToHost));
@@ -1200,10 +1199,11 @@ int ocr_frame_read(ocr_frame* f, uint32_t* depth, uint32_t* tri_id, uint8_t* rgb
     return fail(OCR_ERR_UNSUPPORTED, "ocr_frame_read: the render needs more than 2^31 - 1 raster samples");
   if (c[kOverflow]) {
     // A reserved cut list (or the tile bins) was too small: size the next
-    // render's for this one's count (high word of the packed counter, the
-    // bin total).
+    // render's for this one's count (high word of the packed counter of the
+    // one partition a reserved list has, the bin total).
+    const uint32_t listed = c[kPartWord(0) + 1];
     if (c[kOverflow] & kOverflowCuts)
-      f->want_cut = (uint32_t)std::min<uint64_t>((uint64_t)c[kPacked + 1] + c[kPacked + 1] / 4 + 64, 0xFFFFFFF0ull);
+      f->want_cut = (uint32_t)std::min<uint64_t>((uint64_t)listed + listed / 4 + 64, 0xFFFFFFF0ull);
     if (c[kOverflow] & kOverflowBins)
       f->want_bin = (uint32_t)std::min<uint64_t>((uint64_t)c[kBinTotal] + c[kBinTotal] / 4 + 64, 0xFFFFFFF0ull);
     return fail(OCR_ERR_OVERFLOW, (c[kOverflow] & kOverflowCuts)

@@ -40,7 +40,8 @@ constexpr uint32_t kScanChunk = kScanThreads * 4;   // tiles per scan block
 // Zeroes the render's counters and every tile's entry count.
 __global__ void __launch_bounds__(256) k_bin_reset(uint32_t* __restrict__ counters, uint32_t* __restrict__ cnt,
                                                    uint32_t ntiles) {
-  if (blockIdx.x == 0 && threadIdx.x < kCounterWords) counters[threadIdx.x] = 0u;
+  // a tiled render's list is one partition
+  if (blockIdx.x == 0 && threadIdx.x < kPartWord(1)) counters[threadIdx.x] = 0u;
   for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < ntiles; i += gridDim.x * 256u) cnt[i] = 0u;
 }
 
@@ -120,7 +121,7 @@ __global__ void __launch_bounds__(kScanThreads) k_bin_offsets(TileBins tb, uint3
 __global__ void __launch_bounds__(256) k_bin_scatter(TileBins tb, const uint32_t* __restrict__ counters,
                                                      uint32_t cap_cut) {
   if (counters[kOverflow]) return;
-  const uint32_t ncut = min((uint32_t)(*reinterpret_cast<const unsigned long long*>(counters + kPacked) >> 32), cap_cut);
+  const uint32_t ncut = min((uint32_t)(*reinterpret_cast<const unsigned long long*>(counters + kPartWord(0)) >> 32), cap_cut);
   const uint32_t stride = gridDim.x * 256u;
   // whole wavefronts iterate together (the pair loop needs every lane)
   for (uint32_t base = blockIdx.x * 256u + (threadIdx.x & ~(uint32_t)(kWave - 1)); base < ncut; base += stride) {
@@ -316,7 +317,7 @@ __device__ __forceinline__ void raster_tile(const PassArgs& a, uint32_t tile, bo
   }
   __syncthreads();
   if (ok) {
-    const unsigned long long packed = *reinterpret_cast<const unsigned long long*>(Ls.counters + kPacked);
+    const unsigned long long packed = *reinterpret_cast<const unsigned long long*>(Ls.counters + kPartWord(0));
     const uint32_t ncut = min((uint32_t)(packed >> 32), Ls.cap_cut), total = (uint32_t)packed;
     const uint32_t e0 = tb.off[tile], e1 = tb.off[tile + 1];
     const uint32_t nchunks = (e1 - e0 + kWave - 1) / kWave;

@@ -33,6 +33,11 @@ __device__ __forceinline__ uint32_t wave_total(uint32_t incl) {
   return (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
 }
 
+// Set bits of m below the lane.
+__device__ __forceinline__ uint32_t lanes_below(unsigned long long m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
 // The walk's row of sample q: floor(mad(q, 1/width, min_y)) (cl2.cl:5083).
 // Sample indices are integers below 2^24, exact in binary32.
 __device__ __forceinline__ float row_of(float q, float iw, float min_y) {

@@ -49,3 +49,24 @@ def test_chunks_and_rows_match_oracle(gpu_ctx, oracle, size, tris, spread):
         assert np.array_equal(out[k], ref[k]), k
     fr.close()
     g.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_inst,tris", [(4, 16200), (8, 33000), (40, 300000)])
+def test_partitioned_lists_match_reserved(gpu_ctx, n_inst, tris):
+    """Lists of 1, 2 and 32 partitions (triangle counts around 64 and 128
+    blocks of 256, and far more) give the frames and statistics of a reserved
+    list, which has one partition and blocks of 512."""
+    from openclrenderer_amd import runtime, scenes
+    sc = scenes.small_scene(77 + n_inst, n_inst, tris, box_units=8.0)
+    view = scenes.make_view(401, 303, (0.0, 0.0, -1300.0))
+    g = runtime.GpuScene(gpu_ctx, sc)
+    a, b = runtime.Frame(gpu_ctx, 401, 303), runtime.Frame(gpu_ctx, 401, 303)
+    b.reserve(2 * sc.ntri + 64)
+    oa, ob = a.render_read(g, view), b.render_read(g, view)
+    for k in ("depth", "tri_id", "rgba", "normals"):
+        assert np.array_equal(oa[k], ob[k]), k
+    sa, sb = a.stats(), b.stats()
+    assert sa["n_cut"] == sb["n_cut"] > 0 and sa["n_frag"] == sb["n_frag"] > 0
+    for x in (a, b, g):
+        x.close()
