@@ -125,7 +125,9 @@ __device__ __forceinline__ float sqrt_core(float x) {
 }
 __device__ __forceinline__ float sqrt_cr(float x) {
   float s = sqrt_core(x);
-  if (!sqrt_fast_ok(x)) s = sqrtf(x);
+  const bool full = !sqrt_fast_ok(x);
+  // (a wavefront vote: a per-lane test becomes a select with both computed)
+  if (__any(full)) s = full ? sqrtf(x) : s;
   return s;
 }
 // 1 / sqrt(d), both correctly rounded (the reference's fast_normalize and
