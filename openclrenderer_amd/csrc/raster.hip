@@ -474,7 +474,7 @@ hipError_t launch_prearrange(const PassArgs& a, hipStream_t s) {
 enum class RasterMode { Depth, Id, Shadow };
 
 struct ShadowTarget {
-  uint32_t* map;   // 6 faces of L x L
+  uint32_t* map;   // the group's first map: 6 faces of L x L per light, at most 2^31 texels in all
   uint32_t L;
 };
 
@@ -492,23 +492,25 @@ struct ShadowTarget {
 // That frame's depth pass issues 14.0 M vector instructions instead of 22.0 M;
 // its time alone (78 us) is the memory side's: 0.75 M atomic and 1.7 M read
 // requests.
+// The stage takes 5 KB of LDS per wavefront, so that eight blocks of four fit
+// on a CU (batches: six, their targets differ per triangle).
 template <RasterMode kMode, bool kBatch>
 struct TriLds {
-  static constexpr bool kWide = kBatch || kMode != RasterMode::Depth;   // runs keep their triangle
   // staged triangles drawn by rows, compacted
-  float4 q0[kWave];      // min_x, first row of the range, w, ceil(e6) - 1
-  float4 q1[kWave];      // e0, e1, e2, e3
-  float4 q2[kWave];      // e4, e5, A, B
-  uint4 q3[kWave];       // C, first row's index, rows | lane << 16, first column | last column << 16
+  uint4 qa[kWave];       // min_x | w << 16, first row of the range | rows << 16, first row's index | lane << 24,
+                         // first row's first column | last row's last column << 16
+  float4 qb[kWave];      // e0, e1, e2, ceil(e6) - 1
+  float4 qc[kWave];      // e3, e4, e5, A
+  float2 qd[kWave];      // B, C
   // runs of covered columns, compacted
   uint4 run[kWave];      // pixel - index, x - index, B*y + C, A
-  uint2 ent[kMode == RasterMode::Shadow ? 1 : kWave];   // y << 16, record
-  uint32_t pos[kWide ? kWave : 1];   // the run's triangle in q0..q3, dst, pitch
-  uint32_t start[kWave];             // start[p] == tick: an item begins at index base + p
-  uint32_t* dst[kWide ? kWave : 1];
-  uint32_t pitch[kBatch ? kWave : 1];
-  unsigned long long* ids[kBatch && kMode == RasterMode::Id ? kWave : 1];
-  uint32_t key[kMode == RasterMode::Id ? kWave : 1];
+  uint32_t ent[kMode == RasterMode::Shadow ? 0 : kWave];   // y << 16 | lane
+  uint32_t start[kWave];                                   // start[p] == tick: an item begins at index base + p
+  // per lane: its triangle's target
+  uint32_t face[kMode == RasterMode::Shadow ? kWave : 0];  // the cube face's first texel
+  uint32_t* dst[kBatch ? kWave : 0];
+  uint32_t pitch[kBatch ? kWave : 0];
+  unsigned long long* ids[kBatch && kMode == RasterMode::Id ? kWave : 0];
 };
 
 __device__ __forceinline__ void wave_lds_sync() {
@@ -558,28 +560,29 @@ __device__ __forceinline__ void edge_span(float v, float c, float& lo, float& hi
   hi = c == 0.f && v < 0.f ? -1.f : hi;
 }
 
-// Where a render's samples go: one view's buffers, or the shadow maps (the
-// staged triangles' own targets where kWide).  ent: the chunk's
-// covered-sample entries (see CoverEntries), nent of them so far.
+// Where a pass's samples go: one view's buffers or a group's shadow maps
+// (batches: the staged triangles' own).  ent: the chunk's covered-sample
+// entries (see CoverEntries), nent of them so far.  rast: the list (id pass).
 struct RasterTarget {
   uint32_t pitch;
   uint32_t* depth;
   unsigned long long* ids;
   uint2* ent;
   uint32_t ent_cap, nent;
+  const RasterTri* rast;
 };
 
 // One covered sample per lane (hit lanes): depth d at pixel pix of dst.
 // Called wave-uniformly.
 template <RasterMode kMode, bool kBatch>
 __device__ __forceinline__ void put_sample(RasterTarget& T, bool hit, uint32_t d, uint32_t pix, uint32_t xy,
-                                           uint32_t rec, uint32_t* dst, unsigned long long* ids, uint32_t key) {
+                                           uint32_t rec, uint32_t* dst, unsigned long long* ids) {
   bool keep = false;
   if (hit) {
     if constexpr (kMode == RasterMode::Id) {
       const uint32_t val = dst[pix];
       if (d > val - kBufError && d < val + kBufError)
-        atomicMax(&ids[pix], ((unsigned long long)(key + 1u) << 32) | rec);
+        atomicMax(&ids[pix], ((unsigned long long)((T.rast[rec].key & ~kKeyBoxForm) + 1u) << 32) | rec);
     } else {
       // The L2 performs atomics at ~26.6 G cache-line operations/s; a plain
       // load first drops the samples that cannot win (the stored depth only
@@ -613,81 +616,85 @@ __device__ __forceinline__ void put_sample(RasterTarget& T, bool hit, uint32_t d
   }
 }
 
-// Draws a stage: the lane's triangle t (key without its flag in `key`),
-// record rec, samples [b, e) of it (indices from its first; b >= e: none);
-// dst, pitch, ids: its target where targets differ.  tick: see owner_of, kept
-// by the caller.  Called wave-uniformly.
+// Draws a stage: the lane's triangle t, record rec (consecutive over the
+// lanes), samples [b, e) of it (indices from its first; b >= e: none); face:
+// its cube face's first texel (shadow passes); dst, pitch, ids: its target
+// (batches).  tick: see owner_of, kept by the caller.  Called wave-uniformly.
 template <RasterMode kMode, int kOp, bool kBatch>
 __device__ __forceinline__ void raster_stage(TriLds<kMode, kBatch>& L, RasterTarget& T, const RasterTri& t,
-                                             uint32_t rec, uint32_t b, uint32_t e, uint32_t* dst, uint32_t pitch,
-                                             unsigned long long* ids, uint32_t& tick) {
-  using Lds = TriLds<kMode, kBatch>;
+                                             uint32_t rec, uint32_t b, uint32_t e, uint32_t face, uint32_t* dst,
+                                             uint32_t pitch, unsigned long long* ids, uint32_t& tick) {
+  constexpr bool kShadow = kMode == RasterMode::Shadow;
   const int lane = threadIdx.x & (kWave - 1);
   const bool active = b < e, box = (t.key & kKeyBoxForm) != 0u;
-  const uint32_t key = t.key & ~kKeyBoxForm;
   // ---- the lane's rows
   const float i0 = (float)b, i1 = (float)(e - 1u);   // below 2^24
   const float r0 = floor_div(i0, t.w, t.iw), r1 = floor_div(i1, t.w, t.iw);
   const bool span = active && box && span_exact(t.ek, t.min_x + t.w, t.min_y + r1);
   const uint32_t nrows = span ? (uint32_t)(r1 - r0) + 1u : 0u;
-  const uint32_t rows_incl = wave_incl_scan(nrows), row_begin = rows_incl - nrows;
+  const uint32_t rows_incl = wave_incl_scan(nrows), row_begin = rows_incl - nrows;   // below 2^21
   const uint32_t rows = wave_total(rows_incl);
   const unsigned long long spans = __ballot(span);
   if (span) {
     const uint32_t p = lanes_below(spans);
-    L.q0[p] = make_float4(t.min_x, t.min_y + r0, t.w, ceilf(t.ek[6]) - 1.f);
-    L.q1[p] = make_float4(t.ek[0], t.ek[1], t.ek[2], t.ek[3]);
-    L.q2[p] = make_float4(t.ek[4], t.ek[5], t.A, t.B);
-    L.q3[p] = make_uint4(__float_as_uint(t.C), row_begin, nrows | (uint32_t)lane << 16,
+    L.qa[p] = make_uint4((uint32_t)t.min_x | (uint32_t)t.w << 16, (uint32_t)(t.min_y + r0) | nrows << 16,
+                         row_begin | (uint32_t)lane << 24,
                          (uint32_t)fmaf(-r0, t.w, i0) | (uint32_t)fmaf(-r1, t.w, i1) << 16);
-    if constexpr (Lds::kWide) L.dst[p] = dst;
-    if constexpr (kBatch) L.pitch[p] = pitch;
-    if constexpr (kBatch && kMode == RasterMode::Id) L.ids[p] = ids;
-    if constexpr (kMode == RasterMode::Id) L.key[p] = key;
+    L.qb[p] = make_float4(t.ek[0], t.ek[1], t.ek[2], ceilf(t.ek[6]) - 1.f);
+    L.qc[p] = make_float4(t.ek[3], t.ek[4], t.ek[5], t.A);
+    L.qd[p] = make_float2(t.B, t.C);
+  }
+  if constexpr (kShadow) L.face[lane] = face;
+  if constexpr (kBatch) {
+    L.dst[lane] = dst;
+    L.pitch[lane] = pitch;
+    if constexpr (kMode == RasterMode::Id) L.ids[lane] = ids;
   }
   const uint32_t rec0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(rec - (uint32_t)lane));
   for (uint32_t rb = 0; rb < rows; rb += kWave) {
     // ---- one row per lane
     const int k = owner_of(L, span, row_begin, rb, ++tick);
-    uint32_t n = 0, y = 0, who = 0;
-    float lo = 0.f, x0 = 0.f, rowc = 0.f, pa = 0.f;
+    uint32_t n = 0, y = 0, xs = 0, who = 0;
+    float rowc = 0.f, pa = 0.f;
     if (rb + (uint32_t)lane < rows) {
-      const float4 q0 = L.q0[k], q1 = L.q1[k], q2 = L.q2[k];
-      const uint4 q3 = L.q3[k];
-      const uint32_t r = rb + (uint32_t)lane - q3.y;
-      const float fy = q0.y + (float)r;
-      lo = r == 0u ? (float)(q3.w & 0xFFFFu) : 0.f;
-      float hi = r + 1u == (q3.z & 0xFFFFu) ? (float)(q3.w >> 16) : q0.z - 1.f;
+      const uint4 qa = L.qa[k];
+      const float4 qb = L.qb[k], qc = L.qc[k];
+      const float2 qd = L.qd[k];
+      const uint32_t r = rb + (uint32_t)lane - (qa.z & 0xFFFFFFu);
+      y = (qa.y & 0xFFFFu) + r;
+      const uint32_t min_x = qa.x & 0xFFFFu;
+      const float fy = (float)y, fx = (float)min_x;
+      float lo = r == 0u ? (float)(qa.w & 0xFFFFu) : 0.f;
+      float hi = (float)(r + 1u == qa.y >> 16 ? qa.w >> 16 : (qa.x >> 16) - 1u);
       // s, t and (ceil(e6) - 1) - s - t at the row's first column (exact)
-      const float vs = fmaf(q1.z, fy, fmaf(q1.y, q0.x, q1.x));
-      const float vt = fmaf(q2.y, fy, fmaf(q2.x, q0.x, q1.w));
-      edge_span(vs, q1.y, lo, hi);
-      edge_span(vt, q2.x, lo, hi);
-      edge_span(q0.w - vs - vt, -(q1.y + q2.x), lo, hi);
+      const float vs = fmaf(qb.z, fy, fmaf(qb.y, fx, qb.x));
+      const float vt = fmaf(qc.z, fy, fmaf(qc.y, fx, qc.x));
+      edge_span(vs, qb.y, lo, hi);
+      edge_span(vt, qc.y, lo, hi);
+      edge_span(qb.w - vs - vt, -(qb.y + qc.y), lo, hi);
       n = hi >= lo ? (uint32_t)(hi - lo) + 1u : 0u;
-      x0 = q0.x + lo;
-      y = (uint32_t)fy;
-      pa = q2.z;
-      rowc = fmaf(q2.w, fy, __uint_as_float(q3.x));
-      who = q3.z >> 16;
+      xs = min_x + (uint32_t)lo;
+      pa = qc.w;
+      rowc = fmaf(qd.x, fy, qd.y);
+      who = qa.z >> 24;
     }
     const uint32_t incl = wave_incl_scan(n), begin = incl - n;
     const uint32_t total = wave_total(incl);
     const unsigned long long runs = __ballot(n > 0u);
     if (n) {
-      const uint32_t p = lanes_below(runs), xs = (uint32_t)x0;
-      const uint32_t rp = kBatch ? L.pitch[kBatch ? k : 0] : T.pitch;
+      const uint32_t p = lanes_below(runs);
+      const uint32_t rp = kBatch ? L.pitch[kBatch ? who : 0] : T.pitch;
       // y and the pitch are below 2^16: the 24-bit multiply is exact
-      L.run[p] = make_uint4(__umul24(y, rp) + xs - begin, xs - begin, __float_as_uint(rowc), __float_as_uint(pa));
-      if constexpr (kMode != RasterMode::Shadow) L.ent[p] = make_uint2(y << 16, rec0 + who);
-      if constexpr (Lds::kWide) L.pos[Lds::kWide ? p : 0] = (uint32_t)k;
+      L.run[p] = make_uint4(__umul24(y, rp) + xs - begin + (kShadow ? L.face[kShadow ? who : 0] : 0u), xs - begin,
+                            __float_as_uint(rowc), __float_as_uint(pa));
+      if constexpr (!kShadow) L.ent[p] = y << 16 | who;
     }
     // ---- the runs' pixels, one per lane per step
     for (uint32_t base = 0; base < total; base += kWave) {
       const int m = owner_of(L, n > 0u, begin, base, ++tick);
       const uint32_t j = base + (uint32_t)lane;
       const bool hit = j < total;
-      uint32_t d = 0, pix = 0, xy = 0, rr = 0, kk = 0;
+      uint32_t d = 0, pix = 0, xy = 0, rr = 0;
       uint32_t* to = T.depth;
       unsigned long long* ti = T.ids;
       if (hit) {
@@ -695,19 +702,17 @@ __device__ __forceinline__ void raster_stage(TriLds<kMode, kBatch>& L, RasterTar
         const uint32_t x = j + R.y;
         d = depth_quant(fmaf(__uint_as_float(R.w), (float)x, __uint_as_float(R.z)));
         pix = j + R.x;
-        if constexpr (kMode != RasterMode::Shadow) {
-          const uint2 E = L.ent[m];
-          xy = x | E.x;
-          rr = E.y;
-        }
-        if constexpr (Lds::kWide) {
-          const uint32_t q = L.pos[Lds::kWide ? m : 0];
-          to = L.dst[q];
-          if constexpr (kBatch && kMode == RasterMode::Id) ti = L.ids[q];
-          if constexpr (kMode == RasterMode::Id) kk = L.key[q];
+        if constexpr (!kShadow) {
+          const uint32_t E = L.ent[m];
+          xy = x | (E & 0xFFFF0000u);
+          rr = rec0 + (E & 63u);
+          if constexpr (kBatch) {
+            to = L.dst[E & 63u];
+            if constexpr (kMode == RasterMode::Id) ti = L.ids[E & 63u];
+          }
         }
       }
-      put_sample<kMode, kBatch>(T, hit, d, pix, xy, rr, to, ti, kk);
+      put_sample<kMode, kBatch>(T, hit, d, pix, xy, rr, to, ti);
     }
     // the runs are rewritten by the next 64 rows
     wave_lds_sync();
@@ -719,7 +724,7 @@ __device__ __forceinline__ void raster_stage(TriLds<kMode, kBatch>& L, RasterTar
     left &= left - 1ull;
     auto f = [k](float v) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k)); };
     auto u = [k](uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, k); };
-    const uint32_t ub = u(b), ue = u(e), uk = u(t.key);
+    const uint32_t ub = u(b), ue = u(e), uk = u(t.key), uf = kShadow ? u(face) : 0u;
     const float min_x = f(t.min_x), min_y = f(t.min_y), w = f(t.w), iw = f(t.iw);
     const float A = f(t.A), B = f(t.B), C = f(t.C);
     const float e0 = f(t.ek[0]), e1 = f(t.ek[1]), e2 = f(t.ek[2]), e3 = f(t.ek[3]), e4 = f(t.ek[4]), e5 = f(t.ek[5]),
@@ -727,11 +732,11 @@ __device__ __forceinline__ void raster_stage(TriLds<kMode, kBatch>& L, RasterTar
     uint32_t* to = T.depth;
     unsigned long long* ti = T.ids;
     uint32_t up = T.pitch;
-    if constexpr (Lds::kWide) {
+    if constexpr (kBatch) {
       const uint64_t v = (uint64_t)(uintptr_t)dst;
       to = (uint32_t*)(uintptr_t)((uint64_t)u((uint32_t)(v >> 32)) << 32 | u((uint32_t)v));
+      up = u(pitch);
     }
-    if constexpr (kBatch) up = u(pitch);
     if constexpr (kBatch && kMode == RasterMode::Id) {
       const uint64_t v = (uint64_t)(uintptr_t)ids;
       ti = (unsigned long long*)(uintptr_t)((uint64_t)u((uint32_t)(v >> 32)) << 32 | u((uint32_t)v));
@@ -755,10 +760,10 @@ __device__ __forceinline__ void raster_stage(TriLds<kMode, kBatch>& L, RasterTar
           d = depth_quant(fmaf(A, x, fmaf(B, y, C)));
           const uint32_t xi = (uint32_t)(int)x, yi = (uint32_t)(int)y;
           xy = xi | yi << 16;
-          pix = __umul24(yi, up) + xi;
+          pix = __umul24(yi, up) + xi + uf;
         }
       }
-      put_sample<kMode, kBatch>(T, hit, d, pix, xy, rec0 + (uint32_t)k, to, ti, uk & ~kKeyBoxForm);
+      put_sample<kMode, kBatch>(T, hit, d, pix, xy, rec0 + (uint32_t)k, to, ti);
     }
   }
 }
@@ -895,7 +900,7 @@ __global__ void __launch_bounds__(256) k_raster(PassArgs a, ShadowTarget sh) {
     if (Ls.ent.cnt) id_from_entries<kBatch>(a, Ls, wave0, nwaves, min(ent_chunks, nchunks), ent_cap);
   }
   RasterTarget T{kMode == RasterMode::Shadow ? sh.L : a.view0.v.width,
-                 kMode == RasterMode::Shadow ? sh.map : a.view0.depth, a.view0.idkey, nullptr, ent_cap, 0u};
+                 kMode == RasterMode::Shadow ? sh.map : a.view0.depth, a.view0.idkey, nullptr, ent_cap, 0u, Ls.rast};
   for (uint32_t chunk = wave0; chunk < nchunks; chunk += nwaves) {
     // the chunk's partition: the first whose inclusive chunk count passes it
     const uint32_t part = (uint32_t)__popcll(__ballot(part_chunks <= chunk));
@@ -939,14 +944,13 @@ __global__ void __launch_bounds__(256) k_raster(PassArgs a, ShadowTarget sh) {
       const uint32_t ci = c0 + (uint32_t)lane;
       RasterTri t{};
       uint32_t begin = total, after = total;   // first sample of the lane's triangle and of the next
-      uint32_t* dst = T.depth;
-      unsigned long long* ids = T.ids;
-      uint32_t pitch = T.pitch;
+      uint32_t* dst = nullptr;
+      unsigned long long* ids = nullptr;
+      uint32_t pitch = 0, face = 0;
       if (ci < ncut) {
         t = rast[ci];
         begin = t.sample_begin;
-        if constexpr (kMode == RasterMode::Shadow)
-          dst = sh.map + (size_t)(t.key & ~kKeyBoxForm) * sh.L * sh.L;   // 6 faces of L^2 per light
+        if constexpr (kMode == RasterMode::Shadow) face = (t.key & ~kKeyBoxForm) * sh.L * sh.L;
         if constexpr (kBatch) {
           const DevView& V = a.views[Ls.cuts[first + ci].view];
           dst = V.depth;
@@ -957,8 +961,8 @@ __global__ void __launch_bounds__(256) k_raster(PassArgs a, ShadowTarget sh) {
       }
       const uint32_t stage_end = min(s1, (uint32_t)__builtin_amdgcn_readlane((int)after, kWave - 1));
       const uint32_t b = max(s, begin), e = min(stage_end, after);
-      raster_stage<kMode, kOp, kBatch>(L, T, t, first + ci, b < e ? b - begin : 1u, b < e ? e - begin : 0u, dst, pitch, ids,
-                                       tick);
+      raster_stage<kMode, kOp, kBatch>(L, T, t, first + ci, b < e ? b - begin : 1u, b < e ? e - begin : 0u, face, dst, pitch,
+                                       ids, tick);
       s = stage_end;
       c0 += kWave;
     }
@@ -1002,7 +1006,7 @@ struct FaceTable { SinCos f[6]; };
 // to a block-local work list in LDS, and phase 2: the pairs, one per work
 // item per round, clipped, projected, culled and set up for their face.
 // Pieces become records, key = slot * 6 + face with slot the light's cube
-// map in the scene's map array, for one raster launch over the whole group;
+// map in the group's maps, for one raster launch over the whole group;
 // pieces of at most local_max samples, and any that no longer fit the list,
 // are rasterised at once by the wavefront, their samples spread over its
 // lanes.  (Looping over the six faces per
@@ -1097,7 +1101,7 @@ __global__ void __launch_bounds__(kShadowPreThreads) k_prearrange_shadow(const T
   if (t < (uint32_t)kMaxShadowGroup) S.n_items[t] = 0;
   W.start[lane] = 0u;
   uint32_t tick = 0;
-  RasterTarget T{L, target.map, nullptr, nullptr, 0u, 0u};
+  RasterTarget T{L, target.map, nullptr, nullptr, 0u, 0u, nullptr};
   __syncthreads();
   for (uint32_t li = 0; li < group.n; li++) {
     const f3 lpos = mk3(group.pos[li][0], group.pos[li][1], group.pos[li][2]);
@@ -1141,7 +1145,7 @@ __global__ void __launch_bounds__(kShadowPreThreads) k_prearrange_shadow(const T
         num = face_clip(w, lpos, ft.f[face], tris);
       }
       const uint32_t key = key0 + face;
-      uint32_t* const dst = target.map + (size_t)key * target.L * target.L;
+      const uint32_t first_texel = key * target.L * target.L;
       // the second piece exists only where the near plane cuts
 #pragma unroll 1
       for (int i = 0; i < 2; i++) {
@@ -1178,8 +1182,8 @@ __global__ void __launch_bounds__(kShadowPreThreads) k_prearrange_shadow(const T
         // its samples, so the order in which they arrive does not matter.
         const uint32_t n = listed ? 0u : P.ns;
         if (__any(n != 0u))
-          raster_stage<RasterMode::Shadow, kOpSizeLight, false>(W, T, P.rt, (uint32_t)lane, n ? 0u : 1u, n, dst, 0u,
-                                                                nullptr, tick);
+          raster_stage<RasterMode::Shadow, kOpSizeLight, false>(W, T, P.rt, (uint32_t)lane, n ? 0u : 1u, n,
+                                                                first_texel, nullptr, 0u, nullptr, tick);
       }
     }
   }
@@ -1218,13 +1222,14 @@ hipError_t launch_shadow_group(Scene* sc, const float (*lpos)[3], const uint32_t
   memset(&g, 0, sizeof(g));
   for (uint32_t i = 0; i < n; i++) {
     for (int k = 0; k < 3; k++) g.pos[i][k] = lpos[i][k];
-    g.slot[i] = slots[i];
+    g.slot[i] = slots[i] - slots[0];
   }
   g.n = n;
   // raster setups only: shadow records have no CutTri
   Lists lists{nullptr, sc->sh_rast, sc->sh_counters,
               std::min(sc->sh_cap_cut, env_u32("OCR_SHADOW_LIST_RECORDS", sc->sh_cap_cut)), kListParts};
-  const ShadowTarget target{maps, sc->lbuf_dim};
+  // texels of the group's maps (consecutive slots) are counted from its first
+  const ShadowTarget target{maps + (size_t)slots[0] * 6 * sc->lbuf_dim * sc->lbuf_dim, sc->lbuf_dim};
   hipLaunchKernelGGL(k_zero_shadow_counters, dim3(1), dim3(256), 0, s, sc->sh_counters);
   if (sc->ntri)
     hipLaunchKernelGGL(k_prearrange_shadow, dim3((sc->ntri + kShadowPreThreads - 1) / kShadowPreThreads),
