@@ -156,6 +156,9 @@ __device__ __forceinline__ bool bright_ok(float b) {
 }
 __device__ __forceinline__ f3 fast_normalize(f3 v) { return v * inv_sqrt_cr(dot(v, v)); }
 __device__ __forceinline__ float fast_length(f3 v) { return sqrt_cr(dot(v, v)); }
+// The largest binary32 d with RN(sqrt(d)) <= kDepthFar.  The root does not
+// decrease with d, so fast_length(v) > kDepthFar is dot(v, v) > kDepthFarSq.
+constexpr float kDepthFarSq = 0x1.c8591cp+36f;
 __device__ __forceinline__ float clampf(float x, float lo, float hi) { return fminf(fmaxf(x, lo), hi); }
 __device__ __forceinline__ float min3f(float a, float b, float c) { return fminf(fminf(a, b), c); }
 __device__ __forceinline__ float max3f(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
