@@ -127,7 +127,9 @@ typedef struct ocr_tex_src {
 
 /* Counters of the last render of a frame, and per-pass device times when
  * profiling is on: hipEvent pairs on the render stream, averaged over every
- * render since profiling was (re)enabled. */
+ * render since profiling was (re)enabled.  The clear runs in prearrange's
+ * launch: its time is in ms_prearrange, ms_clear is 0 (or the tiled path's
+ * bins, see ocr_frame_set_raster). */
 typedef struct ocr_frame_stats {
     uint32_t n_cut;             /* cut (post clip/cull) triangles            */
     uint32_t n_frag;            /* fragment records                          */

@@ -39,7 +39,8 @@ struct ocr_batch {
   uint32_t tri_slots = 0, pix_slots = 0, tiles = 0;
   uint64_t sum_tris = 0, sum_pix = 0;
   CutTri* cuts = nullptr;
-  uint32_t* counters = nullptr;
+  uint32_t* counters = nullptr;      // published, then working (make_lists)
+  bool counters_dirty = false;       // a render was not enqueued to its end
   uint32_t cap_cut = 0;
   // tiled raster path (tune.raster_tile != 0): bins over every view's tiles
   TileBins tb{};
@@ -90,7 +91,8 @@ static PassArgs batch_pass(const ocr_batch* b) {
   a.unshadowed = 1u;
   for (const Scene* s : b->scenes)
     if (s->n_shadow) a.unshadowed = 0u;
-  a.lists = make_lists(b->cuts, b->counters, b->cap_cut, b->tune.raster_tile ? 1u : list_parts(b->tri_slots, b->cap_cut));
+  a.lists = make_lists(b->cuts, b->counters, b->cap_cut, b->tune.raster_tile ? 1u : list_parts(b->tri_slots, b->cap_cut),
+                       b->tune.raster_tile != 0);
   a.lists.ent = b->ent;
   if (b->tune.raster_tile) a.lists.tb = b->tb;
   return a;
@@ -285,8 +287,7 @@ static hipError_t enqueue_batch(ocr_batch* b, hipStream_t st) {
     if (e == hipSuccess) e = launch_bins(pa, st);
     if (e == hipSuccess) e = launch_tile_raster(pa, st);
   } else {
-    e = launch_clear(pa, st);
-    if (e == hipSuccess) e = launch_prearrange(pa, st);
+    e = launch_prearrange(pa, st);   // and the clear
     if (e == hipSuccess) e = launch_depth(pa, (int)b->tune.raster_blocks_per_cu, st);
     if (e == hipSuccess) e = launch_id(pa, (int)b->tune.raster_blocks_per_cu, st);
   }
@@ -391,8 +392,8 @@ int ocr_batch_create(ocr_ctx* ctx, uint32_t max_views, ocr_batch** out) {
   b->max_views = max_views;
   hipError_t e = hipMalloc((void**)&b->d_views, sizeof(DevView) * max_views);
   if (e == hipSuccess) e = hipMalloc((void**)&b->d_scenes, sizeof(DevScene) * max_views);
-  if (e == hipSuccess) e = hipMalloc((void**)&b->counters, 4 * kListCounterWords);
-  if (e == hipSuccess) e = hipMemset(b->counters, 0, 4 * kListCounterWords);
+  if (e == hipSuccess) e = hipMalloc((void**)&b->counters, 4 * 2 * kListCounterWords);
+  if (e == hipSuccess) e = hipMemset(b->counters, 0, 4 * 2 * kListCounterWords);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->capture_stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipHostMalloc((void**)&b->ds_host, sizeof(DevScene) * max_views);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&b->ds_done, hipEventDisableTiming);
@@ -555,7 +556,10 @@ int ocr_batch_render(ocr_batch* b, void* stream) {
   OCR_HIP_CHECK(bind_scenes(b, st));
   const bool prof = b->profiling && b->n_profiled < kBatchRing;
   if (prof) OCR_HIP_CHECK(hipEventRecord(b->ev[2 * b->n_profiled], st));
+  if (b->counters_dirty) OCR_HIP_CHECK(launch_zero_work(b->counters, st));
+  b->counters_dirty = true;
   OCR_HIP_CHECK(enqueue_batch(b, st));
+  b->counters_dirty = false;
   OCR_HIP_CHECK(note_scene_reads(b, st));
   if (prof) OCR_HIP_CHECK(hipEventRecord(b->ev[2 * b->n_profiled++ + 1], st));
   return OCR_OK;
@@ -600,6 +604,8 @@ int ocr_batch_launch_graph(ocr_batch* b, void* stream) {
   OCR_HIP_CHECK(bind_scenes(b, st));   // the graph reads d_scenes when it runs
   const bool prof = b->profiling && b->n_profiled < kBatchRing;
   if (prof) OCR_HIP_CHECK(hipEventRecord(b->ev[2 * b->n_profiled], st));
+  if (b->counters_dirty) OCR_HIP_CHECK(launch_zero_work(b->counters, st));
+  b->counters_dirty = false;
   OCR_HIP_CHECK(hipGraphLaunch(b->exec, st));
   OCR_HIP_CHECK(note_scene_reads(b, st));
   if (prof) OCR_HIP_CHECK(hipEventRecord(b->ev[2 * b->n_profiled++ + 1], st));

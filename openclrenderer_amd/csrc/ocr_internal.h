@@ -196,15 +196,19 @@ struct CoverEntries {
 struct Lists {
   CutTri* cuts;
   RasterTri* rast;
-  uint32_t* counters;
+  uint32_t* counters;     // zero when the render begins
+  uint32_t* pub;          // what the shading pass, later passes and the host read
   uint32_t cap_cut;
   uint32_t parts;
   TileBins tb;
   CoverEntries ent;
 };
-inline Lists make_lists(CutTri* cuts, uint32_t* counters, uint32_t cap_cut, uint32_t parts) {
-  return Lists{cuts, reinterpret_cast<RasterTri*>(cuts + cap_cut), counters, cap_cut, parts};
-}
+// counters: 2 * kListCounterWords words, the published ones, then the working
+// ones.  A render finds the working counters zero: its id pass copies them to
+// the published ones and its shading pass zeroes them for the next render, so
+// that no launch of its own clears them.  A tiled render zeroes and uses the
+// published ones.
+inline Lists make_lists(CutTri* cuts, uint32_t* counters, uint32_t cap_cut, uint32_t parts, bool tiled = false);
 constexpr uint32_t kMaxViews = 4096;
 
 // Everything the camera passes need.  A single view travels inline in the
@@ -248,6 +252,10 @@ constexpr int kPartLineWords = 32;
 constexpr int kListCounterWords = kCounterWords + (int)kListParts * kPartLineWords;
 // partition p: packed counter (u64) at word kPartWord(p), valid prefix at +2
 __host__ __device__ constexpr int kPartWord(uint32_t p) { return kCounterWords + (int)p * kPartLineWords; }
+inline Lists make_lists(CutTri* cuts, uint32_t* counters, uint32_t cap_cut, uint32_t parts, bool tiled) {
+  return Lists{cuts, reinterpret_cast<RasterTri*>(cuts + cap_cut), tiled ? counters : counters + kListCounterWords,
+               counters, cap_cut, parts};
+}
 // Triangles per prearrange block, the unit of the partitions.
 constexpr uint32_t kPreThreads = 256;
 // Partitions of a camera list of cap_cut records for tri_slots triangle
@@ -297,6 +305,7 @@ struct Ctx {
   // device address of the no-allocation render's scratch on this device
   // (hipGetSymbolAddress at ocr_create)
   unsigned char* noalloc_scratch = nullptr;
+  bool noalloc_dirty = false;   // a render into it was not enqueued to its end
 };
 
 struct Atlas {
@@ -429,7 +438,8 @@ struct Frame {
     uint32_t* rgba = nullptr;
     uint32_t* normals = nullptr;
     CutTri* cuts = nullptr;
-    uint32_t* counters = nullptr;
+    uint32_t* counters = nullptr;   // published, then working (make_lists)
+    bool counters_dirty = false;    // a render of the set was not enqueued to its end
     uint32_t cap_cut = 0;
     // tiled raster path (tiles.hip): bins of this set's cut list
     TileBins tb{};
@@ -487,6 +497,8 @@ int ensure_bins(TileBins& tb, uint32_t& box_cap, uint32_t cap_cut, uint32_t ntil
                 uint32_t cap_bin, bool exact);
 void free_bins(TileBins& tb, uint32_t& box_cap);
 hipError_t launch_bin_reset(const TileBins& tb, uint32_t* counters, hipStream_t s);
+// Zeroes the working counters of make_lists' array.
+hipError_t launch_zero_work(uint32_t* counters, hipStream_t s);
 uint32_t bin_scan_chunks(uint32_t ntiles);
 
 // ---- error plumbing -------------------------------------------------------
@@ -500,7 +512,8 @@ int fail(int code, const std::string& msg);
   } while (0)
 
 // ---- kernel launchers (defined next to their kernels) --------------------
-hipError_t launch_clear(const PassArgs& a, hipStream_t s);
+// Prearrange, and with it the clear of every view's depth and ids (sample-space
+// renders).
 hipError_t launch_prearrange(const PassArgs& a, hipStream_t s);
 hipError_t launch_depth(const PassArgs& a, int blocks_per_cu, hipStream_t s);
 hipError_t launch_id(const PassArgs& a, int blocks_per_cu, hipStream_t s);

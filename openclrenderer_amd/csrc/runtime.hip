@@ -27,7 +27,7 @@ static thread_local std::string g_last_error;
 // GPU the library runs on holds until the process ends.  Host code reaches
 // it only through the address hipGetSymbolAddress returns for the device
 // (Ctx::noalloc_scratch); calls on one GPU share it and must not overlap.
-constexpr size_t kNoAllocCounterBytes = 4 * (size_t)kListCounterWords;
+constexpr size_t kNoAllocCounterBytes = 4 * 2 * (size_t)kListCounterWords;
 constexpr uint32_t kNoAllocCapCut = 524286;   // records, 64 MiB
 constexpr size_t kNoAllocScratchBytes = kNoAllocCounterBytes + kNoAllocCapCut * (sizeof(CutTri) + sizeof(RasterTri));
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
@@ -147,8 +147,9 @@ static PassArgs single_pass(const Scene* s, const ocr_view* view, Frame* f) {
   a.unshadowed = s->n_shadow == 0 ? 1u : 0u;
   a.tiles = view_tiles(view->width, view->height, a.tile_w_log2);
   const Frame::OutBuf& ob = f->out[f->cur];
+  const bool tiled = f->raster_mode == OCR_RASTER_TILES;
   a.lists = make_lists(ob.cuts, ob.counters, ob.cap_cut,
-                       f->raster_mode == OCR_RASTER_TILES || f->want_cut ? 1u : list_parts(a.tri_slots, ob.cap_cut));
+                       tiled || f->want_cut ? 1u : list_parts(a.tri_slots, ob.cap_cut), tiled);
   a.lists.ent = ob.ent;
   if (f->raster_mode == OCR_RASTER_TILES && ob.tb.bin) {
     a.lists.tb = ob.tb;
@@ -231,12 +232,12 @@ int frame_alloc_set(Frame* f, int b) {
   int rc;
   if ((rc = dev_alloc(&o.depth, npix, "depth")) || (rc = dev_alloc(&o.idkey, npix, "id buffer")) ||
       (rc = dev_alloc(&o.rgba, npix, "rgba")) || (rc = dev_alloc(&o.normals, npix, "normals")) ||
-      (rc = dev_alloc(&o.counters, kListCounterWords, "counters")) ||
+      (rc = dev_alloc(&o.counters, 2 * kListCounterWords, "counters")) ||
       (rc = dev_alloc(&o.ent.ent, (size_t)chunks * kEntCap, "covered-sample entries")) ||
       (rc = dev_alloc(&o.ent.cnt, std::max(chunks, kEntMinCounts), "covered-sample counts")))
     return rc;
   o.ent.chunks = chunks;
-  OCR_HIP_CHECK(hipMemset(o.counters, 0, 4 * kListCounterWords));
+  OCR_HIP_CHECK(hipMemset(o.counters, 0, 4 * 2 * kListCounterWords));
   return OCR_OK;
 }
 
@@ -1021,10 +1022,13 @@ int ocr_render(ocr_scene* s, const ocr_view* view, ocr_frame* f, void* stream) {
     if (prof) OCR_HIP_CHECK(hipEventRecord(ev[3], sb));
     if (prof) OCR_HIP_CHECK(hipEventRecord(ev[4], sb));
   } else {
-    if (prof) OCR_HIP_CHECK(hipEventRecord(ev[0], sb));
-    OCR_HIP_CHECK(launch_clear(pa, sb));
-    if (prof) OCR_HIP_CHECK(hipEventRecord(ev[1], sb));
-    OCR_HIP_CHECK(launch_prearrange(pa, sb));
+    if (f->out[b].counters_dirty) OCR_HIP_CHECK(launch_zero_work(o.counters, sb));
+    f->out[b].counters_dirty = true;   // until the shading pass that zeroes them again is enqueued
+    if (prof) {
+      OCR_HIP_CHECK(hipEventRecord(ev[0], sb));
+      OCR_HIP_CHECK(hipEventRecord(ev[1], sb));
+    }
+    OCR_HIP_CHECK(launch_prearrange(pa, sb));   // and the clear
     if (prof) OCR_HIP_CHECK(hipEventRecord(ev[2], sb));
     OCR_HIP_CHECK(launch_depth(pa, kRasterBlocksPerCu, sb));
     if (prof) OCR_HIP_CHECK(hipEventRecord(ev[3], sb));
@@ -1037,6 +1041,7 @@ int ocr_render(ocr_scene* s, const ocr_view* view, ocr_frame* f, void* stream) {
   OCR_HIP_CHECK(s->wait_shadow_maps(sb));
   if (prof_shade) OCR_HIP_CHECK(hipEventRecord(ev[6], sb));
   OCR_HIP_CHECK(launch_shade(pa, s->ctx->face_sc, sb));
+  if (!tiled) f->out[b].counters_dirty = false;
   OCR_HIP_CHECK(s->note_read(sb, true));
   if (prof_shade) OCR_HIP_CHECK(hipEventRecord(ev[5], sb));
   OCR_HIP_CHECK(hipEventRecord(f->done[b], sb));
@@ -1088,12 +1093,14 @@ int ocr_render_noalloc(ocr_scene* s, const ocr_view* view, uint32_t* depth, unsi
   pa.unshadowed = s->n_shadow == 0 ? 1u : 0u;
   pa.lists = make_lists(cuts, counters, kNoAllocCapCut, list_parts(pa.tri_slots, kNoAllocCapCut));
   OCR_HIP_CHECK(s->wait_geometry(st));
-  OCR_HIP_CHECK(launch_clear(pa, st));
+  if (s->ctx->noalloc_dirty) OCR_HIP_CHECK(launch_zero_work(counters, st));
+  s->ctx->noalloc_dirty = true;
   OCR_HIP_CHECK(launch_prearrange(pa, st));
   OCR_HIP_CHECK(launch_depth(pa, kRasterBlocksPerCu, st));
   OCR_HIP_CHECK(launch_id(pa, kRasterBlocksPerCu, st));
   OCR_HIP_CHECK(s->wait_shadow_maps(st));
   OCR_HIP_CHECK(launch_shade(pa, s->ctx->face_sc, st));
+  s->ctx->noalloc_dirty = false;
   OCR_HIP_CHECK(s->note_read(st, true));
   return OCR_OK;
 }

@@ -443,7 +443,7 @@ __device__ __forceinline__ void shade_pixel(const ShadeLaunch& sl) {
   a.shadow_maps = to_global<const uint32_t>(S.shadow_maps);
   a.static_maps = to_global<const uint32_t>(S.static_maps);
   a.L = S.L;
-  a.counters = to_global<const uint32_t>(sl.p.lists.counters);
+  a.counters = to_global<const uint32_t>(sl.p.lists.pub);
   a.rgba = to_global<uint32_t>(V.rgba);
   a.normals = to_global<uint32_t>(V.normals);
   a.face = sl.face;
@@ -691,9 +691,19 @@ __device__ __forceinline__ void shade_pixel(const ShadeLaunch& sl) {
   a.normals[pix] = encode_normal(normal);
 }
 
+// Zeroes the working counters, which no pass of this render reads any more,
+// for the next render.  Behind the shading: a store in front of it keeps the
+// compiler from loading the view and scene tables through the scalar cache
+// (12-view batch: shading 302 -> 353 us).
+__device__ __forceinline__ void zero_work(const Lists& L) {
+  if (blockIdx.x == 0 && L.counters != L.pub)
+    for (uint32_t i = threadIdx.x; i < (uint32_t)kPartWord(L.parts); i += 256u) L.counters[i] = 0u;
+}
+
 template <bool kCount>
 __global__ void __launch_bounds__(256) k_shade(ShadeLaunch sl) {
   shade_pixel<kCount, true>(sl);
+  zero_work(sl.p.lists);
 }
 
 // Passes whose scenes have no shadow-casting light: without the occlusion
@@ -704,6 +714,7 @@ __global__ void __launch_bounds__(256) k_shade(ShadeLaunch sl) {
 // wavefronts per SIMD spill inside the light loop and run slower.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_shade_unshadowed(ShadeLaunch sl) {
   shade_pixel<false, false>(sl);
+  zero_work(sl.p.lists);
 }
 
 // The linear-space light colours (gamma_fwd of each light's colour, the same
