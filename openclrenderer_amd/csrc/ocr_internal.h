@@ -7,8 +7,10 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <memory>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/ocr.h"
@@ -298,6 +300,17 @@ constexpr uint32_t kShadowWaveSamples = 1u << 25;
 constexpr uint32_t kShadowMaxSamples = 1u << 30;
 constexpr uint32_t kShadowMaxRecords = 14u << 20;
 
+// An event that outlives whichever of its holders ends first.
+struct Event {
+  hipEvent_t ev = nullptr;
+  Event() = default;
+  Event(const Event&) = delete;
+  Event& operator=(const Event&) = delete;
+  ~Event() {
+    if (ev) (void)hipEventDestroy(ev);
+  }
+};
+
 struct Ctx {
   int device = 0;
   hipDeviceProp_t prop{};
@@ -306,6 +319,15 @@ struct Ctx {
   // (hipGetSymbolAddress at ocr_create)
   unsigned char* noalloc_scratch = nullptr;
   bool noalloc_dirty = false;   // a render into it was not enqueued to its end
+  // what ocr_render goes by when it chooses its stream: the last render's end,
+  // and whether a post pass or batch was enqueued since
+  std::mutex mu;
+  std::shared_ptr<Event> last_render;
+  bool other_work = false;
+  void note_other_work() {
+    std::lock_guard<std::mutex> lk(mu);
+    other_work = true;
+  }
 };
 
 struct Atlas {
@@ -362,10 +384,7 @@ struct Scene {
   // current one.  Every pass that reads objs or world enqueues its kernels
   // and records its reader event with ver_mu held (a server's dispatcher
   // thread renders while the application updates).
-  struct Reader {
-    hipStream_t stream;
-    hipEvent_t ev;   // recorded on `stream` after the stream's last pass that read the version
-  };
+  using Reader = std::shared_ptr<Event>;   // recorded after a pass that read the version
   ObjDesc* objs_v[2] = {};
   TriPos* world_v[2] = {};
   int ver = 0;
@@ -374,7 +393,7 @@ struct Scene {
   // device memory (batches) are rebuilt before their next launch
   uint64_t gen = 0;
   std::vector<Reader> readers[2];
-  std::vector<hipEvent_t> ev_pool;
+  std::vector<std::pair<hipStream_t, Reader>> stream_events;
   hipStream_t upd_stream = nullptr;
   std::mutex ver_mu;
   // Dynamic shadow-map versions, the same way: shadow_maps aliases
@@ -386,33 +405,40 @@ struct Scene {
   int mver = 0;
   std::vector<Reader> map_readers[2];
   hipStream_t sh_stream = nullptr;
-  hipError_t note_into(std::vector<Reader>& list, hipStream_t st) {
-    for (Reader& r : list)
-      if (r.stream == st) return hipEventRecord(r.ev, st);
-    hipEvent_t e = nullptr;
-    if (!ev_pool.empty()) {
-      e = ev_pool.back();
-      ev_pool.pop_back();
-    } else {
-      hipError_t c = hipEventCreateWithFlags(&e, hipEventDisableTiming);
-      if (c != hipSuccess) return c;
-    }
-    list.push_back(Reader{st, e});
-    return hipEventRecord(e, st);
+  static void note_into(std::vector<Reader>& list, const Reader& ev) {
+    // an event recorded again stands for its last recording
+    for (const Reader& r : list)
+      if (r == ev) return;
+    list.push_back(ev);
   }
-  // Records that work enqueued on `st` so far reads the current geometry
-  // version (and, for passes that shade, the current shadow maps).
+  // Notes that the work before `ev`'s recording reads the current geometry
+  // version (and, for passes that shade, the current shadow maps; a scene
+  // without any has none to protect).
+  void note_read(const Reader& ev, bool maps = false) {
+    note_into(readers[ver], ev);
+    if (maps && (n_shadow || n_static)) note_into(map_readers[mver], ev);
+  }
+  // The same for work enqueued on `st` so far, for passes with no event of
+  // their own: one event per stream.
   hipError_t note_read(hipStream_t st, bool maps = false) {
-    hipError_t e = note_into(readers[ver], st);
-    if (e == hipSuccess && maps) e = note_into(map_readers[mver], st);
+    Reader ev;
+    for (const auto& s : stream_events)
+      if (s.first == st) ev = s.second;
+    if (!ev) {
+      ev = std::make_shared<Event>();
+      hipError_t e = hipEventCreateWithFlags(&ev->ev, hipEventDisableTiming);
+      if (e != hipSuccess) return e;
+      stream_events.emplace_back(st, ev);
+    }
+    hipError_t e = hipEventRecord(ev->ev, st);
+    if (e == hipSuccess) note_read(ev, maps);
     return e;
   }
   // Makes `st` wait for every pass recorded in `list`, then forgets them.
-  hipError_t wait_readers(std::vector<Reader>& list, hipStream_t st) {
+  static hipError_t wait_readers(std::vector<Reader>& list, hipStream_t st) {
     for (const Reader& r : list) {
-      hipError_t e = hipStreamWaitEvent(st, r.ev, 0);
+      hipError_t e = hipStreamWaitEvent(st, r->ev, 0);
       if (e != hipSuccess) return e;
-      ev_pool.push_back(r.ev);
     }
     list.clear();
     return hipSuccess;
@@ -440,6 +466,7 @@ struct Frame {
     CutTri* cuts = nullptr;
     uint32_t* counters = nullptr;   // published, then working (make_lists)
     bool counters_dirty = false;    // a render of the set was not enqueued to its end
+    bool direct = false;            // the set's last render ran on the caller's stream
     uint32_t cap_cut = 0;
     // tiled raster path (tiles.hip): bins of this set's cut list
     TileBins tb{};
@@ -457,7 +484,7 @@ struct Frame {
   uint32_t* normals = nullptr;
   hipStream_t ss[kSets] = {};   // the streams renders of each set run on
   hipEvent_t entry[kSets] = {}; // caller's stream when a render of the set was issued
-  hipEvent_t done[kSets] = {};  // a render of the set finished
+  std::shared_ptr<Event> done[kSets];   // a render of the set finished; scenes it read hold on to it
   bool entry_valid[kSets] = {};
   uint32_t want_cut = 0;             // capacity set by ocr_frame_reserve (0 = automatic)
   // raster path of ocr_render (ocr_frame_set_raster): the sample space or
