@@ -574,6 +574,8 @@ hipError_t launch_mip(const Atlas& a, uint32_t src_id, uint32_t dst_id, uint32_t
 hipError_t launch_fill_u32(uint32_t* p, uint32_t value, size_t n, hipStream_t s);
 hipError_t launch_light_prep(const ocr_light* lights, uint32_t n, float* lin, hipStream_t s);
 hipError_t launch_world(Scene* sc, hipStream_t s);
+hipError_t launch_tri_ids(const unsigned long long* keys, const uint32_t* depth, uint32_t* out, uint32_t npix,
+                          hipStream_t s);
 
 constexpr int kWave = 64;
 

@@ -62,6 +62,27 @@ hipError_t launch_blend_depth(const uint32_t* src_depth, const uint32_t* dst_dep
   return hipGetLastError();
 }
 
+// The triangle-id image of a frame from its id keys and depth:
+// OCR_NO_TRIANGLE where either is empty, else the key's triangle.  Bound by
+// the 16 bytes a pixel it moves; the keys stay on the device, where a read of
+// all four buffers copied keys and depth to the host once more and formed the
+// ids there (1280x720: 2.04 -> 1.08 ms).
+__global__ void __launch_bounds__(256) k_tri_ids(const unsigned long long* __restrict__ keys,
+                                                 const uint32_t* __restrict__ depth, uint32_t* __restrict__ out,
+                                                 uint32_t npix) {
+  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < npix; i += gridDim.x * 256u) {
+    const unsigned long long k = keys[i];
+    out[i] = k != 0ull && depth[i] != 0xFFFFFFFFu ? (uint32_t)(((k >> 32) - 1ull) >> 1) : OCR_NO_TRIANGLE;
+  }
+}
+
+hipError_t launch_tri_ids(const unsigned long long* keys, const uint32_t* depth, uint32_t* out, uint32_t npix,
+                          hipStream_t s) {
+  const uint32_t blocks = std::max<uint32_t>(1, std::min<uint32_t>((npix + 255) / 256, (uint32_t)device_cu_count() * 8));
+  hipLaunchKernelGGL(k_tri_ids, dim3(blocks), dim3(256), 0, s, keys, depth, out, npix);
+  return hipGetLastError();
+}
+
 // decode_normal(ushort2), cl2.cl:5611-5646: short_to_float is
 // (s / 65535) * 2 - 1 (the POW2e16-1 macro binds as 65536 - 1).
 __device__ __forceinline__ f3 decode_normal_u16(uint32_t packed) {

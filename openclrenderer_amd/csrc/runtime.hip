@@ -1256,17 +1256,18 @@ int ocr_frame_read(ocr_frame* f, uint32_t* depth, uint32_t* tri_id, uint8_t* rgb
                                       : "ocr_frame_read: tile bins overflowed; re-render the frame");
   }
   size_t npix = (size_t)f->width * f->height;
+  uint32_t* tri_ids = nullptr;
+  if (tri_id) {
+    // into the set's covered-sample entries (40 bytes a pixel), which only its
+    // render's depth and id passes use
+    tri_ids = reinterpret_cast<uint32_t*>(f->out[f->cur].ent.ent);
+    OCR_HIP_CHECK(launch_tri_ids(f->idkey, f->depth, tri_ids, (uint32_t)npix, st));
+    OCR_HIP_CHECK(hipStreamSynchronize(st));   // the copies below need not follow `st`
+  }
   if (depth) OCR_HIP_CHECK(hipMemcpy(depth, f->depth, 4 * npix, hipMemcpyDeviceToHost));
   if (rgba8) OCR_HIP_CHECK(hipMemcpy(rgba8, f->rgba, 4 * npix, hipMemcpyDeviceToHost));
   if (normals) OCR_HIP_CHECK(hipMemcpy(normals, f->normals, 4 * npix, hipMemcpyDeviceToHost));
-  if (tri_id) {
-    std::vector<unsigned long long> k(npix);
-    std::vector<uint32_t> d(npix);
-    OCR_HIP_CHECK(hipMemcpy(k.data(), f->idkey, 8 * npix, hipMemcpyDeviceToHost));
-    OCR_HIP_CHECK(hipMemcpy(d.data(), f->depth, 4 * npix, hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < npix; i++)
-      tri_id[i] = (k[i] && d[i] != 0xFFFFFFFFu) ? (uint32_t)(((k[i] >> 32) - 1ull) >> 1) : OCR_NO_TRIANGLE;
-  }
+  if (tri_id) OCR_HIP_CHECK(hipMemcpy(tri_id, tri_ids, 4 * npix, hipMemcpyDeviceToHost));
   return OCR_OK;
 }
 
