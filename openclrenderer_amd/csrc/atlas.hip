@@ -10,6 +10,8 @@
 // cl2.cl:785-889).
 #pragma clang fp contract(off)
 
+#include <algorithm>
+
 #include "ocr_internal.h"
 
 namespace ocr {
@@ -53,26 +55,36 @@ __device__ __forceinline__ void atlas_write(const AtlasRef& a, const uint32_t c[
   *reinterpret_cast<uint32_t*>(a.pages + ((size_t)slice * 2048 * 2048 + (size_t)iy * 2048 + ix) * 4) = v;
 }
 
-__global__ void __launch_bounds__(256) k_atlas_upload(AtlasRef a, uint32_t tid, const uint8_t* __restrict__ src,
-                                                      uint32_t w, uint32_t h) {
+// One launch works on a group of textures (blockIdx.z).
+__global__ void __launch_bounds__(256) k_atlas_upload(AtlasRef a, const uint8_t* __restrict__ staging, AtlasGroup g) {
+  const AtlasTex T = g.tex[blockIdx.z];
   const uint32_t x = blockIdx.x * 16 + (threadIdx.x & 15);
   const uint32_t y = blockIdx.y * 16 + (threadIdx.x >> 4);
-  if (x >= w || y >= h) return;
-  const uint8_t* s = src + ((size_t)y * w + x) * 4;
+  if (x >= T.w || y >= T.h) return;
+  const uint8_t* s = staging + T.offset + ((size_t)y * T.w + x) * 4;
   uint32_t c[4];
 #pragma unroll
   for (int k = 0; k < 4; k++) c[k] = sat_u32(((float)s[k] / 255.0f) * 255.f);
-  float width = (float)a.sizes[a.nums[tid] >> 16];
-  atlas_write(a, c, (float)x, width - (float)(int)y, tid);
+  float width = (float)a.sizes[a.nums[T.tid] >> 16];
+  atlas_write(a, c, (float)x, width - (float)(int)y, T.tid);
 }
 
-__global__ void __launch_bounds__(256) k_atlas_mip(AtlasRef a, uint32_t src_id, uint32_t dst_id, uint32_t gw,
-                                                   uint32_t gh) {
+// Level `lvl` + 1 of each texture of the group from level `lvl` (0: the
+// texture itself).  The reference launches source-sized grids; a work item
+// whose texel lies beyond the half-sized level writes nothing, so the grid
+// covers that level only.
+__global__ void __launch_bounds__(256) k_atlas_mip(AtlasRef a, uint32_t lvl, uint32_t ntex, AtlasGroup g) {
+  const AtlasTex T = g.tex[blockIdx.z];
+  const uint32_t first = T.tid * kMipLevels + ntex;   // descriptor of the texture's first mip
+  const uint32_t src_id = lvl == 0 ? T.tid : first + lvl - 1, dst_id = first + lvl;
   const int x = (int)(blockIdx.x * 16 + (threadIdx.x & 15));
   const int y = (int)(blockIdx.y * 16 + (threadIdx.x >> 4));
-  if (x >= (int)gw || y >= (int)gh) return;
+  if (x >= (int)T.w || y >= (int)T.h) return;
   float width = (float)a.sizes[a.nums[src_id] >> 16];
-  if ((float)x >= width || (float)y >= width) return;
+  float nwidth = (float)a.sizes[a.nums[dst_id] >> 16];
+  float yx = ((float)(x * 2) / width) * nwidth;
+  float yy = ((float)(y * 2) / width) * nwidth;
+  if (yx >= nwidth || yy >= nwidth) return;
   const float gauss[3][3] = {{1, 2, 1}, {2, 4, 2}, {1, 2, 1}};
   float ax = 0, ay = 0, az = 0, aw = 0, div = 0.f;
 #pragma unroll
@@ -89,27 +101,31 @@ __global__ void __launch_bounds__(256) k_atlas_mip(AtlasRef a, uint32_t src_id, 
   ax /= div; ay /= div; az /= div; aw /= div;
   if (aw > 0.00000001f) { ax /= aw; ay /= aw; az /= aw; }
   aw *= 255.f;
-  float nwidth = (float)a.sizes[a.nums[dst_id] >> 16];
-  float yx = ((float)(x * 2) / width) * nwidth;
-  float yy = ((float)(y * 2) / width) * nwidth;
-  if (yx >= nwidth || yy >= nwidth) return;
   uint32_t c[4] = {sat_u32(ax), sat_u32(ay), sat_u32(az), sat_u32(aw)};
   atlas_write(a, c, yx, yy, dst_id);
 }
 
-hipError_t launch_atlas_upload(const Atlas& at, uint32_t tid, const uint8_t* src, uint32_t w, uint32_t h,
-                               hipStream_t s) {
+// Uploads a group's staged textures and builds their mips: five launches,
+// each over every texture (8 textures of 1024^2: 40 launches of 6 to 9 us and
+// 8 waits before).
+hipError_t launch_atlas_group(const Atlas& at, const uint8_t* staging, const AtlasGroup& g, uint32_t n, uint32_t ntex,
+                              hipStream_t s) {
   AtlasRef a{at.pages, at.nums, at.sizes};
-  hipLaunchKernelGGL(k_atlas_upload, dim3((w + 15) / 16, (h + 15) / 16), dim3(256), 0, s, a, tid, src, w, h);
-  return hipGetLastError();
-}
-
-hipError_t launch_mip(const Atlas& at, uint32_t src_id, uint32_t dst_id, uint32_t gw, uint32_t gh,
-                      hipStream_t s) {
-  AtlasRef a{at.pages, at.nums, at.sizes};
-  hipLaunchKernelGGL(k_atlas_mip, dim3((gw + 15) / 16, (gh + 15) / 16), dim3(256), 0, s, a, src_id, dst_id,
-                     gw, gh);
-  return hipGetLastError();
+  uint32_t w = 0, h = 0, base = 0;
+  for (uint32_t i = 0; i < n; i++) {
+    w = std::max(w, g.tex[i].w);
+    h = std::max(h, g.tex[i].h);
+    base = std::max(base, g.tex[i].base);
+  }
+  hipLaunchKernelGGL(k_atlas_upload, dim3((w + 15) / 16, (h + 15) / 16, n), dim3(256), 0, s, a, staging, g);
+  hipError_t e = hipGetLastError();
+  for (uint32_t lvl = 0; lvl < (uint32_t)kMipLevels && e == hipSuccess; lvl++) {
+    const uint32_t half = (base >> lvl) / 2;   // the level's largest side
+    const uint32_t gw = std::max(1u, std::min(w, half)), gh = std::max(1u, std::min(h, half));
+    hipLaunchKernelGGL(k_atlas_mip, dim3((gw + 15) / 16, (gh + 15) / 16, n), dim3(256), 0, s, a, lvl, ntex, g);
+    e = hipGetLastError();
+  }
+  return e;
 }
 
 }  // namespace ocr

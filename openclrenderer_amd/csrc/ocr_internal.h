@@ -324,6 +324,13 @@ struct Ctx {
   std::mutex mu;
   std::shared_ptr<Event> last_render;
   bool other_work = false;
+  // Device staging of scene and texture uploads, at most kStageBytes, held for
+  // the context's life, so that loading a scene allocates only what it keeps.
+  // One upload at a time.
+  static constexpr size_t kStageBytes = (size_t)64 << 20;
+  std::mutex stage_mu;
+  uint8_t* stage = nullptr;
+  size_t stage_bytes = 0;
   void note_other_work() {
     std::lock_guard<std::mutex> lk(mu);
     other_work = true;
@@ -567,10 +574,21 @@ int device_cu_count();
 // light i at lpos[i] writes the 6 faces of map slots[i] of `maps`.
 hipError_t launch_shadow_group(Scene* sc, const float (*lpos)[3], const uint32_t* slots, uint32_t n,
                                int only_static, uint32_t* maps, hipStream_t s);
-hipError_t launch_atlas_upload(const Atlas& a, uint32_t tid, const uint8_t* src, uint32_t w,
-                               uint32_t h, hipStream_t s);
-hipError_t launch_mip(const Atlas& a, uint32_t src_id, uint32_t dst_id, uint32_t gw, uint32_t gh,
-                      hipStream_t s);
+// A group of textures staged for upload: texture i's tightly packed rows at
+// byte `offset` of the staging buffer, its slot size `base` (a power of two).
+struct AtlasTex {
+  uint64_t offset;
+  uint32_t w, h, tid, base;
+};
+constexpr uint32_t kAtlasGroup = 64;
+struct AtlasGroup {
+  AtlasTex tex[kAtlasGroup];
+};
+hipError_t launch_atlas_group(const Atlas& a, const uint8_t* staging, const AtlasGroup& g, uint32_t n, uint32_t ntex,
+                              hipStream_t s);
+// Splits n triangles as the caller lays them out (144 bytes) into the position
+// and attribute records.
+hipError_t launch_split(const ocr_triangle* tris, uint32_t n, TriPos* pos, TriAttr* attr, hipStream_t s);
 hipError_t launch_fill_u32(uint32_t* p, uint32_t value, size_t n, hipStream_t s);
 hipError_t launch_light_prep(const ocr_light* lights, uint32_t n, float* lin, hipStream_t s);
 hipError_t launch_world(Scene* sc, hipStream_t s);

@@ -212,6 +212,41 @@ __device__ __forceinline__ void store_cut(CutTri* dst, const f3 p[3], float rcon
   *dst = c;
 }
 
+// The 144-byte triangle into the 40-byte position record read by every raster
+// pass and the 72-byte attribute record read only by shading.  Bound by the
+// 256 bytes a triangle it moves.
+__global__ void __launch_bounds__(256) k_split(const uint4* __restrict__ tris, uint32_t n, TriPos* __restrict__ pos,
+                                               TriAttr* __restrict__ attr) {
+  const uint32_t id = blockIdx.x * 256u + threadIdx.x;
+  if (id >= n) return;
+  TriPos P;
+  TriAttr A;
+#pragma unroll
+  for (int v = 0; v < 3; v++) {
+    // pos (4 words), normal (4), vt (2), object id, colour
+    const uint4 p = tris[9 * (size_t)id + 3 * v], nm = tris[9 * (size_t)id + 3 * v + 1], r = tris[9 * (size_t)id + 3 * v + 2];
+    P.p[3 * v] = __uint_as_float(p.x);
+    P.p[3 * v + 1] = __uint_as_float(p.y);
+    P.p[3 * v + 2] = __uint_as_float(p.z);
+    A.n[3 * v] = __uint_as_float(nm.x);
+    A.n[3 * v + 1] = __uint_as_float(nm.y);
+    A.n[3 * v + 2] = __uint_as_float(nm.z);
+    A.vt[2 * v] = __uint_as_float(r.x);
+    A.vt[2 * v + 1] = __uint_as_float(r.y);
+    A.col[v] = r.w;
+    if (v == 0) P.oid = r.z;
+  }
+  pos[id] = P;
+  attr[id] = A;
+}
+
+hipError_t launch_split(const ocr_triangle* tris, uint32_t n, TriPos* pos, TriAttr* attr, hipStream_t s) {
+  static_assert(sizeof(ocr_triangle) == 144 && sizeof(ocr_vertex) == 48, "record layout");
+  if (n)
+    hipLaunchKernelGGL(k_split, dim3((n + 255) / 256), dim3(256), 0, s, reinterpret_cast<const uint4*>(tris), n, pos, attr);
+  return hipGetLastError();
+}
+
 // full_rotate_quat's object-to-world step (cl2.cl:700-729): the same for the
 // camera and every light, so it is applied once per object update into the
 // scene's world-space copy of its triangles.

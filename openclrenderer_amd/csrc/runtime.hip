@@ -276,7 +276,13 @@ int ocr_create(int device, ocr_ctx** out) {
   return OCR_OK;
 }
 
-void ocr_destroy(ocr_ctx* ctx) { delete ctx; }
+void ocr_destroy(ocr_ctx* ctx) {
+  if (ctx && ctx->stage) {
+    (void)hipSetDevice(ctx->device);
+    dev_free(ctx->stage);
+  }
+  delete ctx;
+}
 
 int ocr_query_free_hbm(ocr_ctx* ctx, size_t* free_bytes, size_t* total_bytes) {
   if (!ctx) return fail(OCR_ERR_INVALID, "ocr_query_free_hbm: null ctx");
@@ -320,6 +326,22 @@ static void pack_obj(const ocr_obj_desc& s, ObjDesc& d) {
   d.inv_rough2 = 1.0f / d.rough2;
 }
 
+constexpr uint32_t kSplitChunk = 400000;   // 57.6 MB of staging
+static_assert(kSplitChunk * sizeof(ocr_triangle) <= Ctx::kStageBytes, "staging");
+
+// The context's staging buffer with room for `bytes` (stage_mu held).
+static int stage_buffer(Ctx* c, size_t bytes, uint8_t** out) {
+  if (c->stage_bytes < bytes) {
+    dev_free(c->stage);
+    c->stage_bytes = 0;
+    const int rc = dev_alloc(&c->stage, bytes, "upload staging");
+    if (rc) return rc;
+    c->stage_bytes = bytes;
+  }
+  *out = c->stage;
+  return OCR_OK;
+}
+
 int ocr_scene_create(ocr_ctx* ctx, const ocr_triangle* tris, uint32_t ntri, const ocr_obj_desc* objs,
                      uint32_t nobj, ocr_scene** out) {
   if (!ctx || !out || (ntri && !tris) || (nobj && !objs))
@@ -332,23 +354,6 @@ int ocr_scene_create(ocr_ctx* ctx, const ocr_triangle* tris, uint32_t ntri, cons
   s->ctx = ctx;
   s->ntri = ntri;
   s->nobj = nobj;
-  // Split the 144-byte AoS triangle into the 40-byte position record read by
-  // every raster pass and the 72-byte attribute record read only by shading.
-  std::vector<TriPos> pos(ntri);
-  std::vector<TriAttr> attr(ntri);
-  for (uint32_t t = 0; t < ntri; t++) {
-    const ocr_triangle& T = tris[t];
-    for (int v = 0; v < 3; v++) {
-      for (int k = 0; k < 3; k++) {
-        pos[t].p[3 * v + k] = T.vertices[v].pos[k];
-        attr[t].n[3 * v + k] = T.vertices[v].normal[k];
-      }
-      attr[t].vt[2 * v] = T.vertices[v].vt[0];
-      attr[t].vt[2 * v + 1] = T.vertices[v].vt[1];
-      attr[t].col[v] = T.vertices[v].vertex_col;
-    }
-    pos[t].oid = T.vertices[0].object_id;
-  }
   std::vector<ObjDesc> od(nobj);
   std::vector<float> motion((size_t)nobj * 16);
   for (uint32_t o = 0; o < nobj; o++) {
@@ -370,8 +375,24 @@ int ocr_scene_create(ocr_ctx* ctx, const ocr_triangle* tris, uint32_t ntri, cons
   s->objs_v[0] = s->objs;
   s->world_v[0] = s->world;
   hipError_t e = hipSuccess;
-  if (ntri) e = hipMemcpy(s->tri_pos, pos.data(), sizeof(TriPos) * ntri, hipMemcpyHostToDevice);
-  if (e == hipSuccess && ntri) e = hipMemcpy(s->tri_attr, attr.data(), sizeof(TriAttr) * ntri, hipMemcpyHostToDevice);
+  // The caller's triangles go to the device as they are and are split there,
+  // kSplitChunk of them at a time (a host loop over 200,000 triangles and its
+  // two arrays took 2 ms).
+  if (ntri) {
+    std::lock_guard<std::mutex> lk(ctx->stage_mu);
+    uint8_t* stage = nullptr;
+    if ((rc = stage_buffer(ctx, sizeof(ocr_triangle) * (size_t)std::min<uint32_t>(ntri, kSplitChunk), &stage))) {
+      ocr_scene_destroy(s);
+      return rc;
+    }
+    ocr_triangle* const staged = reinterpret_cast<ocr_triangle*>(stage);
+    for (uint32_t t = 0; t < ntri && e == hipSuccess; t += kSplitChunk) {
+      const uint32_t n = std::min<uint32_t>(kSplitChunk, ntri - t);
+      e = hipMemcpy(staged, tris + t, sizeof(ocr_triangle) * (size_t)n, hipMemcpyHostToDevice);
+      if (e == hipSuccess) e = launch_split(staged, n, s->tri_pos + t, s->tri_attr + t, nullptr);
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);   // the staging is free again
+  }
   if (e == hipSuccess && nobj) e = hipMemcpy(s->objs, od.data(), sizeof(ObjDesc) * nobj, hipMemcpyHostToDevice);
   if (e == hipSuccess && nobj) e = hipMemcpy(s->motion, motion.data(), 4 * motion.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = launch_world(s, nullptr);
@@ -583,26 +604,44 @@ int ocr_atlas_upload(ocr_scene* s, const ocr_tex_src* texs, uint32_t ntex) {
   OCR_HIP_CHECK(hipMemset(a.pages, 0, page_bytes * a.npages));
   OCR_HIP_CHECK(hipMemcpy(a.nums, nums.data(), sizeof(uint32_t) * a.nnums, hipMemcpyHostToDevice));
   OCR_HIP_CHECK(hipMemcpy(a.sizes, sizes.data(), sizeof(uint32_t) * a.nsizes, hipMemcpyHostToDevice));
-  // texture::update_me_to_gpu + update_gpu_mipmaps (texture.cpp:323-493).
-  size_t max_bytes = 0;
-  for (uint32_t t = 0; t < ntex; t++) max_bytes = std::max(max_bytes, (size_t)texs[t].width * texs[t].height * 4);
+  // texture::update_me_to_gpu + update_gpu_mipmaps (texture.cpp:323-493), in
+  // groups of at most kAtlasGroup textures and kAtlasStage bytes (a texture
+  // has at most 16 MiB).
+  constexpr size_t kAtlasStage = Ctx::kStageBytes;
+  auto bytes_of = [&](uint32_t t) { return ((size_t)texs[t].width * texs[t].height * 4 + 255) / 256 * 256; };
+  auto group_end = [&](uint32_t t, size_t& bytes) {
+    uint32_t e = t;
+    for (bytes = 0; e < ntex && e - t < kAtlasGroup && (e == t || bytes + bytes_of(e) <= kAtlasStage); e++)
+      bytes += bytes_of(e);
+    return e;
+  };
+  size_t max_bytes = 0, bytes = 0;
+  for (uint32_t t = 0; t < ntex;) {
+    t = group_end(t, bytes);
+    max_bytes = std::max(max_bytes, bytes);
+  }
+  std::lock_guard<std::mutex> stage_lock(s->ctx->stage_mu);
   uint8_t* staging = nullptr;
-  if (ntex && (rc = dev_alloc(&staging, max_bytes, "texture staging"))) return rc;
+  if (ntex && (rc = stage_buffer(s->ctx, max_bytes, &staging))) return rc;
   hipStream_t st = nullptr;
   int status = OCR_OK;
-  for (uint32_t t = 0; t < ntex && status == OCR_OK; t++) {
-    const ocr_tex_src& src = texs[t];
-    hipError_t e = hipMemcpy(staging, src.rgba, (size_t)src.width * src.height * 4, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = launch_atlas_upload(a, t, staging, src.width, src.height, st);
-    if (e == hipSuccess) e = launch_mip(a, t, t * OCR_MIP_LEVELS + ntex, src.width, src.height, st);
-    for (uint32_t lvl = 0; lvl + 1 < OCR_MIP_LEVELS && e == hipSuccess; lvl++) {
-      uint32_t proper = t * OCR_MIP_LEVELS + ntex + lvl;
-      e = launch_mip(a, proper, proper + 1, src.width, src.height, st);
+  for (uint32_t t = 0; t < ntex && status == OCR_OK;) {
+    const uint32_t end = group_end(t, bytes);
+    AtlasGroup g;
+    memset(&g, 0, sizeof(g));
+    hipError_t e = hipSuccess;
+    size_t at = 0;
+    for (uint32_t i = t; i < end && e == hipSuccess; i++) {
+      const ocr_tex_src& src = texs[i];
+      g.tex[i - t] = AtlasTex{at, src.width, src.height, i, base[i]};
+      e = hipMemcpy(staging + at, src.rgba, (size_t)src.width * src.height * 4, hipMemcpyHostToDevice);
+      at += bytes_of(i);
     }
+    if (e == hipSuccess) e = launch_atlas_group(a, staging, g, end - t, ntex, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) status = fail(OCR_ERR_HIP, std::string("ocr_atlas_upload: ") + hipGetErrorString(e));
+    t = end;
   }
-  dev_free(staging);
   return status;
 }
 
@@ -712,11 +751,19 @@ static int ensure_shadow_lists(ocr_scene* s, uint32_t cap_cut) {
 
 // Lights per shadow prearrange launch.  The launch rasterises small pieces
 // itself and lists the large ones while the list has room (then rasterises
-// the rest too), so any list size is correct; the list holds up to 6
-// records per triangle per light, at most kShadowMaxRecords (896 MB).
+// the rest too), so any list size is correct.  It holds one record per
+// triangle and light of a group in every partition, at most kShadowMaxRecords
+// (896 MB): half the triangles face a light, nearly all in one cube face, and
+// at most a tenth exceed the local limit in the scenes measured, so it does
+// not fill up (six records, as a triangle has at most, cost a 200,000-triangle
+// scene with four lights 940 MB of allocation).
 constexpr uint32_t kShadowGroup = 16;
-static uint32_t shadow_list_cap(uint32_t ntri) {
-  return (uint32_t)std::min<uint64_t>(((uint64_t)ntri * 6 + 64) * kShadowGroup, kShadowMaxRecords);
+static uint32_t shadow_list_cap(uint32_t ntri, uint32_t nlights) {
+  constexpr uint32_t kBlock = 512;   // triangles per prearrange block
+  const uint64_t blocks = ((uint64_t)ntri + kBlock - 1) / kBlock;
+  const uint64_t per_part = (blocks + kListParts - 1) / kListParts * std::min(ntri, kBlock) *
+                                std::min(std::max(nlights, 1u), kShadowGroup) + 64;
+  return (uint32_t)std::min<uint64_t>(per_part * kListParts, kShadowMaxRecords);
 }
 
 // Renders the maps of `n` lights (positions, map slots) in groups.
@@ -756,7 +803,7 @@ int ocr_shadow_pass(ocr_scene* s, void* stream) {
   if (s->static_dirty && s->n_static) OCR_HIP_CHECK(s->wait_readers(s->map_readers[s->mver], st));
   OCR_HIP_CHECK(s->wait_geometry(st));   // descriptor updates enqueued on another stream
   {
-    int rc = ensure_shadow_lists(s, shadow_list_cap(s->ntri));
+    int rc = ensure_shadow_lists(s, shadow_list_cap(s->ntri, std::max(s->n_shadow, s->n_static)));
     if (rc) return rc;
   }
   uint32_t* const maps = s->maps_v[nm];
