@@ -179,19 +179,67 @@ __device__ __forceinline__ f4 texture_filter_diff(const ShadeArgs& a, float vtx,
 // with their multiplicities (the same sum of the same per-tap counts); the
 // others run the 25 taps.  Far geometry (world_rad = (2 .. 2.5) * fov /
 // depth below 0.5) takes the short forms.
+//
+// A tap's count is the number of z = -2..2 with d2 > thr[z], thr[z] = RN(depth
+// + z).  Where every thr[z] is depth + z exactly (checked per pixel: only
+// sums that cross a power of two upwards round), that is d2 - depth > z, and
+// the count is clamp(ceil(d2 - depth), -2, 3) + 2: the difference of two
+// depths of at least 20 is exact while it is below 32 and no rounding takes a
+// larger one across 2.  Six instructions a tap instead of ten: 392 -> 247 a
+// pixel where all 25 run, 130 -> 94 for nine (1080p, 1 M triangles: shading
+// alone 95.8 -> 92.7 us).
 struct SsaoTaps {
-  float thr[5];   // depth + z, z = -2..2, as the reference adds them
+  float depth;
   const ShadeArgs* a;
+  __device__ __forceinline__ float load(float wx, float wy) const {
+    return depth_of(ldg(a->depth, (uint32_t)(int)wy * a->v.width + (uint32_t)(int)wx));
+  }
+  // the count less 2
+  __device__ __forceinline__ float exact(float wx, float wy) const {
+    return __builtin_amdgcn_fmed3f(ceilf(load(wx, wy) - depth), -2.f, 3.f);
+  }
   // passing depth tests of the tap at (wx, wy): thr[] is non-decreasing
   // (rounding is monotone), so the count comes from the middle threshold and
   // the pair on its side
-  __device__ __forceinline__ uint32_t at(float wx, float wy) const {
-    const float d2 = depth_of(ldg(a->depth, (uint32_t)(int)wy * a->v.width + (uint32_t)(int)wx));
-    const bool hi = d2 > thr[2];
-    const float ta = hi ? thr[3] : thr[0], tb = hi ? thr[4] : thr[1];
-    return (hi ? 3u : 0u) + (d2 > ta ? 1u : 0u) + (d2 > tb ? 1u : 0u);
+  __device__ __forceinline__ float general(float wx, float wy) const {
+    const float d2 = load(wx, wy);
+    const bool hi = d2 > depth;
+    const float ta = depth + (hi ? 1.f : -2.f), tb = depth + (hi ? 2.f : -1.f);
+    return (hi ? 3.f : 0.f) + (d2 > ta ? 1.f : 0.f) + (d2 > tb ? 1.f : 0.f) - 2.f;
   }
 };
+
+template <bool kExact>
+__device__ __forceinline__ float ssao_count(const SsaoTaps& T, float fsx, float fsy, float world_rad, float m1, float m2,
+                                            float xmax, float ymax) {
+  auto at = [&](float wx, float wy) { return kExact ? T.exact(wx, wy) : T.general(wx, wy); };
+  // the reference sums 1.0f per passing test: every partial sum (at most 125)
+  // is exact, in any order
+  float sum = 0.f;
+  if (__all(m2 == 0.f)) {
+    sum = 25.f * at(clampf(fsx, 1.f, xmax), clampf(fsy, 1.f, ymax));
+  } else if (__all(m1 == 0.f)) {
+    const float xs[3] = {clampf(fsx - m2, 1.f, xmax), clampf(fsx, 1.f, xmax), clampf(fsx + m2, 1.f, xmax)};
+    const float ys[3] = {clampf(fsy - m2, 1.f, ymax), clampf(fsy, 1.f, ymax), clampf(fsy + m2, 1.f, ymax)};
+    const float mult[3] = {1.f, 3.f, 1.f};
+#pragma unroll
+    for (int j = 0; j < 3; j++)
+#pragma unroll
+      for (int i = 0; i < 3; i++) sum += mult[j] * mult[i] * at(xs[i], ys[j]);
+  } else {
+#pragma unroll
+    for (int y = -2; y <= 2; y++) {
+      float oy = roundf((float)y * world_rad);
+      float wy = clampf(fsy + oy, 1.f, ymax);
+#pragma unroll
+      for (int x = -2; x <= 2; x++) {
+        float ox = roundf((float)x * world_rad);
+        sum += at(clampf(fsx + ox, 1.f, xmax), wy);
+      }
+    }
+  }
+  return sum + 50.f;
+}
 
 __device__ __forceinline__ float ssao(const ShadeArgs& a, int sx, int sy) {
   const uint32_t W = a.v.width, H = a.v.height;
@@ -209,38 +257,14 @@ __device__ __forceinline__ float ssao(const ShadeArgs& a, int sx, int sy) {
   if (__all(depth >= 1.f)) world_rad = div_rcp(rad * a.v.fov, depth, rcp_rn(depth));
   else world_rad = rad * a.v.fov / depth;
   float fsx = (float)sx, fsy = (float)sy;
-  SsaoTaps T;
-  T.a = &a;
-#pragma unroll
-  for (int z = 0; z < 5; z++) T.thr[z] = depth + (float)(z - 2);
+  SsaoTaps T{depth, &a};
   const float xmax = (float)W - 2.f, ymax = (float)H - 2.f;
   const float m1 = roundf(world_rad), m2 = roundf(2.f * world_rad);
-  // the reference sums 1.0f per passing test; the count (<= 125) is exact
-  // in binary32, so it is kept as an integer and converted once
-  uint32_t count = 0;
-  if (__all(m2 == 0.f)) {
-    count = 25u * T.at(clampf(fsx, 1.f, xmax), clampf(fsy, 1.f, ymax));
-  } else if (__all(m1 == 0.f)) {
-    const float xs[3] = {clampf(fsx - m2, 1.f, xmax), clampf(fsx, 1.f, xmax), clampf(fsx + m2, 1.f, xmax)};
-    const float ys[3] = {clampf(fsy - m2, 1.f, ymax), clampf(fsy, 1.f, ymax), clampf(fsy + m2, 1.f, ymax)};
-    const uint32_t mult[3] = {1u, 3u, 1u};
-#pragma unroll
-    for (int j = 0; j < 3; j++)
-#pragma unroll
-      for (int i = 0; i < 3; i++) count += mult[j] * mult[i] * T.at(xs[i], ys[j]);
-  } else {
-#pragma unroll
-    for (int y = -2; y <= 2; y++) {
-      float oy = roundf((float)y * world_rad);
-      float wy = clampf(fsy + oy, 1.f, ymax);
-#pragma unroll
-      for (int x = -2; x <= 2; x++) {
-        float ox = roundf((float)x * world_rad);
-        count += T.at(clampf(fsx + ox, 1.f, xmax), wy);
-      }
-    }
-  }
-  float acc = (float)count;
+  const bool exact = depth >= 20.f && (depth + 1.f) - depth == 1.f && (depth + 2.f) - depth == 2.f &&
+                     depth - (depth - 1.f) == 1.f && depth - (depth - 2.f) == 2.f;
+  float acc;
+  if (__all(exact)) acc = ssao_count<true>(T, fsx, fsy, world_rad, m1, m2, xmax, ymax);
+  else acc = ssao_count<false>(T, fsx, fsy, world_rad, m1, m2, xmax, ymax);
   acc = div_rcp(acc, 125.f, kInv125);
   return 1.f - div_rcp(1.f - acc, kSsaoDiv, kInvSsaoDiv);
 }
