@@ -583,7 +583,7 @@ struct TriLds {
   float4 qc[kWave];      // e3, e4, e5, A
   float2 qd[kWave];      // B, C
   // runs of covered columns, compacted
-  uint4 run[kWave];      // pixel - index, x - index, B*y + C, A
+  uint4 run[kWave];      // pixel - index (shadow passes: the row's offset), x - index, B*y + C, A
   uint32_t ent[kMode == RasterMode::Shadow ? 0 : kWave];   // y << 16 | lane
   uint32_t start[kWave];                                   // start[p] == tick: an item begins at index base + p
   // per lane: its triangle's target
@@ -650,6 +650,7 @@ struct RasterTarget {
   uint2* ent;
   uint32_t ent_cap, nent;
   const RasterTri* rast;
+  MapLayout lay;   // shadow passes
 };
 
 // One covered sample per lane (hit lanes): depth d at pixel pix of dst.
@@ -765,8 +766,8 @@ __device__ __forceinline__ void raster_stage(TriLds<kMode, kBatch>& L, RasterTar
       const uint32_t p = lanes_below(runs);
       const uint32_t rp = kBatch ? L.pitch[kBatch ? who : 0] : T.pitch;
       // y and the pitch are below 2^16: the 24-bit multiply is exact
-      L.run[p] = make_uint4(__umul24(y, rp) + xs - begin + (kShadow ? L.face[kShadow ? who : 0] : 0u), xs - begin,
-                            __float_as_uint(rowc), __float_as_uint(pa));
+      const uint32_t row = kShadow ? map_row(T.lay, y) + L.face[kShadow ? who : 0] : __umul24(y, rp) + xs - begin;
+      L.run[p] = make_uint4(row, xs - begin, __float_as_uint(rowc), __float_as_uint(pa));
       if constexpr (!kShadow) L.ent[p] = y << 16 | who;
     }
     // ---- the runs' pixels, one per lane per step
@@ -781,7 +782,7 @@ __device__ __forceinline__ void raster_stage(TriLds<kMode, kBatch>& L, RasterTar
         const uint4 R = L.run[m];
         const uint32_t x = j + R.y;
         d = depth_quant(fmaf(__uint_as_float(R.w), (float)x, __uint_as_float(R.z)));
-        pix = j + R.x;
+        pix = kShadow ? R.x + map_col(T.lay, x) : j + R.x;
         if constexpr (!kShadow) {
           const uint32_t E = L.ent[m];
           xy = x | (E & 0xFFFF0000u);
@@ -840,7 +841,7 @@ __device__ __forceinline__ void raster_stage(TriLds<kMode, kBatch>& L, RasterTar
           d = depth_quant(fmaf(A, x, fmaf(B, y, C)));
           const uint32_t xi = (uint32_t)(int)x, yi = (uint32_t)(int)y;
           xy = xi | yi << 16;
-          pix = __umul24(yi, up) + xi + uf;
+          pix = kShadow ? map_row(T.lay, yi) + map_col(T.lay, xi) + uf : __umul24(yi, up) + xi;
         }
       }
       put_sample<kMode, kBatch>(T, hit, d, pix, xy, rec0 + (uint32_t)k, to, ti);
@@ -984,7 +985,8 @@ __global__ void __launch_bounds__(256) k_raster(PassArgs a, ShadowTarget sh) {
     if (Ls.ent.cnt) id_from_entries<kBatch>(a, Ls, wave0, nwaves, min(ent_chunks, nchunks), ent_cap);
   }
   RasterTarget T{kMode == RasterMode::Shadow ? sh.L : a.view0.v.width,
-                 kMode == RasterMode::Shadow ? sh.map : a.view0.depth, a.view0.idkey, nullptr, ent_cap, 0u, Ls.rast};
+                 kMode == RasterMode::Shadow ? sh.map : a.view0.depth, a.view0.idkey, nullptr, ent_cap, 0u, Ls.rast,
+                 map_layout(sh.L)};
   for (uint32_t chunk = wave0; chunk < nchunks; chunk += nwaves) {
     // the chunk's partition: the first whose inclusive chunk count passes it
     const uint32_t part = (uint32_t)__popcll(__ballot(part_chunks <= chunk));
@@ -1221,7 +1223,7 @@ __global__ void __launch_bounds__(kShadowPreThreads) k_prearrange_shadow(const T
   if (t < (uint32_t)kMaxShadowGroup) S.n_items[t] = 0;
   W.start[lane] = 0u;
   uint32_t tick = 0;
-  RasterTarget T{L, target.map, nullptr, nullptr, 0u, 0u, nullptr};
+  RasterTarget T{L, target.map, nullptr, nullptr, 0u, 0u, nullptr, map_layout(L)};
   __syncthreads();
   for (uint32_t li = 0; li < group.n; li++) {
     const f3 lpos = mk3(group.pos[li][0], group.pos[li][1], group.pos[li][2]);
@@ -1380,6 +1382,24 @@ hipError_t launch_shadow_group(Scene* sc, const float (*lpos)[3], const uint32_t
   a.lists = lists;
   hipLaunchKernelGGL((k_raster<RasterMode::Shadow, kOpSizeLight, false>), dim3(device_cu_count() * 8), dim3(256), 0, s,
                      a, target);
+  return hipGetLastError();
+}
+
+// Strips of four map rows from blocks of 4 x 4 texels to row order, four
+// texels a work item.
+__global__ void __launch_bounds__(256) k_map_rows(const uint4* __restrict__ map, uint32_t L, uint32_t n,
+                                                  uint4* __restrict__ rows) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;   // below 2^22
+  if (i >= n) return;
+  const uint32_t strip = i / L, q = i % L, across = L / 4u;
+  rows[i] = map[strip * L + (q % across) * 4u + q / across];
+}
+
+hipError_t launch_map_rows(const uint32_t* map, uint32_t L, uint32_t strips, uint32_t* rows, hipStream_t s) {
+  const uint32_t n = strips * L;
+  if (n)
+    hipLaunchKernelGGL(k_map_rows, dim3((n + 255) / 256), dim3(256), 0, s, reinterpret_cast<const uint4*>(map), L, n,
+                       reinterpret_cast<uint4*>(rows));
   return hipGetLastError();
 }
 

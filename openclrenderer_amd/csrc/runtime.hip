@@ -847,17 +847,41 @@ int ocr_shadow_pass(ocr_scene* s, void* stream) {
   return OCR_OK;
 }
 
+// n cube maps of a scene to the host, row by row: maps of 4 x 4 blocks are put
+// in order on the device, a part at a time through the context's staging.
+static int read_maps(Scene* s, const uint32_t* maps, uint32_t n, uint32_t* out) {
+  const uint32_t L = s->lbuf_dim;
+  const size_t total = (size_t)6 * L * L * n;
+  if (map_layout(L).kx == 0u) {
+    OCR_HIP_CHECK(hipMemcpy(out, maps, total * 4, hipMemcpyDeviceToHost));
+    return OCR_OK;
+  }
+  constexpr size_t kPart = 16u << 20;
+  const size_t strip = (size_t)4 * L, strips = total / strip;   // four rows each
+  const size_t part = std::min(strips, kPart / (strip * 4));
+  std::lock_guard<std::mutex> lk(s->ctx->stage_mu);
+  uint8_t* stage = nullptr;
+  const int rc = stage_buffer(s->ctx, part * strip * 4, &stage);
+  if (rc) return rc;
+  uint32_t* const rows = reinterpret_cast<uint32_t*>(stage);
+  for (size_t i = 0; i < strips; i += part) {
+    const size_t k = std::min(part, strips - i);
+    OCR_HIP_CHECK(launch_map_rows(maps + i * strip, L, (uint32_t)k, rows, nullptr));
+    OCR_HIP_CHECK(hipMemcpy(out + i * strip, rows, k * strip * 4, hipMemcpyDeviceToHost));
+  }
+  return OCR_OK;
+}
+
 int ocr_scene_read_shadow_maps(ocr_scene* s, uint32_t* dynamic_maps, uint32_t* static_maps) {
   if (!s) return fail(OCR_ERR_INVALID, "ocr_scene_read_shadow_maps: null scene");
   OCR_HIP_CHECK(hipSetDevice(s->ctx->device));
   OCR_HIP_CHECK(hipDeviceSynchronize());
   uint32_t ov = 0;
   OCR_HIP_CHECK(hipMemcpy(&ov, s->sh_counters + kOverflow, 4, hipMemcpyDeviceToHost));
-  const size_t per = (size_t)6 * s->lbuf_dim * s->lbuf_dim * 4;
-  if (dynamic_maps && s->n_shadow)
-    OCR_HIP_CHECK(hipMemcpy(dynamic_maps, s->shadow_maps, per * s->n_shadow, hipMemcpyDeviceToHost));
-  if (static_maps && s->n_static)
-    OCR_HIP_CHECK(hipMemcpy(static_maps, s->static_maps, per * s->n_static, hipMemcpyDeviceToHost));
+  int rc = OCR_OK;
+  if (dynamic_maps && s->n_shadow) rc = read_maps(s, s->shadow_maps, s->n_shadow, dynamic_maps);
+  if (!rc && static_maps && s->n_static) rc = read_maps(s, s->static_maps, s->n_static, static_maps);
+  if (rc) return rc;
   if (ov) return fail(OCR_ERR_UNSUPPORTED, "shadow pass: more raster samples than one pass can hold");
   return OCR_OK;
 }

@@ -284,7 +284,7 @@ struct ShadowSetup {
   float px, py;      // clamped position on the face
   float dpth;        // the pixel's depth from the light
   float bias;
-  uint32_t face_off; // (iy - 1) * L + (ix - 1) within the face
+  uint32_t ix, iy;   // the first tap: one before the position's texel on each axis
   int face;
 };
 
@@ -302,8 +302,8 @@ __device__ __forceinline__ ShadowSetup shadow_setup(const ShadeArgs& a, f3 lpos,
   s.dpth = post.z;
   s.px = clampf(post.x, 3.f, lf - 4.f);
   s.py = clampf(post.y, 3.f, lf - 4.f);
-  const int ix = (int)s.px, iy = (int)s.py;
-  s.face_off = (uint32_t)(iy - 1) * L + (uint32_t)(ix - 1);
+  s.ix = (uint32_t)((int)s.px - 1);
+  s.iy = (uint32_t)((int)s.py - 1);
   float acos_res = rational_acos(clampf(dot(normal, ptl_n), 0.05f, 0.95f));
   if (acos_res >= kTanOneFrom) {
     s.bias = (float)kShadowBias;
@@ -321,13 +321,17 @@ template <bool kCount>
 __device__ __forceinline__ float shadow_taps(const ShadeArgs& a, const ShadowSetup& s,
                                              gptr<const uint32_t> buf, uint32_t* touch_bits, int shnum) {
   const uint32_t L = a.L;
-  const uint32_t map_off = ((uint32_t)s.face + (uint32_t)shnum * 6u) * L * L + s.face_off;
+  const uint32_t map_off = ((uint32_t)s.face + (uint32_t)shnum * 6u) * L * L;
+  const MapLayout lay = map_layout(L);
   uint32_t cond = 0;   // 4x4 taps, bit (y+1)*4 + (x+1)
+  uint32_t col[4];
+#pragma unroll
+  for (int x = 0; x < 4; x++) col[x] = map_col(lay, s.ix + (uint32_t)x);
 #pragma unroll
   for (int y = 0; y < 4; y++)
 #pragma unroll
     for (int x = 0; x < 4; x++) {
-      const uint32_t t = map_off + (uint32_t)y * L + (uint32_t)x;
+      const uint32_t t = map_off + map_row(lay, s.iy + (uint32_t)y) + col[x];
       touch<kCount>(touch_bits, t);
       float ldp = depth_of(ldg(buf, t));
       cond |= (s.dpth > ldp + s.bias ? 1u : 0u) << (y * 4 + x);
