@@ -49,7 +49,7 @@ namespace ocr {
 // other's loads, barriers and allocation atomic (16-light shadow pass over
 // 4 M triangles 5.09 -> 4.82 ms).
 constexpr int kPreThreadsOne = 512;
-constexpr int kShadowPreThreads = 512;
+constexpr int kShadowPreThreads = 256;
 
 template <int kWaves>
 struct BlockAllocLds {
@@ -174,16 +174,18 @@ __device__ __forceinline__ uint32_t triangle_samples(const RasterTri& t, float m
   return s > (uint64_t)kMaxTriSamples ? kMaxTriSamples : (uint32_t)s;
 }
 
-// Clip/cull/count of one projected triangle (cl2.cl:4344-4380): returns the
-// reference's fragment count ceil(bbox_area / op_size), 0 if culled.
-__device__ __forceinline__ uint32_t cull_count(const f3 p[3], float ew, float eh, bool two_sided,
-                                               int op_size, float& rconst) {
+// Culling of one projected triangle (cl2.cl:4344-4380): whether it is kept.
+__device__ __forceinline__ bool piece_kept(const f3 p[3], float ew, float eh, bool two_sided) {
   bool valid = two_sided || front_facing(p[0], p[1], p[2]);
   bool cond = (p[0].x < 0 && p[1].x < 0 && p[2].x < 0) ||
               (p[0].x >= ew && p[1].x >= ew && p[2].x >= ew) ||
               (p[0].y < 0 && p[1].y < 0 && p[2].y < 0) ||
               (p[0].y >= eh && p[1].y >= eh && p[2].y >= eh);
-  if (!valid || cond) return 0;
+  return valid && !cond;
+}
+
+// The reference's fragment count ceil(bbox_area / op_size) of one kept.
+__device__ __forceinline__ uint32_t frag_count(const f3 p[3], float ew, float eh, int op_size, float& rconst) {
   f3 xpv = mk3(roundf(p[0].x), roundf(p[1].x), roundf(p[2].x));
   f3 ypv = mk3(roundf(p[0].y), roundf(p[1].y), roundf(p[2].y));
   rconst = rconstant(xpv, ypv);
@@ -314,19 +316,15 @@ struct Piece {
   uint32_t nf, seen, ns;
 };
 
-// Project, cull, count and set up a clipped triangle.  A piece whose walk
+// Count and set up a projected triangle P.p that is kept.  A piece whose walk
 // visits exactly its box gets the box form: one sample per box pixel, mapped
 // without the walk's fragment arithmetic.  A piece of zero rounded area with
 // exact edge sums covers no pixel (s >= 0 and t >= 0 leave no s + t < 0): it
 // counts, but is not listed.  Of the 1080p, 1 M-triangle frame's 446,000
 // pieces 105,000 are such, of a 1024^2 cube face's small ones in that scene
 // half.
-__device__ __forceinline__ void cut_piece(const f3 tri[3], float fovc, float ew, float eh, bool two_sided, int op,
-                                          Piece& P) {
-  P.nf = P.seen = P.ns = 0u;
-#pragma unroll
-  for (int i = 0; i < 3; i++) P.p[i] = depth_project_clipped(tri[i], ew, eh, fovc);
-  P.nf = cull_count(P.p, ew, eh, two_sided, op, P.rc);
+__device__ __forceinline__ void setup_piece(float ew, float eh, int op, Piece& P) {
+  P.nf = frag_count(P.p, ew, eh, op, P.rc);
   if (!P.nf) return;
   raster_setup(P.p, P.rc, ew, eh, P.rt, P.my);
   // the box holds at most 16,000,000 pixels (frames and cube faces), an exact
@@ -340,6 +338,33 @@ __device__ __forceinline__ void cut_piece(const f3 tri[3], float fovc, float ew,
   P.seen = box ? (uint32_t)area : triangle_samples(P.rt, P.my, op, P.nf);
   const bool empty = P.rt.ek[6] == 0.f && span_exact(P.rt.ek, P.rt.min_x + P.rt.w, P.my);
   P.ns = empty ? 0u : P.seen;
+}
+
+// Project, cull, count and set up a clipped triangle.
+__device__ __forceinline__ void cut_piece(const f3 tri[3], float fovc, float ew, float eh, bool two_sided, int op,
+                                          Piece& P) {
+  P.nf = P.seen = P.ns = 0u;
+#pragma unroll
+  for (int i = 0; i < 3; i++) P.p[i] = depth_project_clipped(tri[i], ew, eh, fovc);
+  if (piece_kept(P.p, ew, eh, two_sided)) setup_piece(ew, eh, op, P);
+}
+
+// Whether setup_piece finds P.p empty beyond doubt, in a quarter of its
+// instructions: its vertices round, none of them from halfway (there roundf
+// and this rounding may differ), to integers of zero area in [0, 1182], where
+// every edge sum of span_exact is at most 3 * 1182^2 and their sum below 2^23.
+__device__ __forceinline__ bool piece_empty(const f3 p[3]) {
+  float x[3], y[3], off = 0.f;
+#pragma unroll
+  for (int i = 0; i < 3; i++) {
+    x[i] = rintf(p[i].x);
+    y[i] = rintf(p[i].y);
+    off = max3f(off, fabsf(p[i].x - x[i]), fabsf(p[i].y - y[i]));
+  }
+  const float lo = fminf(min3f(x[0], x[1], x[2]), min3f(y[0], y[1], y[2]));
+  const float hi = fmaxf(max3f(x[0], x[1], x[2]), max3f(y[0], y[1], y[2]));
+  return off < 0.5f && lo >= 0.f && hi <= 1150.f &&
+         (x[1] - x[0]) * (y[2] - y[0]) == (x[2] - x[0]) * (y[1] - y[0]);
 }
 
 // Appends the work items' cut pieces that hold samples with their sample
@@ -1085,19 +1110,22 @@ hipError_t launch_id(const PassArgs& a, int blocks_per_cu, hipStream_t s) {
 struct FaceTable { SinCos f[6]; };
 
 // prearrange_realtime_shadowing (cl2.cl:4419-4636) and kernel1's shadow
-// raster (cl2.cl:4638-4700) for a group of lights in one launch.  Phase 1:
-// one triangle per work item — its world-space vertices into LDS, read from
-// HBM once for the whole group.  Then for each light of the group: the faces
-// the vertices fall in (ret_cubeface), each (triangle, face) pair appended
-// to a block-local work list in LDS, and phase 2: the pairs, one per work
-// item per round, clipped, projected, culled and set up for their face.
-// Pieces become records, key = slot * 6 + face with slot the light's cube
-// map in the group's maps, for one raster launch over the whole group;
-// pieces of at most local_max samples, and any that no longer fit the list,
-// are rasterised at once by the wavefront, their samples spread over its
-// lanes.  (Looping over the six faces per
-// triangle would leave most lanes idle: a triangle touches one to three
-// faces.)
+// raster (cl2.cl:4638-4700) for a group of lights in one launch, each
+// wavefront on its own with 64 triangles, read from HBM once for the whole
+// group.  For each light: the faces a triangle's vertices fall in
+// (ret_cubeface), one to three of the six, each (triangle, face) pair an item
+// in the wavefront's list.  Whenever 64 items wait, of whatever lights, they
+// are clipped, projected and culled, one per lane; the pieces that are left (on
+// small faces half of them round to nothing) wait in registers until 64 of them
+// are together, are set up, and become records, key = slot * 6 + face with slot
+// the light's cube map in the group's maps, for one raster launch over the
+// whole group; pieces of at most local_max samples, and any that no longer fit
+// the list, are rasterised at once by the wavefront.
+// Half of a light's items face away, so a block that gathered the items of one
+// light at a time left half of its wavefronts waiting at each light's barrier,
+// and every second piece of a draw was an empty one: 500 M -> 407 M vector
+// instructions, 1.26 -> 0.85 ms (16 lights, 4 M triangles), where issuing the
+// instructions takes 0.73 ms.
 constexpr int kMaxShadowGroup = 16;
 struct ShadowGroup {
   float pos[kMaxShadowGroup][3];
@@ -1143,15 +1171,33 @@ __device__ __forceinline__ bool wave_alloc_fit(const Lists& L, uint32_t ncut, ui
 }
 
 using ShadowStage = TriLds<RasterMode::Shadow, false>;
+struct PieceSwap {
+  float4 a[kWave], b[kWave];   // p[0], p[1].x; p[1].yz, p[2].xy
+  float2 c[kWave];             // p[2].z, the map's key
+  __device__ __forceinline__ void put(uint32_t s, const f3 p[3], uint32_t key) {
+    a[s] = make_float4(p[0].x, p[0].y, p[0].z, p[1].x);
+    b[s] = make_float4(p[1].y, p[1].z, p[2].x, p[2].y);
+    c[s] = make_float2(p[2].z, __uint_as_float(key));
+  }
+  __device__ __forceinline__ void get(uint32_t s, f3 p[3], uint32_t& key) const {
+    const float4 u = a[s], v = b[s];
+    const float2 w = c[s];
+    p[0] = mk3(u.x, u.y, u.z);
+    p[1] = mk3(u.w, v.x, v.y);
+    p[2] = mk3(v.z, v.w, w.x);
+    key = __float_as_uint(w.y);
+  }
+};
+static_assert(sizeof(PieceSwap) <= offsetof(ShadowStage, start), "the stage's start[] keeps its marks");
 
 // Whether front_facing is false beyond doubt for a triangle that lies in one
 // cube face of a light: nrm its normal, edge the largest component of its
 // edges, rel0 its first vertex from the light, near and far the smallest and
 // largest distance along the face's axis (the largest component of a vertex).
 // Per 64 (triangle, face) pairs the clip, projection and set-up that this
-// saves are ~400 instructions; half of all pairs face away.  With the faces
-// found by selects from vertices kept in registers the pass issues 606 M ->
-// 498 M vector instructions (16 lights, 4 M triangles; 1.48 -> 1.31 ms).
+// saves are ~400 instructions; half of all pairs face away: with the faces
+// found by selects from vertices kept in registers 606 M -> 498 M vector
+// instructions a pass (16 lights, 4 M triangles).
 //
 // With u = 2^-24, L texels a side and e = edge / near: a projected coordinate
 // is (L/2) x/z + L/2 with |x| <= z, formed within 10 L u (u from the difference
@@ -1170,11 +1216,20 @@ __device__ __forceinline__ bool faces_away(f3 nrm, float edge, f3 rel0, float ne
 }
 
 struct ShadowLds {
-  float wpos[kShadowPreThreads][9];
-  // (local triangle << 4 | two_sided << 3 | face) work items, one list per
-  // light, two lists alternating
-  uint32_t items[2][kShadowPreThreads * 3];
-  uint32_t n_items[kMaxShadowGroup];
+  float lpos[kMaxShadowGroup][3];
+  uint32_t key[kMaxShadowGroup];   // of the light's first face
+  SinCos face[6];
+  struct Wave {
+    float wpos[kWave][9];
+    // light << 16 | lane << 4 | two_sided << 3 | face: fewer than 64 left over
+    // and up to three of each lane
+    uint32_t items[4 * kWave];
+    // pieces on their way between lanes share the stage's place
+    union {
+      ShadowStage stage;
+      PieceSwap swap;
+    };
+  } wave[kShadowPreThreads / kWave];
 };
 
 __global__ void __launch_bounds__(kShadowPreThreads) k_prearrange_shadow(const TriPos* __restrict__ world, uint32_t ntri,
@@ -1183,15 +1238,19 @@ __global__ void __launch_bounds__(kShadowPreThreads) k_prearrange_shadow(const T
                                                            int only_static, uint32_t local_max, FaceTable ft,
                                                            Lists lists) {
   __shared__ ShadowLds S;
-  __shared__ ShadowStage stage_all[kShadowPreThreads / kWave];
-  ShadowStage& W = stage_all[threadIdx.x / kWave];
   const uint32_t t = threadIdx.x;
   const int lane = t & (kWave - 1);
-  const uint32_t wave = t / kWave;
+  ShadowLds::Wave& M = S.wave[t / kWave];
+  ShadowStage& W = M.stage;
+  PieceSwap& Q = M.swap;
   const uint32_t id = blockIdx.x * blockDim.x + t;
+  if (t < 3u * kMaxShadowGroup) (&S.lpos[0][0])[t] = (&group.pos[0][0])[t];
+  if (t < (uint32_t)kMaxShadowGroup) S.key[t] = group.slot[t] * 6u;
+  if (t < 6u) S.face[t] = ft.f[t];
+  __syncthreads();   // the only one: the wavefronts are independent from here
   const uint32_t L = target.L;
   const float ew = (float)L, eh = (float)L, efov = (float)L / 2.0f;
-  // ---- phase 1: the triangle, once for every light of the group
+  // ---- the triangle, once for every light of the group
   bool live = false;
   uint32_t two_sided = 0;
   f3 wp = mk3(0.f, 0.f, 0.f);
@@ -1207,9 +1266,9 @@ __global__ void __launch_bounds__(kShadowPreThreads) k_prearrange_shadow(const T
 #pragma unroll
         for (int k = 0; k < 3; k++) {
           wv[k] = mk3(T.p[3 * k], T.p[3 * k + 1], T.p[3 * k + 2]);
-          S.wpos[t][3 * k] = wv[k].x;
-          S.wpos[t][3 * k + 1] = wv[k].y;
-          S.wpos[t][3 * k + 2] = wv[k].z;
+          M.wpos[lane][3 * k] = wv[k].x;
+          M.wpos[lane][3 * k + 1] = wv[k].y;
+          M.wpos[lane][3 * k + 2] = wv[k].z;
         }
         two_sided = (G.flags & OCR_FEATURE_TWO_SIDED) > 0 ? 1u : 0u;
       }
@@ -1220,115 +1279,145 @@ __global__ void __launch_bounds__(kShadowPreThreads) k_prearrange_shadow(const T
   const f3 nrm = cross(a, b);
   const float edge = max3f(max3f(fabsf(a.x), fabsf(a.y), fabsf(a.z)), max3f(fabsf(b.x), fabsf(b.y), fabsf(b.z)),
                            max3f(fabsf(c.x), fabsf(c.y), fabsf(c.z)));
-  if (t < (uint32_t)kMaxShadowGroup) S.n_items[t] = 0;
   W.start[lane] = 0u;
   uint32_t tick = 0;
   RasterTarget T{L, target.map, nullptr, nullptr, 0u, 0u, nullptr, map_layout(L)};
-  __syncthreads();
-  for (uint32_t li = 0; li < group.n; li++) {
-    const f3 lpos = mk3(group.pos[li][0], group.pos[li][1], group.pos[li][2]);
-    const uint32_t key0 = group.slot[li] * 6u;
-    uint32_t* const items = S.items[li & 1u];
-    // Light li's items go to list li & 1.  Every wavefront has finished
-    // light li - 2's rounds on that list before it passed light li - 1's
-    // barrier, and writes here come after that barrier.
-    uint32_t touched = 0;
-    const f3 to_obj = wp - lpos;
-    if (live && !(dot(to_obj, to_obj) > kDepthFarSq)) {
-      float near = 3.0e38f, far = 0.f;
-      f3 rel0 = mk3(0.f, 0.f, 0.f);
+  // projected pieces that wait for a full wavefront: one in each lane below nq
+  f3 qp[3] = {wp, wp, wp};
+  uint32_t qkey = 0, nq = 0;
+  auto draw = [&](bool have) {
+    Piece P;
+    P.nf = P.seen = P.ns = 0u;
+    if (have) {
 #pragma unroll
-      for (int k = 0; k < 3; k++) {
-        const f3 rel = wv[k] - lpos;
-        if (k == 0) rel0 = rel;
-        const float ax = fabsf(rel.x), ay = fabsf(rel.y), az = fabsf(rel.z);
-        const float z = max3f(ax, ay, az);
-        near = fminf(near, z);
-        far = fmaxf(far, z);
-        // the bit of ret_cubeface's answer (cl2.cl:1745-1790), by selects
-        const bool cx = (ax >= ay) & (ax >= az), cy = (ay > ax) & (ay >= az);
-        const bool cz = (az > ax) & (az > ay) & (rel.z < 0.f);
-        const uint32_t bz = cz ? 1u << 2 : 1u, by = rel.y < 0.f ? 1u << 1 : 1u << 3, bx = rel.x < 0.f ? 1u << 4 : 1u << 5;
-        touched |= cx ? bx : (cy ? by : bz);
+      for (int k = 0; k < 3; k++) P.p[k] = qp[k];
+      setup_piece(ew, eh, kOpSizeLight, P);
+    }
+    // pieces above local_max samples to the list, in allocations of at
+    // most kShadowWaveSamples samples (each takes the lanes whose running
+    // sum fits, at least the first waiting lane); pieces of the list's
+    // failed allocations and the small ones rasterised here
+    const uint32_t mine = P.ns > local_max ? P.ns : 0u;   // < 2^24
+    bool waiting = mine > 0, listed = false;
+    while (__ballot(waiting)) {
+      const uint32_t upto = wave_incl_scan(waiting ? mine : 0u);
+      const bool take = waiting && upto <= kShadowWaveSamples;
+      uint32_t c, smp;
+      const bool ok = wave_alloc_fit(lists, take ? 1u : 0u, take ? mine : 0u, c, smp);
+      if (take) {
+        waiting = false;
+        listed = ok;
+        if (ok) {
+          P.rt.key = qkey | (P.rt.key & kKeyBoxForm);
+          P.rt.sample_begin = smp;
+          lists.rast[c] = P.rt;
+        }
       }
-      // certainly facing away: no piece of it would pass the culling
-      if (!two_sided && (touched & (touched - 1u)) == 0u && faces_away(nrm, edge, rel0, near, far)) touched = 0u;
     }
-    const uint32_t mine = (uint32_t)__popc(touched);
-    const uint32_t incl = wave_incl_scan(mine);
-    const uint32_t wtotal = wave_total(incl);
-    uint32_t wbase = 0;
-    if (lane == 0 && wtotal) wbase = atomicAdd(&S.n_items[li], wtotal);
-    wbase = (uint32_t)__builtin_amdgcn_readfirstlane((int)wbase);
-    uint32_t slot = wbase + incl - mine;
-    // one to three faces, nearly always one
-    while (touched) {
-      const uint32_t f = (uint32_t)__ffs((int)touched) - 1u;
-      touched &= touched - 1u;
-      items[slot++] = t << 4 | two_sided << 3 | f;
+    // The rest, straight into the maps: a map keeps the minimum depth of
+    // its samples, so the order in which they arrive does not matter.
+    const uint32_t n = listed ? 0u : P.ns;
+    if (__any(n != 0u))
+      raster_stage<RasterMode::Shadow, kOpSizeLight, false>(W, T, P.rt, (uint32_t)lane, n ? 0u : 1u, n, qkey * L * L,
+                                                            nullptr, 0u, nullptr, tick);
+  };
+  uint32_t nit = 0;
+  for (uint32_t li = 0; li <= group.n; li++) {   // and a last turn for what is left
+    if (li < group.n) {
+      // ---- the faces that the lane's triangle may fall on
+      const f3 lpos = mk3(group.pos[li][0], group.pos[li][1], group.pos[li][2]);
+      uint32_t touched = 0;
+      const f3 to_obj = wp - lpos;
+      if (live && !(dot(to_obj, to_obj) > kDepthFarSq)) {
+        float near = 3.0e38f, far = 0.f;
+        f3 rel0 = mk3(0.f, 0.f, 0.f);
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+          const f3 rel = wv[k] - lpos;
+          if (k == 0) rel0 = rel;
+          const float ax = fabsf(rel.x), ay = fabsf(rel.y), az = fabsf(rel.z);
+          const float z = max3f(ax, ay, az);
+          near = fminf(near, z);
+          far = fmaxf(far, z);
+          // the bit of ret_cubeface's answer (cl2.cl:1745-1790), by selects
+          const bool cx = (ax >= ay) & (ax >= az), cy = (ay > ax) & (ay >= az);
+          const bool cz = (az > ax) & (az > ay) & (rel.z < 0.f);
+          const uint32_t bz = cz ? 1u << 2 : 1u, by = rel.y < 0.f ? 1u << 1 : 1u << 3, bx = rel.x < 0.f ? 1u << 4 : 1u << 5;
+          touched |= cx ? bx : (cy ? by : bz);
+        }
+        // certainly facing away: no piece of it would pass the culling
+        if (!two_sided && (touched & (touched - 1u)) == 0u && faces_away(nrm, edge, rel0, near, far)) touched = 0u;
+      }
+      const uint32_t mine = (uint32_t)__popc(touched);
+      const uint32_t incl = wave_incl_scan(mine);
+      uint32_t slot = nit + incl - mine;
+      nit += wave_total(incl);
+      // one to three faces, nearly always one
+      while (touched) {
+        const uint32_t f = (uint32_t)__ffs((int)touched) - 1u;
+        touched &= touched - 1u;
+        M.items[slot++] = li << 16 | (uint32_t)lane << 4 | two_sided << 3 | f;
+      }
+      wave_lds_sync();
     }
-    __syncthreads();
-    const uint32_t n_items = S.n_items[li];
-    // ---- phase 2: 64 work items per wavefront per round, the wavefronts
-    // independent of each other
-    for (uint32_t r0 = wave * kWave; r0 < n_items; r0 += kShadowPreThreads) {
+    // ---- 64 items at a time, the last ones first
+    while (nit >= (uint32_t)kWave || (li == group.n && nit)) {
+      const uint32_t cnt = min(nit, (uint32_t)kWave);
+      nit -= cnt;
       f3 tris[2][3];
       int num = 0;
-      uint32_t face = 0;
+      uint32_t key = 0;
       bool both = false;
-      if (r0 + lane < n_items) {
-        const uint32_t it = items[r0 + lane];
-        const uint32_t lt = it >> 4;
-        face = it & 7u;
+      if ((uint32_t)lane < cnt) {
+        const uint32_t it = M.items[nit + (uint32_t)lane];
+        const uint32_t lt = (it >> 4) & 63u, face = it & 7u, l = it >> 16;
         both = ((it >> 3) & 1u) != 0u;
         f3 w[3];
 #pragma unroll
-        for (int k = 0; k < 3; k++) w[k] = mk3(S.wpos[lt][3 * k], S.wpos[lt][3 * k + 1], S.wpos[lt][3 * k + 2]);
-        num = face_clip(w, lpos, ft.f[face], tris);
+        for (int k = 0; k < 3; k++) w[k] = mk3(M.wpos[lt][3 * k], M.wpos[lt][3 * k + 1], M.wpos[lt][3 * k + 2]);
+        key = S.key[l] + face;
+        num = face_clip(w, mk3(S.lpos[l][0], S.lpos[l][1], S.lpos[l][2]), S.face[face], tris);
       }
-      const uint32_t key = key0 + face;
-      const uint32_t first_texel = key * target.L * target.L;
       // the second piece exists only where the near plane cuts
 #pragma unroll 1
       for (int i = 0; i < 2; i++) {
         if (!__any(num > i)) break;
-        Piece P;
-        P.ns = 0u;
-        if (num > i) {
-          const f3 tri[3] = {i == 0 ? tris[0][0] : tris[1][0], i == 0 ? tris[0][1] : tris[1][1],
-                             i == 0 ? tris[0][2] : tris[1][2]};
-          cut_piece(tri, efov, ew, eh, both, kOpSizeLight, P);
+        f3 p[3] = {wp, wp, wp};
+        bool keep = num > i;
+        if (keep) {
+#pragma unroll
+          for (int k = 0; k < 3; k++) p[k] = depth_project_clipped(i == 0 ? tris[0][k] : tris[1][k], ew, eh, efov);
+          keep = piece_kept(p, ew, eh, both) && !piece_empty(p);
         }
-        // pieces above local_max samples to the list, in allocations of at
-        // most kShadowWaveSamples samples (each takes the lanes whose running
-        // sum fits, at least the first waiting lane); pieces of the list's
-        // failed allocations and the small ones rasterised here
-        const uint32_t mine = P.ns > local_max ? P.ns : 0u;   // < 2^24
-        bool waiting = mine > 0, listed = false;
-        while (__ballot(waiting)) {
-          const uint32_t upto = wave_incl_scan(waiting ? mine : 0u);
-          const bool take = waiting && upto <= kShadowWaveSamples;
-          uint32_t c, smp;
-          const bool ok = wave_alloc_fit(lists, take ? 1u : 0u, take ? mine : 0u, c, smp);
-          if (take) {
-            waiting = false;
-            listed = ok;
-            if (ok) {
-              P.rt.key = key | (P.rt.key & kKeyBoxForm);
-              P.rt.sample_begin = smp;
-              lists.rast[c] = P.rt;
-            }
+        // the kept pieces, compacted: those that the waiting ones leave room
+        // for join them, and a full wavefront is drawn before the rest do
+        const unsigned long long kept = __ballot(keep);
+        const uint32_t n = (uint32_t)__popcll(kept);
+        if (keep) Q.put(lanes_below(kept), p, key);
+        wave_lds_sync();
+        const uint32_t from = (uint32_t)lane - nq;
+        if (from < n) Q.get(from, qp, qkey);
+        nq += n;
+        if (nq >= (uint32_t)kWave) {
+          f3 rp[3] = {wp, wp, wp};
+          uint32_t rkey = 0;
+          nq -= kWave;
+          const bool rest = (uint32_t)lane < nq;
+          if (rest) Q.get(n - nq + (uint32_t)lane, rp, rkey);
+          wave_lds_sync();
+          draw(true);
+          if (rest) {
+#pragma unroll
+            for (int k = 0; k < 3; k++) qp[k] = rp[k];
+            qkey = rkey;
           }
         }
-        // The rest, straight into the maps: a map keeps the minimum depth of
-        // its samples, so the order in which they arrive does not matter.
-        const uint32_t n = listed ? 0u : P.ns;
-        if (__any(n != 0u))
-          raster_stage<RasterMode::Shadow, kOpSizeLight, false>(W, T, P.rt, (uint32_t)lane, n ? 0u : 1u, n,
-                                                                first_texel, nullptr, 0u, nullptr, tick);
+        wave_lds_sync();
       }
+      wave_lds_sync();   // items[] is rewritten
     }
   }
+  if (nq) draw((uint32_t)lane < nq);
 }
 
 // A shadow pass's counters: the render words and every partition's packed
