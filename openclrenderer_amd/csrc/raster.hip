@@ -678,6 +678,16 @@ struct RasterTarget {
   MapLayout lay;   // shadow passes
 };
 
+// A pointer to device memory.  A batch's targets come from tables and LDS, where
+// the compiler cannot tell; through generic pointers their loads and atomics
+// count as LDS operations too, so that every later wait for LDS also waits for
+// memory (12-view batch: depth pass 117.7 -> 115.9 us, ids 91.4 ->
+// 89.6, 453 -> 451 in all).
+template <typename T>
+__device__ __forceinline__ __attribute__((address_space(1))) T* dev_ptr(T* p) {
+  return (__attribute__((address_space(1))) T*)(uintptr_t)p;
+}
+
 // One covered sample per lane (hit lanes): depth d at pixel pix of dst.
 // Called wave-uniformly.
 template <RasterMode kMode, bool kBatch>
@@ -686,9 +696,10 @@ __device__ __forceinline__ void put_sample(RasterTarget& T, bool hit, uint32_t d
   bool keep = false;
   if (hit) {
     if constexpr (kMode == RasterMode::Id) {
-      const uint32_t val = dst[pix];
+      const uint32_t val = dev_ptr(dst)[pix];
       if (d > val - kBufError && d < val + kBufError)
-        atomicMax(&ids[pix], ((unsigned long long)((T.rast[rec].key & ~kKeyBoxForm) + 1u) << 32) | rec);
+        __hip_atomic_fetch_max(dev_ptr(ids) + pix, ((unsigned long long)((T.rast[rec].key & ~kKeyBoxForm) + 1u) << 32) | rec,
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     } else {
       // The L2 performs atomics at ~26.6 G cache-line operations/s; a plain
       // load first drops the samples that cannot win (the stored depth only
@@ -702,8 +713,8 @@ __device__ __forceinline__ void put_sample(RasterTarget& T, bool hit, uint32_t d
         val = *g;
         if (d < val) __hip_atomic_fetch_min(g, d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       } else {
-        val = dst[pix];
-        if (d < val) atomicMin(&dst[pix], d);
+        val = dev_ptr(dst)[pix];
+        if (d < val) __hip_atomic_fetch_min(dev_ptr(dst) + pix, d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
       // a sample at or beyond val + BUF_ERROR stays outside the id pass's
       // window of the final depth (<= val) unless val + BUF_ERROR wraps
@@ -961,13 +972,14 @@ __device__ __forceinline__ void id_from_entries(const PassArgs& a, const Lists& 
 #pragma unroll
       for (int i = 0; i < kPer; i++) {
         const uint32_t e = e0 + (uint32_t)lane + (uint32_t)(i * kWave);
-        if (e < n) val[i] = dep[i][pix[i]];
+        if (e < n) val[i] = dev_ptr(dep[i])[pix[i]];
       }
 #pragma unroll
       for (int i = 0; i < kPer; i++) {
         const uint32_t e = e0 + (uint32_t)lane + (uint32_t)(i * kWave);
         if (e < n && d[i] > val[i] - kBufError && d[i] < val[i] + kBufError)
-          atomicMax(&ids[i][pix[i]], ((unsigned long long)(key[i] + 1u) << 32) | v[i].y);
+          __hip_atomic_fetch_max(dev_ptr(ids[i]) + pix[i], ((unsigned long long)(key[i] + 1u) << 32) | v[i].y,
+                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
   }
