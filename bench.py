@@ -125,7 +125,7 @@ def shadow_group_size(ntri):
 
 def shade_algorithmic_bytes(W, H, V, O, x_tex, x_shadow, L):
     """Minimal field bytes of one shading launch: 16 B per pixel (depth 4,
-    triangle id 4, RGBA8 4, normal 4; the next render's clear is k_clear's),
+    triangle id 4, RGBA8 4, normal 4; the next render's clear is prearrange's),
     132 B per distinct visible triangle (112 B of vertex fields + 20 B
     fragment record), 52 B per distinct visible object, 4 B per distinct
     atlas / cube-map texel and 56 B per light."""

@@ -382,7 +382,7 @@ int  ocr_batch_get_tuning(ocr_batch* b, ocr_batch_tuning* t);
 int  ocr_batch_set_profiling(ocr_batch* b, int enable);
 /* clear -> prearrange -> depth -> id -> shade for all views on `stream`. */
 int  ocr_batch_render(ocr_batch* b, void* stream);
-/* The same five launches captured once into a hipGraph and replayed. */
+/* The same launches captured once into a hipGraph and replayed. */
 int  ocr_batch_launch_graph(ocr_batch* b, void* stream);
 /* Synchronises `stream`; counters of the last render (OCR_ERR_UNSUPPORTED if
  * the views needed more than 2^31 - 1 raster samples together). */

@@ -187,10 +187,10 @@ constexpr uint32_t kBoxRect = 1u << 31;
 // count; the id pass reads the entries, forms each one's depth again from
 // its record's plane, instead of sweeping the chunk's samples again (chunks
 // with more, or past `chunks`, are swept).
-// 2048-sample chunks: half the wavefronts of 1024-sample ones, which leaves
-// room for the other renders' shading beside the raster passes (1080p/1M
-// frame 0.183 -> 0.178 ms, though the depth pass alone takes 84 us, not 75;
-// 512 and 4096 measured slower).
+// Chunks of up to 2048 samples: half the wavefronts of 1024-sample ones, which
+// leaves room for the other renders' shading beside the raster passes (1080p,
+// 1 M triangles 170 us a frame, 178 with 1024; a batch of 12 views 547 us, 557
+// with 4096).
 constexpr int kChunkLog2 = 11;
 constexpr uint32_t kChunk = 1u << kChunkLog2;   // raster samples per wavefront work item, at most
 constexpr uint32_t kEntCap = kChunk / 2;

@@ -13,12 +13,12 @@
 // to op_size + 1 samples, so one work item per fragment leaves most lanes of
 // a wavefront idle.  Here prearrange computes each cut triangle's exact
 // sample count over all of its fragments and appends the triangle with its
-// range in one global sample space: one packed 64-bit atomicAdd per
-// wavefront returns both the record index and the sample offset, so the cut
-// list is sorted by sample offset and its ranges tile [0, total).  The raster
-// passes split that sample space into equal chunks: a wavefront finds the
-// chunk's first triangle with a 64-ary search, stages 64 triangles' setup in
-// LDS and sweeps the chunk with all lanes.  No per-fragment records exist.
+// range in a sample space: one packed 64-bit atomicAdd per block returns both
+// the record index and the sample offset, so each partition of the cut list
+// is sorted by sample offset and its ranges tile [0, total).  The raster
+// passes split the sample spaces into equal chunks: a wavefront finds the
+// chunk's first triangle with a 64-ary search, stages 64 triangles, one per
+// lane, and draws their rows with all lanes.  No per-fragment records exist.
 #pragma clang fp contract(off)
 
 #include <stdlib.h>
@@ -45,11 +45,8 @@ namespace ocr {
 // 5.00 -> 4.88 ms.
 // Lists of one partition (reserved or tiled) use blocks of 512, which append
 // half as often to the one counter.
-// The shadow prearrange (104 VGPRs) uses 512: two blocks per CU hide each
-// other's loads, barriers and allocation atomic (16-light shadow pass over
-// 4 M triangles 5.09 -> 4.82 ms).
 constexpr int kPreThreadsOne = 512;
-constexpr int kShadowPreThreads = 256;
+constexpr int kShadowPreThreads = 256;   // independent wavefronts: 113 VGPRs and 8.5 KB of LDS each, 16 on a CU
 
 template <int kWaves>
 struct BlockAllocLds {

@@ -759,7 +759,7 @@ static int ensure_shadow_lists(ocr_scene* s, uint32_t cap_cut) {
 // scene with four lights 940 MB of allocation).
 constexpr uint32_t kShadowGroup = 16;
 static uint32_t shadow_list_cap(uint32_t ntri, uint32_t nlights) {
-  constexpr uint32_t kBlock = 512;   // triangles per prearrange block
+  constexpr uint32_t kBlock = 256;   // triangles per shadow prearrange block
   const uint64_t blocks = ((uint64_t)ntri + kBlock - 1) / kBlock;
   const uint64_t per_part = (blocks + kListParts - 1) / kListParts * std::min(ntri, kBlock) *
                                 std::min(std::max(nlights, 1u), kShadowGroup) + 64;

@@ -691,11 +691,10 @@ __global__ void __launch_bounds__(256) k_shade_batch(ShadeLaunch sl) {
 }
 
 // Passes whose scenes have no shadow-casting light: without the occlusion
-// code the kernel fits 96 VGPRs, five wavefronts per SIMD instead of the
-// three of the general kernel's 139, which hides more of its gathers and
+// code the kernel takes 85 VGPRs, five wavefronts per SIMD instead of the
+// four of the general kernel's 113, which hides more of its gathers and
 // leaves room for the next render's raster passes (1080p, 1 M triangles,
-// 4 lights: shading alone 124 -> 108 us).  With shadows, even four
-// wavefronts per SIMD spill inside the light loop and run slower.
+// 4 lights, five wavefronts against three: shading alone 124 -> 108 us).
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_shade_unshadowed(ShadeLaunch sl) {
   shade_pixel<false, false, false>(sl);
   zero_work(sl.p.lists);
