@@ -106,15 +106,13 @@ DevScene dev_scene(const Scene* sc) {
   d.tri_attr = sc->tri_attr;
   d.objs = sc->objs;
   d.pages = sc->atlas.pages;
-  d.nums = sc->atlas.nums;
-  d.sizes = sc->atlas.sizes;
+  d.tex = sc->atlas.tex;
   d.lights = sc->lights;
   d.light_lin = sc->light_lin;
   d.shadow_maps = sc->shadow_maps;
   d.static_maps = sc->static_maps;
   d.ntri = sc->ntri;
   d.nobj = sc->nobj;
-  d.mip_start = sc->atlas.mip_start;
   d.nlights = sc->nlights;
   d.L = sc->lbuf_dim;
   return d;
@@ -489,7 +487,8 @@ int ocr_scene_update_objs_async(ocr_scene* s, uint32_t first, uint32_t n, const 
 
 static void free_atlas(Atlas& a) {
   dev_free(a.pages);
-  dev_free(a.nums);
+  dev_free(a.tex);
+  a.nums = nullptr;   // in tex's allocation
   dev_free(a.sizes);
   a.npages = a.nnums = a.nsizes = a.mip_start = 0;
 }
@@ -588,6 +587,17 @@ int ocr_atlas_upload(ocr_scene* s, const ocr_tex_src* texs, uint32_t ntex) {
   std::vector<uint32_t> sizes(std::max<size_t>(pages.size(), 2), 16);
   for (size_t p = 0; p < pages.size(); p++) sizes[p] = pages[p].size;
 
+  // what shading reads of each texture's levels, and nums behind it (objects
+  // of a scene without textures have id 0)
+  const uint32_t ntab = std::max<uint32_t>(ntex, 1);
+  std::vector<TexDesc> desc(kTexLevels * (size_t)ntab + (nums.size() + 1) / 2);
+  for (uint32_t t = 0; t < ntab; t++)
+    for (int j = 0; j <= OCR_MIP_LEVELS; j++) {
+      const uint32_t num = nums[j == 0 ? t : ntex + t * OCR_MIP_LEVELS + (uint32_t)(j - 1)];
+      desc[kTexLevels * (size_t)t + (size_t)j] = TexDesc{num, (float)sizes[num >> 16]};
+    }
+  memcpy(&desc[kTexLevels * (size_t)ntab], nums.data(), sizeof(uint32_t) * nums.size());
+
   free_atlas(s->atlas);
   Atlas& a = s->atlas;
   a.npages = (uint32_t)std::max<size_t>(pages.size(), 1);
@@ -596,13 +606,14 @@ int ocr_atlas_upload(ocr_scene* s, const ocr_tex_src* texs, uint32_t ntex) {
   a.mip_start = ntex;
   int rc;
   size_t page_bytes = (size_t)OCR_ATLAS_DIM * OCR_ATLAS_DIM * 4;
-  if ((rc = dev_alloc(&a.pages, page_bytes * a.npages, "atlas")) || (rc = dev_alloc(&a.nums, a.nnums, "nums")) ||
+  if ((rc = dev_alloc(&a.pages, page_bytes * a.npages, "atlas")) || (rc = dev_alloc(&a.tex, desc.size(), "texture descriptors")) ||
       (rc = dev_alloc(&a.sizes, a.nsizes, "sizes"))) {
     free_atlas(a);
     return rc;
   }
   OCR_HIP_CHECK(hipMemset(a.pages, 0, page_bytes * a.npages));
-  OCR_HIP_CHECK(hipMemcpy(a.nums, nums.data(), sizeof(uint32_t) * a.nnums, hipMemcpyHostToDevice));
+  a.nums = reinterpret_cast<uint32_t*>(a.tex + kTexLevels * ntab);
+  OCR_HIP_CHECK(hipMemcpy(a.tex, desc.data(), sizeof(TexDesc) * desc.size(), hipMemcpyHostToDevice));
   OCR_HIP_CHECK(hipMemcpy(a.sizes, sizes.data(), sizeof(uint32_t) * a.nsizes, hipMemcpyHostToDevice));
   // texture::update_me_to_gpu + update_gpu_mipmaps (texture.cpp:323-493), in
   // groups of at most kAtlasGroup textures and kAtlasStage bytes (a texture

@@ -28,7 +28,7 @@ __device__ __forceinline__ gptr<T> to_global(T* p) {
 template <typename T>
 __device__ __forceinline__ T ldg(gptr<const T> base, uint32_t idx) {
   gptr<const char> p = (gptr<const char>)base + idx * (uint32_t)sizeof(T);
-  if constexpr (sizeof(T) <= 8) {
+  if constexpr (!__is_class(T)) {
     return *(gptr<const T>)p;
   } else if constexpr (sizeof(T) % 16 == 0 && alignof(T) >= 16) {
     // records: whole 16-byte words, assembled in registers
@@ -61,9 +61,7 @@ struct ShadeArgs {
   gptr<const TriAttr> tri_attr;
   gptr<const ObjDesc> objs;
   gptr<const uint32_t> pages;     // RGBA8 texels as u32
-  gptr<const uint32_t> nums;
-  gptr<const uint32_t> sizes;
-  uint32_t mip_start;
+  gptr<const TexDesc> tex;
   gptr<const ocr_light> lights;
   gptr<const float> light_lin;
   uint32_t nlights;
@@ -145,26 +143,29 @@ __device__ __forceinline__ float tmod(float v) {
 template <bool kCount>
 __device__ __forceinline__ f4 texture_filter_diff(const ShadeArgs& a, float vtx, float vty, float dx,
                                                   float dy, int tid2) {
-  int nv = (int)ldg(a.nums, (uint32_t)tid2);
-  int tsize = (int)ldg(a.sizes, (uint32_t)(nv >> 16));
+  const uint32_t levels = (uint32_t)tid2 * kTexLevels;
+  const float tsize = ldg(a.tex, levels).size;
   float vmx = tmod(vtx), vmy = tmod(vty);
-  float tx = dx * (float)tsize, ty = dy * (float)tsize;
+  float tx = dx * tsize, ty = dy * tsize;
   float worst = sqrt_cr(tx * tx + ty * ty);
   float wf = fmaxf(log2_approx(worst), 0.f);
   float mip_lower = clampf(floorf(wf), 0.f, (float)kMipLevels);
   float fmd = wf - mip_lower;
-  int tid_lower = mip_lower == 0 ? tid2 : (int)(mip_lower - 1 + (float)a.mip_start + (float)(tid2 * kMipLevels));
-  int tid_higher = (int)(clampf(mip_lower, 0.f, kMipLevels - 1.f) + (float)a.mip_start + (float)(tid2 * kMipLevels));
-  int lnv = (int)ldg(a.nums, (uint32_t)tid_lower);
-  float sl = (float)ldg(a.sizes, (uint32_t)(lnv >> 16));
+  // level 0 is the texture itself, level k its mip k - 1; the higher of the two
+  // is at most the last
+  const uint32_t lower = (uint32_t)mip_lower, higher = min(lower + 1u, (uint32_t)kMipLevels);
+  const TexDesc dl = ldg(a.tex, levels + lower);
+  const int lnv = (int)dl.num;
+  const float sl = dl.size;
   f4 c1 = bilinear_pre<kCount>(a, vmx * sl, vmy * sl, lnv & 0xFFFF, lnv >> 16, sl);
   const float i255 = 1.f / 255.f;
   // From mip level 4 on both fetches read the last level: c2 = c1, the
   // blend c1 + 0 * fmd is c1 (fmd is finite), and a wavefront whose lanes
   // are all there skips the second fetch
-  if (__all(tid_lower == tid_higher)) return f4{c1.x * i255, c1.y * i255, c1.z * i255, c1.w * i255};
-  int hnv = (int)ldg(a.nums, (uint32_t)tid_higher);
-  float sh = (float)ldg(a.sizes, (uint32_t)(hnv >> 16));
+  if (__all(lower == higher)) return f4{c1.x * i255, c1.y * i255, c1.z * i255, c1.w * i255};
+  const TexDesc dh = ldg(a.tex, levels + higher);
+  const int hnv = (int)dh.num;
+  const float sh = dh.size;
   f4 c2 = bilinear_pre<kCount>(a, vmx * sh, vmy * sh, hnv & 0xFFFF, hnv >> 16, sh);
   return f4{(c1.x + (c2.x - c1.x) * fmd) * i255, (c1.y + (c2.y - c1.y) * fmd) * i255,
             (c1.z + (c2.z - c1.z) * fmd) * i255, (c1.w + (c2.w - c1.w) * fmd) * i255};
@@ -415,9 +416,7 @@ __device__ __forceinline__ void shade_pixel(const ShadeLaunch& sl) {
   a.tri_attr = to_global<const TriAttr>(S.tri_attr);
   a.objs = to_global<const ObjDesc>(S.objs);
   a.pages = to_global<const uint32_t>(reinterpret_cast<const uint32_t*>(S.pages));
-  a.nums = to_global<const uint32_t>(S.nums);
-  a.sizes = to_global<const uint32_t>(S.sizes);
-  a.mip_start = S.mip_start;
+  a.tex = to_global<const TexDesc>(S.tex);
   a.lights = to_global<const ocr_light>(S.lights);
   a.light_lin = to_global<const float>(S.light_lin);
   a.nlights = S.nlights;
