@@ -26,14 +26,19 @@ struct alignas(8) TriPos {
 };
 static_assert(sizeof(TriPos) == 40, "TriPos layout");
 
-// Shading attributes of a triangle (normals, vt, vertex colours), read only
-// for visible triangles by the shading pass (cl2.cl:5872-5938).
-struct TriAttr {
+// What the shading pass reads of a triangle, visible ones only
+// (cl2.cl:5872-5938): object-space vertices (again: the raster side streams
+// TriPos alone), normals, vt, vertex colours.  Whole 16-byte words of one
+// place: seven loads per pixel where the vertices and a 72-byte record took
+// fourteen of 8 bytes (1080p, 1 M triangles 160.9 -> 156.7 us a frame).
+struct alignas(16) TriAttr {
+  float p[9];
   float n[9];
   float vt[6];
   uint32_t col[3];
+  uint32_t _pad;
 };
-static_assert(sizeof(TriAttr) == 72, "TriAttr layout");
+static_assert(sizeof(TriAttr) == 112, "TriAttr layout");
 
 // The obj_g_descriptor fields the path reads (52 bytes), and what kernel3
 // derives from them identically for every pixel of the object, formed once
@@ -142,7 +147,6 @@ constexpr uint32_t kTexLevels = 8;   // five used
 static_assert(kMipLevels + 1 <= (int)kTexLevels, "levels");
 
 struct DevScene {
-  const TriPos* tri_pos;
   const TriPos* world;      // world-space vertices (object transform applied)
   const TriAttr* tri_attr;
   const ObjDesc* objs;

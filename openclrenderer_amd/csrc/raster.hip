@@ -212,8 +212,8 @@ __device__ __forceinline__ void store_cut(CutTri* dst, const f3 p[3], float rcon
 }
 
 // The 144-byte triangle into the 40-byte position record read by every raster
-// pass and the 72-byte attribute record read only by shading.  Bound by the
-// 256 bytes a triangle it moves.
+// pass and the 112-byte record read only by shading.  Bound by the 296 bytes a
+// triangle it moves.
 __global__ void __launch_bounds__(256) k_split(const uint4* __restrict__ tris, uint32_t n, TriPos* __restrict__ pos,
                                                TriAttr* __restrict__ attr) {
   const uint32_t id = blockIdx.x * 256u + threadIdx.x;
@@ -224,9 +224,9 @@ __global__ void __launch_bounds__(256) k_split(const uint4* __restrict__ tris, u
   for (int v = 0; v < 3; v++) {
     // pos (4 words), normal (4), vt (2), object id, colour
     const uint4 p = tris[9 * (size_t)id + 3 * v], nm = tris[9 * (size_t)id + 3 * v + 1], r = tris[9 * (size_t)id + 3 * v + 2];
-    P.p[3 * v] = __uint_as_float(p.x);
-    P.p[3 * v + 1] = __uint_as_float(p.y);
-    P.p[3 * v + 2] = __uint_as_float(p.z);
+    A.p[3 * v] = P.p[3 * v] = __uint_as_float(p.x);
+    A.p[3 * v + 1] = P.p[3 * v + 1] = __uint_as_float(p.y);
+    A.p[3 * v + 2] = P.p[3 * v + 2] = __uint_as_float(p.z);
     A.n[3 * v] = __uint_as_float(nm.x);
     A.n[3 * v + 1] = __uint_as_float(nm.y);
     A.n[3 * v + 2] = __uint_as_float(nm.z);
@@ -235,6 +235,7 @@ __global__ void __launch_bounds__(256) k_split(const uint4* __restrict__ tris, u
     A.col[v] = r.w;
     if (v == 0) P.oid = r.z;
   }
+  A._pad = 0u;
   pos[id] = P;
   attr[id] = A;
 }

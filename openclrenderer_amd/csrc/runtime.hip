@@ -101,7 +101,6 @@ int device_cu_count() { return g_cu_count > 0 ? g_cu_count : 256; }
 DevScene dev_scene(const Scene* sc) {
   DevScene d;
   memset(&d, 0, sizeof(d));
-  d.tri_pos = sc->tri_pos;
   d.world = sc->world;
   d.tri_attr = sc->tri_attr;
   d.objs = sc->objs;

@@ -23,11 +23,8 @@ __device__ __forceinline__ gptr<T> to_global(T* p) {
   return (gptr<T>)(uintptr_t)p;
 }
 
-// Element `idx` with a 32-bit byte offset (every buffer the shading pass
-// reads is far below 4 GiB), which the scalar-base addressing form takes.
 template <typename T>
-__device__ __forceinline__ T ldg(gptr<const T> base, uint32_t idx) {
-  gptr<const char> p = (gptr<const char>)base + idx * (uint32_t)sizeof(T);
+__device__ __forceinline__ T load_at(gptr<const char> p) {
   if constexpr (!__is_class(T)) {
     return *(gptr<const T>)p;
   } else if constexpr (sizeof(T) % 16 == 0 && alignof(T) >= 16) {
@@ -50,6 +47,17 @@ __device__ __forceinline__ T ldg(gptr<const T> base, uint32_t idx) {
     return out;
   }
 }
+// Element `idx` with a 32-bit byte offset (the buffers it is used on are below
+// 4 GiB), which the scalar-base addressing form takes.
+template <typename T>
+__device__ __forceinline__ T ldg(gptr<const T> base, uint32_t idx) {
+  return load_at<T>((gptr<const char>)base + idx * (uint32_t)sizeof(T));
+}
+// The same for a buffer of any size (triangles).
+template <typename T>
+__device__ __forceinline__ T ldg_far(gptr<const T> base, uint32_t idx) {
+  return load_at<T>((gptr<const char>)base + (uint64_t)idx * sizeof(T));
+}
 
 // What one shading block reads: its view, its scene and the frame's lists.
 struct ShadeArgs {
@@ -57,7 +65,6 @@ struct ShadeArgs {
   gptr<const uint32_t> depth;
   gptr<const unsigned long long> idkey;
   gptr<const CutTri> cuts;
-  gptr<const TriPos> tri_pos;
   gptr<const TriAttr> tri_attr;
   gptr<const ObjDesc> objs;
   gptr<const uint32_t> pages;     // RGBA8 texels as u32
@@ -412,7 +419,6 @@ __device__ __forceinline__ void shade_pixel(const ShadeLaunch& sl) {
   a.depth = to_global<const uint32_t>(V.depth);
   a.idkey = to_global<const unsigned long long>(V.idkey);
   a.cuts = to_global<const CutTri>(sl.p.lists.cuts);
-  a.tri_pos = to_global<const TriPos>(S.tri_pos);
   a.tri_attr = to_global<const TriAttr>(S.tri_attr);
   a.objs = to_global<const ObjDesc>(S.objs);
   a.pages = to_global<const uint32_t>(reinterpret_cast<const uint32_t*>(S.pages));
@@ -453,13 +459,12 @@ __device__ __forceinline__ void shade_pixel(const ShadeLaunch& sl) {
   const CutTri ct = ldg(a.cuts, (uint32_t)key);
   const uint32_t tri = (uint32_t)(key >> 32) - 1u;
   const uint32_t tri_global = tri >> 1;
-  const TriPos T = ldg(a.tri_pos, tri_global);
-  const TriAttr TA = ldg(a.tri_attr, tri_global);
+  const TriAttr TA = ldg_far(a.tri_attr, tri_global);
   const ObjDesc G = ldg(a.objs, ct.oid);
   const f3 camera_pos = mk3(a.v.cpos[0], a.v.cpos[1], a.v.cpos[2]);
-  const f3 p1 = mk3(T.p[0], T.p[1], T.p[2]) * G.scale;
-  const f3 p2 = mk3(T.p[3], T.p[4], T.p[5]) * G.scale;
-  const f3 p3 = mk3(T.p[6], T.p[7], T.p[8]) * G.scale;
+  const f3 p1 = mk3(TA.p[0], TA.p[1], TA.p[2]) * G.scale;
+  const f3 p2 = mk3(TA.p[3], TA.p[4], TA.p[5]) * G.scale;
+  const f3 p3 = mk3(TA.p[6], TA.p[7], TA.p[8]) * G.scale;
   const f3 wpos = mk3(G.wp[0], G.wp[1], G.wp[2]);
   // the object's quaternion as rot_quat normalises it, and its inverse as
   // back_rot_quat forms and rot_quat then normalises it (formed once per
