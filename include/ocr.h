@@ -284,7 +284,7 @@ int  ocr_render(ocr_scene* s, const ocr_view* view, ocr_frame* f, void* stream);
  * the caller's device buffers of view->width * view->height elements: depth
  * (u32), id_key (u64: ((2*tri + piece + 1) << 32) | record, 0 where nothing
  * is drawn; ocr_frame_read's triangle id is (key >> 32) - 1 >> 1), rgba8
- * (u32) and normals (u32, two u16).  The work lists live in a 64 MiB device
+ * (u32) and normals (u32, two u16).  The work lists live in a 48 MiB device
  * scratch array the library holds per GPU (524,286 cut-triangle records, two
  * per scene triangle), so the scene may have at most 262,111 triangles
  * (OCR_ERR_UNSUPPORTED beyond); the scene's lights must already be uploaded.  Calls on one GPU share the

@@ -182,7 +182,7 @@ static int ensure_lists(ocr_batch* b) {
   if (b->cuts) (void)hipFree(b->cuts);
   b->cuts = nullptr;
   b->cap_cut = 0;
-  hipError_t e = hipMalloc((void**)&b->cuts, sizeof(CutTri) * want_cut * 2);
+  hipError_t e = hipMalloc((void**)&b->cuts, sizeof(CutTri) * list_units(want_cut));
   if (e != hipSuccess) {
     (void)hipGetLastError();
     return fail(OCR_ERR_OOM, std::string("batch cut list: ") + hipGetErrorString(e));

@@ -64,24 +64,21 @@ struct alignas(16) ObjDesc {
 };
 static_assert(sizeof(ObjDesc) == 96, "ObjDesc layout");
 
-// A clipped, culled, projected triangle: screen x, y and camera z of its
-// three vertices, its 1/det constant, its sort key (2*tri + sub for a camera
-// view, cube face for a shadow map), object id, view, and for camera views
-// the screen-space plane of 1/z (get_vtdiff's interpolate_get_const,
-// cl2.cl:5691-5760), which shading needs once per visible triangle.  Records
-// are in sample order: prearrange allocates records and sample ranges
-// together, once per block.
+// What the passes after the raster side read of a clipped, culled, projected
+// triangle: the screen-space plane of 1/z (get_vtdiff's interpolate_get_const,
+// cl2.cl:5691-5760), object id, whether it faces the camera, and its view: one
+// 16-byte load per pixel in shading (with the projected vertices, from which
+// the facing was formed again, four: 1080p, 1 M triangles 158 -> 151 us a frame,
+// 12-view batch 447 -> 418).  Records are in sample order:
+// prearrange allocates records and sample ranges together, once per block.
+constexpr uint32_t kCutFront = 1u << 31;   // objects: far below 2^31 (96 B each)
 struct alignas(16) CutTri {
-  float x[3];
-  float y[3];
-  float z[3];
-  float rconst;
-  uint32_t key;
-  uint32_t oid;
+  float da, db, dc;
+  uint32_t oid;       // | kCutFront
   uint32_t view;
-  float da, db, dc;   // 1/z plane (0 for shadow faces)
+  uint32_t _pad[3];
 };
-static_assert(sizeof(CutTri) == 64, "CutTri layout");
+static_assert(sizeof(CutTri) == 32, "CutTri layout");
 
 // The raster setup of a cut triangle, computed once by prearrange and read
 // by every raster pass: bounding-box origin and width, 1/width, the 1/z plane
@@ -220,8 +217,8 @@ struct CoverEntries {
 };
 
 // The cut list and counters shared by the views of one render.  One
-// allocation of 2 * cap_cut records holds the CutTri records followed by
-// their RasterTri setups.  The list is `parts` partitions (a power of two up
+// allocation (list_units) holds the CutTri records followed by their RasterTri
+// setups.  The list is `parts` partitions (a power of two up
 // to kListParts) of cap_cut / parts records, each with a sample space and a
 // counter of its own; prearrange block b appends to partition b mod parts.
 // tb.bin is null unless the render is tiled (one partition).
@@ -284,8 +281,14 @@ constexpr int kPartLineWords = 32;
 constexpr int kListCounterWords = kCounterWords + (int)kListParts * kPartLineWords;
 // partition p: packed counter (u64) at word kPartWord(p), valid prefix at +2
 __host__ __device__ constexpr int kPartWord(uint32_t p) { return kCounterWords + (int)p * kPartLineWords; }
+// A list's allocation in CutTri records: the CutTri records (an even number, so
+// that the setups begin a line) and the setups.
+inline size_t list_cuts(uint64_t cap_cut) { return (size_t)(cap_cut + (cap_cut & 1u)); }
+inline size_t list_units(uint64_t cap_cut) {
+  return list_cuts(cap_cut) + (size_t)cap_cut * (sizeof(RasterTri) / sizeof(CutTri));
+}
 inline Lists make_lists(CutTri* cuts, uint32_t* counters, uint32_t cap_cut, uint32_t parts, bool tiled) {
-  return Lists{cuts, reinterpret_cast<RasterTri*>(cuts + cap_cut), tiled ? counters : counters + kListCounterWords,
+  return Lists{cuts, reinterpret_cast<RasterTri*>(cuts + list_cuts(cap_cut)), tiled ? counters : counters + kListCounterWords,
                counters, cap_cut, parts};
 }
 // Triangles per prearrange block, the unit of the partitions.

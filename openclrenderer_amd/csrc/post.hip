@@ -265,7 +265,7 @@ __global__ void __launch_bounds__(256) k_motion_blur(const MotionArgs a) {
     const unsigned long long key = a.idkey[pix];
     covered = ft != 0xFFFFFFFFu && key != 0ull;
     if (covered) {
-      oid = a.cuts[(uint32_t)key].oid;
+      oid = a.cuts[(uint32_t)key].oid & ~kCutFront;
       covered = oid < a.nobj;
     }
   }

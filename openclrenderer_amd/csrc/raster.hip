@@ -194,15 +194,11 @@ __device__ __forceinline__ uint32_t frag_count(const f3 p[3], float ew, float eh
   return n > 0.f ? (uint32_t)n : 0u;
 }
 
-__device__ __forceinline__ void store_cut(CutTri* dst, const f3 p[3], float rconst, uint32_t key, uint32_t oid,
-                                          uint32_t view) {
+__device__ __forceinline__ void store_cut(CutTri* dst, const f3 p[3], float rconst, uint32_t oid, uint32_t view) {
   CutTri c;
-#pragma unroll
-  for (int i = 0; i < 3; i++) { c.x[i] = p[i].x; c.y[i] = p[i].y; c.z[i] = p[i].z; }
-  c.rconst = rconst;
-  c.key = key;
-  c.oid = oid;
+  c.oid = oid | (front_facing(p[0], p[1], p[2]) ? kCutFront : 0u);
   c.view = view;
+  c._pad[0] = c._pad[1] = c._pad[2] = 0u;
   // the plane kernel3's get_vtdiff builds per pixel (cl2.cl:5691-5760)
   const f3 xpv = mk3(roundf(p[0].x), roundf(p[1].x), roundf(p[2].x));
   const f3 ypv = mk3(roundf(p[0].y), roundf(p[1].y), roundf(p[2].y));
@@ -380,7 +376,7 @@ __device__ __forceinline__ void append_cut(const Lists& L, BlockAllocLds<kWaves>
   if (!block_alloc(L, sh, have ? 1u : 0u, P.ns, P.seen, P.seen ? P.nf : 0u, more, c, smp)) return;
   uint4 box{};
   if (have) {
-    store_cut(&L.cuts[c], P.p, P.rc, key, oid, view);
+    store_cut(&L.cuts[c], P.p, P.rc, oid, view);
     P.rt.key = key | (P.rt.key & kKeyBoxForm);
     P.rt.sample_begin = smp;
     L.rast[c] = P.rt;

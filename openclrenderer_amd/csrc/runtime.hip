@@ -28,7 +28,7 @@ static thread_local std::string g_last_error;
 // it only through the address hipGetSymbolAddress returns for the device
 // (Ctx::noalloc_scratch); calls on one GPU share it and must not overlap.
 constexpr size_t kNoAllocCounterBytes = 4 * 2 * (size_t)kListCounterWords;
-constexpr uint32_t kNoAllocCapCut = 524286;   // records, 64 MiB
+constexpr uint32_t kNoAllocCapCut = 524286;   // records, 48 MiB
 constexpr size_t kNoAllocScratchBytes = kNoAllocCounterBytes + kNoAllocCapCut * (sizeof(CutTri) + sizeof(RasterTri));
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
@@ -1027,7 +1027,7 @@ static int ensure_frame_list(ocr_frame* f, int b, uint32_t ntri) {
   OCR_HIP_CHECK(hipDeviceSynchronize());
   dev_free(lb.cuts);
   lb.cap_cut = 0;
-  int rc = dev_alloc(&lb.cuts, (size_t)want * 2, "cut list");
+  int rc = dev_alloc(&lb.cuts, list_units(want), "cut list");
   if (rc) return rc;
   lb.cap_cut = (uint32_t)want;
   return OCR_OK;
@@ -1187,7 +1187,7 @@ int ocr_render_noalloc(ocr_scene* s, const ocr_view* view, uint32_t* depth, unsi
   if (!s->lights) return fail(OCR_ERR_INVALID, "ocr_render_noalloc: upload the scene's lights first (ocr_lights_upload)");
   // at most two cut pieces per triangle: the list cannot overflow
   if ((uint64_t)s->ntri * 2 + 64 > kNoAllocCapCut)
-    return fail(OCR_ERR_UNSUPPORTED, "ocr_render_noalloc: scene larger than the 64 MiB scratch holds (at most " +
+    return fail(OCR_ERR_UNSUPPORTED, "ocr_render_noalloc: scene larger than the 48 MiB scratch holds (at most " +
                                          std::to_string((kNoAllocCapCut - 64) / 2) + " triangles)");
   if (!s->ctx->noalloc_scratch) return fail(OCR_ERR_INVALID, "ocr_render_noalloc: context has no scratch");
   OCR_HIP_CHECK(hipSetDevice(s->ctx->device));

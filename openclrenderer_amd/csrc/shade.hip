@@ -460,7 +460,7 @@ __device__ __forceinline__ void shade_pixel(const ShadeLaunch& sl) {
   const uint32_t tri = (uint32_t)(key >> 32) - 1u;
   const uint32_t tri_global = tri >> 1;
   const TriAttr TA = ldg_far(a.tri_attr, tri_global);
-  const ObjDesc G = ldg(a.objs, ct.oid);
+  const ObjDesc G = ldg(a.objs, ct.oid & ~kCutFront);
   const f3 camera_pos = mk3(a.v.cpos[0], a.v.cpos[1], a.v.cpos[2]);
   const f3 p1 = mk3(TA.p[0], TA.p[1], TA.p[2]) * G.scale;
   const f3 p2 = mk3(TA.p[3], TA.p[4], TA.p[5]) * G.scale;
@@ -548,8 +548,7 @@ __device__ __forceinline__ void shade_pixel(const ShadeLaunch& sl) {
   const int ff = G.flags;
   const bool two_sided = (ff & OCR_FEATURE_TWO_SIDED) > 0;
   const bool recv_dyn = !((ff & OCR_FEATURE_DOES_NOT_RECEIVE_DYNAMIC_SHADOWS) > 0);
-  const bool is_front = front_facing(mk3(ct.x[0], ct.y[0], ct.z[0]), mk3(ct.x[1], ct.y[1], ct.z[1]),
-                                     mk3(ct.x[2], ct.y[2], ct.z[2]));
+  const bool is_front = (ct.oid & kCutFront) != 0u;
   if (!is_front && two_sided) normal = -normal;
   normal = fast_normalize(normal);
   // rseed / 100: each component is 0 or of magnitude >= 2^-25, where the
