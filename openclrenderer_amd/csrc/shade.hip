@@ -558,7 +558,7 @@ __device__ __forceinline__ void shade_pixel(const ShadeLaunch& sl) {
   const float ambient = linear ? gamma_fwd(kAmbient) : kAmbient;
 
   const float ndv = fmaxf(0.f, dot(normal, l2p));
-  const bool spec_finite = ndv >= 0x1p-60f && fabsf(G.spec_mult) < 0x1p60f;
+  const bool spec_finite = ndv >= 0x1p-24f && fabsf(G.spec_mult) < 0x1p30f;
 
   int shnum = 0, static_num = 0;
   f3 diffuse_sum = mk3(0, 0, 0), specular_sum = mk3(0, 0, 0);
@@ -604,11 +604,15 @@ __device__ __forceinline__ void shade_pixel(const ShadeLaunch& sl) {
     if (!stat) ptl_n = ptl * inv_len;
     ptl = ptl_n;
     const float nl = dot(ptl, lighting_normal), n_ptl = dot(normal, ptl);
-    // Whether this light's specular term is a finite number whatever comes
-    // below: the divisors v.h (at least 0.07 where l2p . ptl > -0.99) and n.v
-    // are away from 0 and nothing that multiplies is infinite or NaN.
+    // Whether this light's specular term is below 2^112 and the sum so far below
+    // 2^126, neither of them NaN: the divisors v.h (at least 0.07 where l2p . ptl
+    // > -0.99) and n.v are away from 0, so spec is below 2^23, and the colour,
+    // the illumination and the object's factor are below 2^30 each.  A sum that
+    // is infinite or NaN stays on the full path, whose fmaxf(sum + term, 0) turns
+    // the NaN of an infinite sum in full shadow into 0.
     const bool finite = spec_finite && dot(l2p, ptl) > -0.99f &&
-                        fabsf(light_col.x) + fabsf(light_col.y) + fabsf(light_col.z) < 0x1p60f && illumination < 0x1p60f;
+                        fabsf(light_col.x) + fabsf(light_col.y) + fabsf(light_col.z) < 0x1p30f && illumination < 0x1p30f &&
+                        specular_sum.x + specular_sum.y + specular_sum.z < 0x1p126f;
     // Then a light behind the surface (n.l <= 0) has a geometric term of 0 and
     // adds no specular, and behind the jittered normal too no diffuse.
     const bool no_spec = finite && n_ptl <= 0.f, dark = no_spec && nl <= 0.f;
