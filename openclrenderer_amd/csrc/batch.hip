@@ -63,7 +63,7 @@ struct ocr_batch {
   hipStream_t capture_stream = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
-  uint32_t graph_unshadowed = 0;     // the shading variant the graph was captured with
+  uint32_t graph_unshadowed = 0, graph_far = 0;   // the shading variant the graph was captured with
   bool profiling = false;
   std::vector<hipEvent_t> ev;        // kRing x 2 (begin, end of a batch)
   int n_profiled = 0;
@@ -89,8 +89,10 @@ static PassArgs batch_pass(const ocr_batch* b) {
   a.tiles = b->tiles;
   a.tile_w_log2 = b->tune.shade_tile_w_log2;
   a.unshadowed = 1u;
-  for (const Scene* s : b->scenes)
+  for (const Scene* s : b->scenes) {
     if (s->n_shadow) a.unshadowed = 0u;
+    if (needs_far(*s, b->cap_cut)) a.far = 1u;
+  }
   a.lists = make_lists(b->cuts, b->counters, b->cap_cut, b->tune.raster_tile ? 1u : list_parts(b->tri_slots, b->cap_cut),
                        b->tune.raster_tile != 0);
   a.lists.ent = b->ent;
@@ -581,9 +583,10 @@ int ocr_batch_launch_graph(ocr_batch* b, void* stream) {
   }
   int rc = ensure_lists(b);
   if (rc) return rc;
-  // the graph holds one shading kernel: capture again when a light upload
-  // changed whether any scene casts shadows
-  if (b->exec && batch_pass(b).unshadowed != b->graph_unshadowed) drop_graph(b);
+  // the graph holds one shading kernel: capture again when an upload changed
+  // whether any scene casts shadows or has buffers above 4 GiB
+  const PassArgs now = batch_pass(b);
+  if (b->exec && (now.unshadowed != b->graph_unshadowed || now.far != b->graph_far)) drop_graph(b);
   if (!b->exec) {
     // Capture on the batch's own stream (the legacy stream cannot be
     // captured); the passes use fill kernels, never memset nodes.
@@ -596,7 +599,8 @@ int ocr_batch_launch_graph(ocr_batch* b, void* stream) {
       return fail(OCR_ERR_HIP, std::string("batch graph capture: ") + hipGetErrorString(e != hipSuccess ? e : e2));
     }
     b->graph = g;
-    b->graph_unshadowed = batch_pass(b).unshadowed;
+    b->graph_unshadowed = now.unshadowed;
+    b->graph_far = now.far;
     OCR_HIP_CHECK(hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
   }
   hipStream_t st = (hipStream_t)stream;

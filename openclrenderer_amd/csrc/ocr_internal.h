@@ -251,6 +251,7 @@ struct PassArgs {
   uint32_t tri_slots, pix_slots, tiles;
   uint32_t tile_w_log2;    // shading tile = (1 << tile_w_log2) x (256 >> tile_w_log2)
   uint32_t unshadowed;     // no scene of the pass has a shadow-casting light
+  uint32_t far;            // shading addresses a buffer above 4 GiB (needs_far)
   Lists lists;
 };
 
@@ -492,6 +493,17 @@ struct Scene {
     return written_valid ? hipStreamWaitEvent(st, written, 0) : hipSuccess;
   }
 };
+
+// Whether shading of the scene with a list of cap_cut records addresses a
+// buffer of more than 2^32 bytes: the cut records (from 134 million on; the
+// records of the last partition lie at the end whatever the content), objects,
+// atlas pages, the cube maps of one kind.
+inline bool needs_far(const Scene& s, uint64_t cap_cut) {
+  constexpr uint64_t k4G = 1ull << 32;
+  const uint64_t map = 24ull * s.lbuf_dim * s.lbuf_dim;
+  return cap_cut * sizeof(CutTri) > k4G || s.nobj * (uint64_t)sizeof(ObjDesc) > k4G ||
+         s.atlas.npages * (4ull * OCR_ATLAS_DIM * OCR_ATLAS_DIM) > k4G || map * s.n_shadow > k4G || map * s.n_static > k4G;
+}
 
 struct Frame {
   Ctx* ctx = nullptr;

@@ -148,6 +148,7 @@ static PassArgs single_pass(const Scene* s, const ocr_view* view, Frame* f) {
   a.lists = make_lists(ob.cuts, ob.counters, ob.cap_cut,
                        tiled || f->want_cut ? 1u : list_parts(a.tri_slots, ob.cap_cut), tiled);
   a.lists.ent = ob.ent;
+  a.far = needs_far(*s, ob.cap_cut) ? 1u : 0u;
   if (f->raster_mode == OCR_RASTER_TILES && ob.tb.bin) {
     a.lists.tb = ob.tb;
     a.view0.bin_begin = 0;
@@ -1211,6 +1212,7 @@ int ocr_render_noalloc(ocr_scene* s, const ocr_view* view, uint32_t* depth, unsi
   pa.scene0 = dev_scene(s);
   pa.unshadowed = s->n_shadow == 0 ? 1u : 0u;
   pa.lists = make_lists(cuts, counters, kNoAllocCapCut, list_parts(pa.tri_slots, kNoAllocCapCut));
+  pa.far = needs_far(*s, kNoAllocCapCut) ? 1u : 0u;
   OCR_HIP_CHECK(s->wait_geometry(st));
   if (s->ctx->noalloc_dirty) OCR_HIP_CHECK(launch_zero_work(counters, st));
   s->ctx->noalloc_dirty = true;

@@ -8,6 +8,8 @@
 // 16x16 work groups, engine.cpp:2018-2022); the tile shape is a tuning knob.
 #pragma clang fp contract(off)
 
+#include <type_traits>
+
 #include "ocr_internal.h"
 
 namespace ocr {
@@ -47,16 +49,26 @@ __device__ __forceinline__ T load_at(gptr<const char> p) {
     return out;
   }
 }
-// Element `idx` with a 32-bit byte offset (the buffers it is used on are below
-// 4 GiB), which the scalar-base addressing form takes.
+// Index into a buffer that grows with the scene or the list, and its element:
+// in the near kernels, which run while those buffers have at most 4 GiB each
+// (needs_far), with a 32-bit byte offset, which the scalar-base addressing form
+// takes, in the far ones with 64 bits throughout.
+template <bool kFar>
+using index_of = std::conditional_t<kFar, uint64_t, uint32_t>;
+template <bool kFar, typename T>
+__device__ __forceinline__ T ldg_of(gptr<const T> base, index_of<kFar> idx) {
+  return load_at<T>((gptr<const char>)base + idx * (index_of<kFar>)sizeof(T));
+}
+// The same for buffers that are always below 4 GiB (a frame's, lights, texture
+// levels).
 template <typename T>
 __device__ __forceinline__ T ldg(gptr<const T> base, uint32_t idx) {
-  return load_at<T>((gptr<const char>)base + idx * (uint32_t)sizeof(T));
+  return ldg_of<false>(base, idx);
 }
-// The same for a buffer of any size (triangles).
+// Triangles are 112 bytes: 64-bit offsets in every kernel.
 template <typename T>
 __device__ __forceinline__ T ldg_far(gptr<const T> base, uint32_t idx) {
-  return load_at<T>((gptr<const char>)base + (uint64_t)idx * sizeof(T));
+  return ldg_of<true>(base, idx);
 }
 
 // What one shading block reads: its view, its scene and the frame's lists.
@@ -99,7 +111,7 @@ __device__ __forceinline__ void touch(uint32_t* bits, size_t idx) {
 }
 
 // read_tex_array_all_precalculated, cl2.cl:820-851.
-template <bool kCount>
+template <bool kCount, bool kFar>
 __device__ __forceinline__ f4 read_tex_pre(const ShadeArgs& a, float cx, float cy, int which, int slice,
                                            float width) {
   const float imax_tex_size = 1.f / 2048;
@@ -114,21 +126,21 @@ __device__ __forceinline__ f4 read_tex_pre(const ShadeArgs& a, float cx, float c
   cy = clampf(cy, 0.001f, width - 0.001f);
   int ix = (int)fmaf(tnumx, width, cx);
   int iy = (int)fmaf(tnumy, width, cy);
-  const uint32_t t = (uint32_t)slice * (2048u * 2048u) + (uint32_t)iy * 2048u + (uint32_t)ix;
+  const index_of<kFar> t = (index_of<kFar>)(uint32_t)slice * (2048u * 2048u) + (uint32_t)iy * 2048u + (uint32_t)ix;
   touch<kCount>(a.tex_touch, t);
-  uint32_t c = ldg(a.pages, t);
+  uint32_t c = ldg_of<kFar>(a.pages, t);
   return f4{(float)(c & 0xFF), (float)((c >> 8) & 0xFF), (float)((c >> 16) & 0xFF), (float)(c >> 24)};
 }
 
 // return_bilinear_col_all_precalculated, cl2.cl:1426-1455.
-template <bool kCount>
+template <bool kCount, bool kFar>
 __device__ __forceinline__ f4 bilinear_pre(const ShadeArgs& a, float mx, float my, int which, int slice,
                                            float width) {
   float px = floorf(mx), py = floorf(my);
-  f4 c0 = read_tex_pre<kCount>(a, px, py, which, slice, width);
-  f4 c1 = read_tex_pre<kCount>(a, px + 1, py, which, slice, width);
-  f4 c2 = read_tex_pre<kCount>(a, px, py + 1, which, slice, width);
-  f4 c3 = read_tex_pre<kCount>(a, px + 1, py + 1, which, slice, width);
+  f4 c0 = read_tex_pre<kCount, kFar>(a, px, py, which, slice, width);
+  f4 c1 = read_tex_pre<kCount, kFar>(a, px + 1, py, which, slice, width);
+  f4 c2 = read_tex_pre<kCount, kFar>(a, px, py + 1, which, slice, width);
+  f4 c3 = read_tex_pre<kCount, kFar>(a, px + 1, py + 1, which, slice, width);
   float ux = mx - px, uy = my - py;
   float bx = 1.f - ux, by = 1.f - uy;
   f4 r;
@@ -147,7 +159,7 @@ __device__ __forceinline__ float tmod(float v) {
 }
 
 // texture_filter_diff, cl2.cl:1511-1573.
-template <bool kCount>
+template <bool kCount, bool kFar>
 __device__ __forceinline__ f4 texture_filter_diff(const ShadeArgs& a, float vtx, float vty, float dx,
                                                   float dy, int tid2) {
   const uint32_t levels = (uint32_t)tid2 * kTexLevels;
@@ -164,7 +176,7 @@ __device__ __forceinline__ f4 texture_filter_diff(const ShadeArgs& a, float vtx,
   const TexDesc dl = ldg(a.tex, levels + lower);
   const int lnv = (int)dl.num;
   const float sl = dl.size;
-  f4 c1 = bilinear_pre<kCount>(a, vmx * sl, vmy * sl, lnv & 0xFFFF, lnv >> 16, sl);
+  f4 c1 = bilinear_pre<kCount, kFar>(a, vmx * sl, vmy * sl, lnv & 0xFFFF, lnv >> 16, sl);
   const float i255 = 1.f / 255.f;
   // From mip level 4 on both fetches read the last level: c2 = c1, the
   // blend c1 + 0 * fmd is c1 (fmd is finite), and a wavefront whose lanes
@@ -173,7 +185,7 @@ __device__ __forceinline__ f4 texture_filter_diff(const ShadeArgs& a, float vtx,
   const TexDesc dh = ldg(a.tex, levels + higher);
   const int hnv = (int)dh.num;
   const float sh = dh.size;
-  f4 c2 = bilinear_pre<kCount>(a, vmx * sh, vmy * sh, hnv & 0xFFFF, hnv >> 16, sh);
+  f4 c2 = bilinear_pre<kCount, kFar>(a, vmx * sh, vmy * sh, hnv & 0xFFFF, hnv >> 16, sh);
   return f4{(c1.x + (c2.x - c1.x) * fmd) * i255, (c1.y + (c2.y - c1.y) * fmd) * i255,
             (c1.z + (c2.z - c1.z) * fmd) * i255, (c1.w + (c2.w - c1.w) * fmd) * i255};
 }
@@ -325,11 +337,11 @@ __device__ __forceinline__ ShadowSetup shadow_setup(const ShadeArgs& a, f3 lpos,
 // Returns the shadow term (0 = lit).  A 4x4 block of depth compares feeds 9
 // bilinear filters of 0/1 values; when all 16 compares agree the filters are
 // evaluated with those constants (all zero: the sum is exactly 0).
-template <bool kCount>
+template <bool kCount, bool kFar>
 __device__ __forceinline__ float shadow_taps(const ShadeArgs& a, const ShadowSetup& s,
                                              gptr<const uint32_t> buf, uint32_t* touch_bits, int shnum) {
   const uint32_t L = a.L;
-  const uint32_t map_off = ((uint32_t)s.face + (uint32_t)shnum * 6u) * L * L;
+  const index_of<kFar> map_off = (index_of<kFar>)((uint32_t)s.face + (uint32_t)shnum * 6u) * (L * L);
   const MapLayout lay = map_layout(L);
   uint32_t cond = 0;   // 4x4 taps, bit (y+1)*4 + (x+1)
   uint32_t col[4];
@@ -339,9 +351,9 @@ __device__ __forceinline__ float shadow_taps(const ShadeArgs& a, const ShadowSet
   for (int y = 0; y < 4; y++)
 #pragma unroll
     for (int x = 0; x < 4; x++) {
-      const uint32_t t = map_off + map_row(lay, s.iy + (uint32_t)y) + col[x];
+      const index_of<kFar> t = map_off + map_row(lay, s.iy + (uint32_t)y) + col[x];
       touch<kCount>(touch_bits, t);
-      float ldp = depth_of(ldg(buf, t));
+      float ldp = depth_of(ldg_of<kFar>(buf, t));
       cond |= (s.dpth > ldp + s.bias ? 1u : 0u) << (y * 4 + x);
     }
   if (cond == 0u) return 0.f;
@@ -409,7 +421,7 @@ __device__ __forceinline__ const DevView& batch_view(const PassArgs& p, uint32_t
 // moved each back: 1080p, 1 M triangles 92.7 ->
 // 85.8 us alone, a frame 172 -> 162; closeup frame 58 -> 50; 12-view batch
 // shading 297 -> 256, 494 -> 454 in all).
-template <bool kCount, bool kShadows, bool kBatch>
+template <bool kCount, bool kShadows, bool kBatch, bool kFar>
 __device__ __forceinline__ void shade_pixel(const ShadeLaunch& sl) {
   const uint32_t block_tile = shade_tile_index();
   const DevView& V = kBatch ? batch_view(sl.p, block_tile) : sl.p.view0;
@@ -456,11 +468,11 @@ __device__ __forceinline__ void shade_pixel(const ShadeLaunch& sl) {
   // SSAO reads only the depth buffer: formed first, while little else is live
   const float occ_ssao = ssao(a, x, y);
   const float fov = a.v.fov;
-  const CutTri ct = ldg(a.cuts, (uint32_t)key);
+  const CutTri ct = ldg_of<kFar>(a.cuts, (uint32_t)key);
   const uint32_t tri = (uint32_t)(key >> 32) - 1u;
   const uint32_t tri_global = tri >> 1;
   const TriAttr TA = ldg_far(a.tri_attr, tri_global);
-  const ObjDesc G = ldg(a.objs, ct.oid & ~kCutFront);
+  const ObjDesc G = ldg_of<kFar>(a.objs, ct.oid & ~kCutFront);
   const f3 camera_pos = mk3(a.v.cpos[0], a.v.cpos[1], a.v.cpos[2]);
   const f3 p1 = mk3(TA.p[0], TA.p[1], TA.p[2]) * G.scale;
   const f3 p2 = mk3(TA.p[3], TA.p[4], TA.p[5]) * G.scale;
@@ -529,7 +541,7 @@ __device__ __forceinline__ void shade_pixel(const ShadeLaunch& sl) {
 
   f4 col;
   if (TA.col[0] == 0u) {
-    col = texture_filter_diff<kCount>(a, vtx, vty, vdx, vdy, (int)G.tid);
+    col = texture_filter_diff<kCount, kFar>(a, vtx, vty, vdx, vdy, (int)G.tid);
   } else {
     f4 c0 = vcol(TA.col[0]), c1 = vcol(TA.col[1]), c2 = vcol(TA.col[2]);
     col = f4{fmaf(c0.x, l1, fmaf(c1.x, l2, c2.x * l3)), fmaf(c0.y, l1, fmaf(c1.y, l2, c2.y * l3)),
@@ -579,7 +591,7 @@ __device__ __forceinline__ void shade_pixel(const ShadeLaunch& sl) {
     if (stat) {
       ptl_n = ptl * inv_len;
       ss = shadow_setup(a, lpos, normal, ptl_n, global_position);
-      occlusion = 1.f - shadow_taps<kCount>(a, ss, a.static_maps, a.static_touch, static_num);
+      occlusion = 1.f - shadow_taps<kCount, kFar>(a, ss, a.static_maps, a.static_touch, static_num);
       static_num++;
     }
     // 1/radius from the light upload (0 when the radius is out of range)
@@ -623,7 +635,7 @@ __device__ __forceinline__ void shade_pixel(const ShadeLaunch& sl) {
       // keeps what it counts)
       if (kCount || __any(!dark || specular_sum.x != 0.f || specular_sum.y != 0.f || specular_sum.z != 0.f)) {
         if (!stat) ss = shadow_setup(a, lpos, normal, ptl_n, global_position);
-        float dyn = 1.f - shadow_taps<kCount>(a, ss, a.shadow_maps, a.shadow_touch, shnum);
+        float dyn = 1.f - shadow_taps<kCount, kFar>(a, ss, a.shadow_maps, a.shadow_touch, shnum);
         occlusion = fminf(occlusion, dyn);
       }
       shnum++;
@@ -687,27 +699,38 @@ __device__ __forceinline__ void zero_work(const Lists& L) {
     for (uint32_t i = threadIdx.x; i < (uint32_t)kPartWord(L.parts); i += 256u) L.counters[i] = 0u;
 }
 
+// (the variant that counts the texels it touches takes buffers of any size)
 template <bool kCount>
 __global__ void __launch_bounds__(256) k_shade(ShadeLaunch sl) {
-  shade_pixel<kCount, true, false>(sl);
+  shade_pixel<kCount, true, false, kCount>(sl);
   zero_work(sl.p.lists);
 }
 __global__ void __launch_bounds__(256) k_shade_batch(ShadeLaunch sl) {
-  shade_pixel<false, true, true>(sl);
+  shade_pixel<false, true, true, false>(sl);
+  zero_work(sl.p.lists);
+}
+// A pass with a buffer above 4 GiB (needs_far): one kernel each, whether or
+// not there are shadows.  They hold a 64-bit address per gather in flight.
+__global__ void __launch_bounds__(256) k_shade_far(ShadeLaunch sl) {
+  shade_pixel<false, true, false, true>(sl);
+  zero_work(sl.p.lists);
+}
+__global__ void __launch_bounds__(256) k_shade_batch_far(ShadeLaunch sl) {
+  shade_pixel<false, true, true, true>(sl);
   zero_work(sl.p.lists);
 }
 
 // Passes whose scenes have no shadow-casting light: without the occlusion
-// code the kernel takes 85 VGPRs, five wavefronts per SIMD instead of the
+// code the kernel takes 79 VGPRs, five wavefronts per SIMD instead of the
 // four of the general kernel's 113, which hides more of its gathers and
 // leaves room for the next render's raster passes (1080p, 1 M triangles,
 // 4 lights, five wavefronts against three: shading alone 124 -> 108 us).
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_shade_unshadowed(ShadeLaunch sl) {
-  shade_pixel<false, false, false>(sl);
+  shade_pixel<false, false, false, false>(sl);
   zero_work(sl.p.lists);
 }
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_shade_batch_unshadowed(ShadeLaunch sl) {
-  shade_pixel<false, false, true>(sl);
+  shade_pixel<false, false, true, false>(sl);
   zero_work(sl.p.lists);
 }
 
@@ -734,8 +757,9 @@ hipError_t launch_shade(const PassArgs& p, const SinCos face[6], hipStream_t s) 
   sl.p = p;
   for (int i = 0; i < 6; i++) sl.face[i] = face[i];
   sl.tex_touch = sl.shadow_touch = sl.static_touch = nullptr;
-  const auto kernel = p.views ? (p.unshadowed ? k_shade_batch_unshadowed : k_shade_batch)
-                              : (p.unshadowed ? k_shade_unshadowed : k_shade<false>);
+  const auto kernel = p.far ? (p.views ? k_shade_batch_far : k_shade_far)
+                            : p.views ? (p.unshadowed ? k_shade_batch_unshadowed : k_shade_batch)
+                                      : (p.unshadowed ? k_shade_unshadowed : k_shade<false>);
   hipLaunchKernelGGL(kernel, dim3(p.tiles > 0 ? p.tiles : 1), dim3(256), 0, s, sl);
   return hipGetLastError();
 }
