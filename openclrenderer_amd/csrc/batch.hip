@@ -40,7 +40,7 @@ struct ocr_batch {
   uint64_t sum_tris = 0, sum_pix = 0;
   CutTri* cuts = nullptr;
   uint32_t* counters = nullptr;      // published, then working (make_lists)
-  bool counters_dirty = false;       // a render was not enqueued to its end
+  WorkState work;
   uint32_t cap_cut = 0;
   // tiled raster path (tune.raster_tile != 0): bins over every view's tiles
   TileBins tb{};
@@ -559,10 +559,9 @@ int ocr_batch_render(ocr_batch* b, void* stream) {
   OCR_HIP_CHECK(bind_scenes(b, st));
   const bool prof = b->profiling && b->n_profiled < kBatchRing;
   if (prof) OCR_HIP_CHECK(hipEventRecord(b->ev[2 * b->n_profiled], st));
-  if (b->counters_dirty) OCR_HIP_CHECK(launch_zero_work(b->counters, st));
-  b->counters_dirty = true;
+  OCR_HIP_CHECK(begin_work(b->work, b->counters, st));
   OCR_HIP_CHECK(enqueue_batch(b, st));
-  b->counters_dirty = false;
+  end_work(b->work);
   OCR_HIP_CHECK(note_scene_reads(b, st));
   if (prof) OCR_HIP_CHECK(hipEventRecord(b->ev[2 * b->n_profiled++ + 1], st));
   return OCR_OK;
@@ -610,9 +609,9 @@ int ocr_batch_launch_graph(ocr_batch* b, void* stream) {
   OCR_HIP_CHECK(bind_scenes(b, st));   // the graph reads d_scenes when it runs
   const bool prof = b->profiling && b->n_profiled < kBatchRing;
   if (prof) OCR_HIP_CHECK(hipEventRecord(b->ev[2 * b->n_profiled], st));
-  if (b->counters_dirty) OCR_HIP_CHECK(launch_zero_work(b->counters, st));
-  b->counters_dirty = false;
+  OCR_HIP_CHECK(begin_work(b->work, b->counters, st));
   OCR_HIP_CHECK(hipGraphLaunch(b->exec, st));
+  end_work(b->work);
   OCR_HIP_CHECK(note_scene_reads(b, st));
   if (prof) OCR_HIP_CHECK(hipEventRecord(b->ev[2 * b->n_profiled++ + 1], st));
   return OCR_OK;

@@ -334,6 +334,12 @@ constexpr uint32_t kShadowWaveSamples = 1u << 25;
 constexpr uint32_t kShadowMaxSamples = 1u << 30;
 constexpr uint32_t kShadowMaxRecords = 14u << 20;
 
+// What is known of a list's working counters between renders.
+struct WorkState {
+  bool dirty = false;       // a render that uses them was not enqueued to its end
+  bool capturing = false;   // the present render is recorded, not run
+};
+
 // An event that outlives whichever of its holders ends first.
 struct Event {
   hipEvent_t ev = nullptr;
@@ -352,7 +358,6 @@ struct Ctx {
   // device address of the no-allocation render's scratch on this device
   // (hipGetSymbolAddress at ocr_create)
   unsigned char* noalloc_scratch = nullptr;
-  bool noalloc_dirty = false;   // a render into it was not enqueued to its end
   // what ocr_render goes by when it chooses its stream: the last render's end,
   // and whether a post pass or batch was enqueued since
   std::mutex mu;
@@ -518,7 +523,7 @@ struct Frame {
     uint32_t* normals = nullptr;
     CutTri* cuts = nullptr;
     uint32_t* counters = nullptr;   // published, then working (make_lists)
-    bool counters_dirty = false;    // a render of the set was not enqueued to its end
+    WorkState work;
     bool direct = false;            // the set's last render ran on the caller's stream
     uint32_t cap_cut = 0;
     // tiled raster path (tiles.hip): bins of this set's cut list
@@ -579,6 +584,13 @@ void free_bins(TileBins& tb, uint32_t& box_cap);
 hipError_t launch_bin_reset(const TileBins& tb, uint32_t* counters, hipStream_t s);
 // Zeroes the working counters of make_lists' array.
 hipError_t launch_zero_work(uint32_t* counters, hipStream_t s);
+// Around a render's launches on s with `counters`: begin zeroes the working
+// counters where they may not be zero, `end` tells that the shading pass, which
+// zeroes them again, is enqueued.
+hipError_t begin_work(WorkState& w, uint32_t* counters, hipStream_t s);
+inline void end_work(WorkState& w) {
+  if (!w.capturing) w.dirty = false;
+}
 uint32_t bin_scan_chunks(uint32_t ntiles);
 
 // ---- error plumbing -------------------------------------------------------

@@ -31,6 +31,14 @@ constexpr size_t kNoAllocCounterBytes = 4 * 2 * (size_t)kListCounterWords;
 constexpr uint32_t kNoAllocCapCut = 524286;   // records, 48 MiB
 constexpr size_t kNoAllocScratchBytes = kNoAllocCounterBytes + kNoAllocCapCut * (sizeof(CutTri) + sizeof(RasterTri));
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
+// The state of each GPU's scratch, whichever context uses it: calls on one GPU
+// do not overlap, those on different GPUs may.
+static std::mutex g_noalloc_mu;
+static std::map<int, WorkState> g_noalloc_work;   // nodes stay where they are
+static WorkState& noalloc_work(int device) {
+  std::lock_guard<std::mutex> lk(g_noalloc_mu);
+  return g_noalloc_work[device];
+}
 
 void set_error(const std::string& msg) { g_last_error = msg; }
 int fail(int code, const std::string& msg) {
@@ -92,6 +100,26 @@ static ViewParams make_view_params(const ocr_view* v) {
   sincos_of(v->c_rot, p.cam);
   for (int i = 0; i < 4; i++) p.clear[i] = v->clear_col[i];
   return p;
+}
+
+// A recorded render runs later, after whatever is enqueued in between and
+// possibly behind one that was not enqueued to its end: it always zeroes its
+// counters itself and says nothing about their present state.  (The query
+// leaves another thread's capture alone; a stream that cannot tell is taken for
+// one that runs, with counters that are not zero.)
+hipError_t begin_work(WorkState& w, uint32_t* counters, hipStream_t s) {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  hipError_t q = hipThreadExchangeStreamCaptureMode(&mode);
+  if (q == hipSuccess) {
+    q = hipStreamIsCapturing(s, &cap);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
+  if (q != hipSuccess) (void)hipGetLastError();
+  w.capturing = q == hipSuccess && cap != hipStreamCaptureStatusNone;
+  const hipError_t e = w.dirty || w.capturing || q != hipSuccess ? launch_zero_work(counters, s) : hipSuccess;
+  if (!w.capturing) w.dirty = true;
+  return e;
 }
 
 static int g_cu_count = 0;
@@ -1138,8 +1166,7 @@ int ocr_render(ocr_scene* s, const ocr_view* view, ocr_frame* f, void* stream) {
     if (prof) OCR_HIP_CHECK(hipEventRecord(ev[3], sb));
     if (prof) OCR_HIP_CHECK(hipEventRecord(ev[4], sb));
   } else {
-    if (f->out[b].counters_dirty) OCR_HIP_CHECK(launch_zero_work(o.counters, sb));
-    f->out[b].counters_dirty = true;   // until the shading pass that zeroes them again is enqueued
+    OCR_HIP_CHECK(begin_work(f->out[b].work, o.counters, sb));
     if (prof) {
       OCR_HIP_CHECK(hipEventRecord(ev[0], sb));
       OCR_HIP_CHECK(hipEventRecord(ev[1], sb));
@@ -1157,7 +1184,7 @@ int ocr_render(ocr_scene* s, const ocr_view* view, ocr_frame* f, void* stream) {
   OCR_HIP_CHECK(s->wait_shadow_maps(sb));
   if (prof_shade) OCR_HIP_CHECK(hipEventRecord(ev[6], sb));
   OCR_HIP_CHECK(launch_shade(pa, s->ctx->face_sc, sb));
-  if (!tiled) f->out[b].counters_dirty = false;
+  if (!tiled) end_work(f->out[b].work);
   if (prof_shade) OCR_HIP_CHECK(hipEventRecord(ev[5], sb));
   OCR_HIP_CHECK(hipEventRecord(f->done[b]->ev, sb));
   s->note_read(f->done[b], true);
@@ -1214,14 +1241,14 @@ int ocr_render_noalloc(ocr_scene* s, const ocr_view* view, uint32_t* depth, unsi
   pa.lists = make_lists(cuts, counters, kNoAllocCapCut, list_parts(pa.tri_slots, kNoAllocCapCut));
   pa.far = needs_far(*s, kNoAllocCapCut) ? 1u : 0u;
   OCR_HIP_CHECK(s->wait_geometry(st));
-  if (s->ctx->noalloc_dirty) OCR_HIP_CHECK(launch_zero_work(counters, st));
-  s->ctx->noalloc_dirty = true;
+  WorkState& work = noalloc_work(s->ctx->device);
+  OCR_HIP_CHECK(begin_work(work, counters, st));
   OCR_HIP_CHECK(launch_prearrange(pa, st));
   OCR_HIP_CHECK(launch_depth(pa, kRasterBlocksPerCu, st));
   OCR_HIP_CHECK(launch_id(pa, kRasterBlocksPerCu, st));
   OCR_HIP_CHECK(s->wait_shadow_maps(st));
   OCR_HIP_CHECK(launch_shade(pa, s->ctx->face_sc, st));
-  s->ctx->noalloc_dirty = false;
+  end_work(work);
   OCR_HIP_CHECK(s->note_read(st, true));
   return OCR_OK;
 }
