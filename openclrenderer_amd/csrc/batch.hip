@@ -630,6 +630,7 @@ int ocr_batch_get_stats(ocr_batch* b, void* stream, ocr_frame_stats* out) {
       OCR_HIP_CHECK(hipMemcpy(g, b->subs[k]->counters, sizeof(g), hipMemcpyDeviceToHost));
       c[kCutCount] += g[kCutCount];
       c[kFragCount] += g[kFragCount];
+      c[kFragMore] += g[kFragMore];
       c[kOverflow] |= g[kOverflow];
       // a group whose bins overflowed grows them for its next render
       if (g[kOverflow] & kOverflowBins)
@@ -642,7 +643,7 @@ int ocr_batch_get_stats(ocr_batch* b, void* stream, ocr_frame_stats* out) {
   }
   memset(out, 0, sizeof(*out));
   out->n_cut = c[kCutCount];
-  out->n_frag = c[kFragCount];
+  out->n_frag = c[kFragCount] + c[kFragMore];
   out->overflow = c[kOverflow] ? 1u : 0u;
   out->n_profiled = (uint32_t)b->n_profiled;
   if (b->n_profiled) {

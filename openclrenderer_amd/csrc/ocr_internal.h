@@ -268,6 +268,7 @@ enum Counter : int {
   kOverflow = 2,
   kFragCount = 32,         // reference fragments and cut pieces (statistics; one u64), byte 128
   kCutCount = 33,
+  kFragMore = 34,          // fragments of blocks with many (block_alloc), modulo 2^32 like their sum
   kBinTotal = 48,          // tiled path: bin entries the render needed, byte 192
   kCounterWords = 64,
 };

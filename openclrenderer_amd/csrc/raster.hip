@@ -101,9 +101,15 @@ __device__ __forceinline__ bool block_alloc(const Lists& L, BlockAllocLds<kWaves
       if ((end >> 32) > cap) bad |= kOverflowCuts;
       if ((uint32_t)end > kMaxSamples) bad |= kOverflowSamples;
     }
-    // fragments stay far below 2^32 (one per piece and one per 500 samples)
-    if (tn)
-      atomicAdd(reinterpret_cast<unsigned long long*>(L.counters + kFragCount), ((unsigned long long)tn << 32) + tf);
+    // Pieces and fragments in one add.  A block has at most two appends: those
+    // with fragments below 2^31 / gridDim.x cannot together carry into the
+    // pieces; the others (no ordinary frame's) add theirs apart.
+    if (tn) {
+      const bool apart = ((unsigned long long)tf * gridDim.x >> 31) != 0ull;
+      atomicAdd(reinterpret_cast<unsigned long long*>(L.counters + kFragCount),
+                ((unsigned long long)tn << 32) + (apart ? 0u : tf));
+      if (apart) atomicAdd(&L.counters[kFragMore], tf);
+    }
     if (bad) atomicOr(&L.counters[kOverflow], bad);
     sh.base = base + ((unsigned long long)(part * cap) << 32);
     sh.ok = bad == 0;

@@ -1262,7 +1262,7 @@ int ocr_frame_get_stats(ocr_frame* f, void* stream, ocr_frame_stats* out) {
   OCR_HIP_CHECK(hipMemcpy(c, f->out[f->cur].counters, sizeof(c), hipMemcpyDeviceToHost));
   memset(out, 0, sizeof(*out));
   out->n_cut = c[kCutCount];
-  out->n_frag = c[kFragCount];
+  out->n_frag = c[kFragCount] + c[kFragMore];
   out->overflow = c[kOverflow] ? 1u : 0u;
   out->n_profiled = (uint32_t)f->n_profiled;
   if (f->n_profiled > 0) {
