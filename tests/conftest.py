@@ -12,6 +12,16 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (runs through the HIP library)")
 
 
+def pytest_collection_modifyitems(items):
+    # the tests over the reference's own files skip where its tree is absent;
+    # an empty folder in its place is the same
+    tree = "/root/reference"
+    if os.path.isdir(tree) and not os.listdir(tree):
+        for item in items:
+            if item.name.startswith("test_reference_"):
+                item.add_marker(pytest.mark.skip(reason="reference tree not present"))
+
+
 def _ensure_built():
     """Tests load what is built and build only when nothing is."""
     from openclrenderer_amd import build as b
