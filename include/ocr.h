@@ -273,9 +273,7 @@ int  ocr_frame_set_profiling(ocr_frame* f, int enable);
  * waits for the work on `stream` enqueued before render N-1 was issued:
  * enqueue what reads a render's outputs (ocr_frame_device_buffers changes
  * with every render) on `stream` before the next ocr_render on the frame,
- * and use one stream for the renders of one frame.  With the renders before
- * it finished when it is issued, a render runs on `stream` itself, behind
- * whatever is enqueued there.  A frame serves either ocr_render or batches:
+ * and use one stream for the renders of one frame.  A frame serves either ocr_render or batches:
  * a frame already set on a batch is refused (OCR_ERR_INVALID). */
 int  ocr_render(ocr_scene* s, const ocr_view* view, ocr_frame* f, void* stream);
 /* No counterpart in the reference: ocr_render for callers that cannot

@@ -541,7 +541,6 @@ int ocr_batch_set_profiling(ocr_batch* b, int enable) {
 int ocr_batch_render(ocr_batch* b, void* stream) {
   if (!b || b->nviews == 0) return fail(OCR_ERR_INVALID, "ocr_batch_render: no views");
   OCR_HIP_CHECK(hipSetDevice(b->ctx->device));
-  b->ctx->note_other_work();
   hipStream_t st = (hipStream_t)stream;
   if (group_count(b) > 1) {
     const bool prof = b->profiling && b->n_profiled < kBatchRing;
@@ -570,7 +569,6 @@ int ocr_batch_render(ocr_batch* b, void* stream) {
 int ocr_batch_launch_graph(ocr_batch* b, void* stream) {
   if (!b || b->nviews == 0) return fail(OCR_ERR_INVALID, "ocr_batch_launch_graph: no views");
   OCR_HIP_CHECK(hipSetDevice(b->ctx->device));
-  b->ctx->note_other_work();
   if (group_count(b) > 1) {
     hipStream_t gst = (hipStream_t)stream;
     const bool prof = b->profiling && b->n_profiled < kBatchRing;

@@ -359,11 +359,6 @@ struct Ctx {
   // device address of the no-allocation render's scratch on this device
   // (hipGetSymbolAddress at ocr_create)
   unsigned char* noalloc_scratch = nullptr;
-  // what ocr_render goes by when it chooses its stream: the last render's end,
-  // and whether a post pass or batch was enqueued since
-  std::mutex mu;
-  std::shared_ptr<Event> last_render;
-  bool other_work = false;
   // Device staging of scene and texture uploads, at most kStageBytes, held for
   // the context's life, so that loading a scene allocates only what it keeps.
   // One upload at a time.
@@ -371,10 +366,6 @@ struct Ctx {
   std::mutex stage_mu;
   uint8_t* stage = nullptr;
   size_t stage_bytes = 0;
-  void note_other_work() {
-    std::lock_guard<std::mutex> lk(mu);
-    other_work = true;
-  }
 };
 
 struct Atlas {
@@ -525,7 +516,6 @@ struct Frame {
     CutTri* cuts = nullptr;
     uint32_t* counters = nullptr;   // published, then working (make_lists)
     WorkState work;
-    bool direct = false;            // the set's last render ran on the caller's stream
     uint32_t cap_cut = 0;
     // tiled raster path (tiles.hip): bins of this set's cut list
     TileBins tb{};

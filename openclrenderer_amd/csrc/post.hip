@@ -367,7 +367,6 @@ extern "C" int ocr_frame_blend_with_depth(ocr_frame* src, ocr_frame* dst, void* 
   if (src->width != dst->width || src->height != dst->height)
     return fail(OCR_ERR_INVALID, "ocr_frame_blend_with_depth: frame sizes differ");
   OCR_HIP_CHECK(hipSetDevice(dst->ctx->device));
-  dst->ctx->note_other_work();
   OCR_HIP_CHECK(launch_blend_depth(src->depth, dst->depth, src->rgba, dst->rgba, dst->width * dst->height,
                                    (hipStream_t)stream));
   return OCR_OK;
@@ -379,7 +378,6 @@ extern "C" int ocr_frame_blend_with_depth(ocr_frame* src, ocr_frame* dst, void* 
 extern "C" int ocr_frame_pseudo_aa(ocr_frame* f, void* stream) {
   if (!f) return fail(OCR_ERR_INVALID, "ocr_frame_pseudo_aa: null frame");
   OCR_HIP_CHECK(hipSetDevice(f->ctx->device));
-  f->ctx->note_other_work();
   const size_t npix = (size_t)f->width * f->height;
   if (!f->post_in) {
     hipError_t e = hipMalloc((void**)&f->post_in, 4 * npix);
@@ -410,7 +408,6 @@ extern "C" int ocr_frame_motion_blur(ocr_frame* f, ocr_scene* s, const ocr_view*
   if (!(fov >= 0x1p-60f && fov <= 0x1p60f))
     return fail(OCR_ERR_INVALID, "ocr_frame_motion_blur: fov_const must be in [2^-60, 2^60]");
   OCR_HIP_CHECK(hipSetDevice(f->ctx->device));
-  f->ctx->note_other_work();
   const size_t npix = (size_t)f->width * f->height;
   if (!f->post_in) {
     hipError_t e = hipMalloc((void**)&f->post_in, 4 * npix);

@@ -1062,41 +1062,6 @@ static int ensure_frame_list(ocr_frame* f, int b, uint32_t ntri) {
   return OCR_OK;
 }
 
-static bool finished(hipEvent_t e) {
-  const hipError_t q = hipEventQuery(e);
-  if (q != hipSuccess && q != hipErrorNotReady) (void)hipGetLastError();
-  return q == hipSuccess;
-}
-
-// Whether a render of set b goes straight to the caller's stream: with the
-// context's last render and the frame's own finished there is nothing to
-// overlap, and a stream of its own only adds the waits between the two
-// (alone: thumbnail 50 -> 40 us, 1080p closeup 93 -> 74, 1080p, 1 M triangles
-// 265 -> 250).  Not after a post pass or a batch, which may still be running
-// on the caller's stream, and not while a shadow pass or an update of the
-// scene is under way: raster passes on a stream of their own overlap these.
-// Not on a stream under capture.  (The queries leave another thread's capture
-// alone.)
-static bool render_direct(const Scene* s, const Frame* f, int b, hipStream_t st) {
-  std::shared_ptr<Event> last;
-  {
-    std::lock_guard<std::mutex> lk(f->ctx->mu);
-    last = f->ctx->last_render;
-    const bool other = f->ctx->other_work;
-    f->ctx->other_work = false;
-    if (other) return false;
-  }
-  if (!f->rendered) return false;
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return false;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  const bool ok = hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
-                  finished(f->done[f->cur]->ev) && finished(f->done[b]->ev) && (!last || finished(last->ev)) &&
-                  (!s->geom_valid || finished(s->geom_written)) && (!s->written_valid || finished(s->written));
-  (void)hipThreadExchangeStreamCaptureMode(&mode);
-  return ok;
-}
-
 int ocr_render(ocr_scene* s, const ocr_view* view, ocr_frame* f, void* stream) {
   if (!s || !view || !f) return fail(OCR_ERR_INVALID, "ocr_render: null argument");
   if (view->width != f->width || view->height != f->height)
@@ -1135,14 +1100,9 @@ int ocr_render(ocr_scene* s, const ocr_view* view, ocr_frame* f, void* stream) {
   // kSets-1 renders before it; the caller's stream then waits for it.  The
   // first renders follow the caller's stream.
   const int oldest = (b + 1) % Frame::kSets;
-  const bool direct = render_direct(s, f, b, st);
-  hipStream_t sb = direct ? st : f->ss[b];
+  hipStream_t sb = f->ss[b];
   OCR_HIP_CHECK(hipEventRecord(f->entry[b], st));
-  if (!direct) {
-    OCR_HIP_CHECK(hipStreamWaitEvent(sb, f->entry_valid[oldest] ? f->entry[oldest] : f->entry[b], 0));
-    if (f->out[b].direct) OCR_HIP_CHECK(hipStreamWaitEvent(sb, f->done[b]->ev, 0));
-  }
-  f->out[b].direct = direct;
+  OCR_HIP_CHECK(hipStreamWaitEvent(sb, f->entry_valid[oldest] ? f->entry[oldest] : f->entry[b], 0));
   // and the scene's last stream-ordered descriptor update; the render reads
   // the current geometry version, registered as its reader below
   std::lock_guard<std::mutex> lk(s->ver_mu);
@@ -1188,11 +1148,7 @@ int ocr_render(ocr_scene* s, const ocr_view* view, ocr_frame* f, void* stream) {
   if (prof_shade) OCR_HIP_CHECK(hipEventRecord(ev[5], sb));
   OCR_HIP_CHECK(hipEventRecord(f->done[b]->ev, sb));
   s->note_read(f->done[b], true);
-  if (!direct) OCR_HIP_CHECK(hipStreamWaitEvent(st, f->done[b]->ev, 0));
-  {
-    std::lock_guard<std::mutex> lc(f->ctx->mu);
-    f->ctx->last_render = f->done[b];
-  }
+  OCR_HIP_CHECK(hipStreamWaitEvent(st, f->done[b]->ev, 0));
   if (prof_shade) f->n_profiled++;
   f->rendered = true;
   return OCR_OK;
