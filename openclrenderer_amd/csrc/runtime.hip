@@ -790,18 +790,27 @@ static int ensure_shadow_lists(ocr_scene* s, uint32_t cap_cut) {
 
 // Lights per shadow prearrange launch.  The launch rasterises small pieces
 // itself and lists the large ones while the list has room (then rasterises
-// the rest too), so any list size is correct.  It holds one record per
-// triangle and light of a group in every partition, at most kShadowMaxRecords
-// (896 MB): half the triangles face a light, nearly all in one cube face, and
-// at most a tenth exceed the local limit in the scenes measured, so it does
-// not fill up (six records, as a triangle has at most, cost a 200,000-triangle
-// scene with four lights 940 MB of allocation).
+// the rest too, each by one wavefront), so any list size is correct, but a full
+// one is slow: a two-sided room around 16 lights takes 315 ms from 12 triangles
+// with room for one record per triangle and light in every partition, 0.80 ms
+// with room for all its pieces.
+// A triangle has at most six pieces per light (three cube faces, each cut in
+// two): every list of up to kShadowListFull records (64 MB) holds as many.
+// Beyond, triangles are many and small, or share the faces' texels: few reach
+// over a face's edge, and there are two records per triangle and light, at
+// most kShadowMaxRecords (896 MB).  Rooms of 12,288 triangles and 4 lights,
+// 196,608 and 16, 983,040 and 4 in 20 layers: 474 us, 3.23, 5.53 ms with one
+// record, 249 us, 2.98, 4.47 ms with 1.25, 2 or 6.  A scene of 200,000 triangles
+// with four lights keeps 109 MB.
 constexpr uint32_t kShadowGroup = 16;
+constexpr uint64_t kShadowListFull = 1u << 20;
 static uint32_t shadow_list_cap(uint32_t ntri, uint32_t nlights) {
   constexpr uint32_t kBlock = 256;   // triangles per shadow prearrange block
   const uint64_t blocks = ((uint64_t)ntri + kBlock - 1) / kBlock;
-  const uint64_t per_part = (blocks + kListParts - 1) / kListParts * std::min(ntri, kBlock) *
-                                std::min(std::max(nlights, 1u), kShadowGroup) + 64;
+  // triangles times lights of a partition
+  const uint64_t pairs = (blocks + kListParts - 1) / kListParts * std::min(ntri, kBlock) *
+                         std::min(std::max(nlights, 1u), kShadowGroup);
+  const uint64_t per_part = std::min(6 * pairs + 64, std::max(kShadowListFull / kListParts, 2 * pairs + 64));
   return (uint32_t)std::min<uint64_t>(per_part * kListParts, kShadowMaxRecords);
 }
 
