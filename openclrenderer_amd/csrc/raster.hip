@@ -1001,9 +1001,18 @@ constexpr uint32_t kChunkTarget = 8192;
 // samples; finding a chunk's first record reads ~150 lines of the list.  Up to
 // 8192 samples a chunk (16 lights, 4 M triangles: 90 M samples): 866 -> 815 us
 // alone, the whole pass 3.03 -> 2.94 ms; 4096: 805 us, 2.98 ms.
+// They begin to grow at twice the camera's chunks, two to four per resident
+// wavefront: large triangles' chunks differ in what they cover, and with one or
+// less per wavefront the longest set the pass's time (a two-sided room of
+// 12,288 triangles around 4 lights 249 -> 236 us a pass, of 768 355 -> 341;
+// passes of more samples have kShadowChunkLog2 either way).
 constexpr int kShadowChunkLog2 = 13;
-__device__ __forceinline__ int chunk_log2(uint32_t units, int most) {   // units of 2^kChunkMinLog2 samples
-  return min(kChunkMinLog2 + (units > kChunkTarget ? 32 - __clz((int)((units - 1u) / kChunkTarget)) : 0), most);
+constexpr uint32_t kShadowChunkTarget = 16384;
+template <RasterMode kMode>
+__device__ __forceinline__ int chunk_log2(uint32_t units) {   // units of 2^kChunkMinLog2 samples
+  constexpr uint32_t kTarget = kMode == RasterMode::Shadow ? kShadowChunkTarget : kChunkTarget;
+  constexpr int kMost = kMode == RasterMode::Shadow ? kShadowChunkLog2 : kChunkLog2;
+  return min(kChunkMinLog2 + (units > kTarget ? 32 - __clz((int)((units - 1u) / kTarget)) : 0), kMost);
 }
 
 template <RasterMode kMode, int kOp, bool kBatch>
@@ -1043,7 +1052,7 @@ __global__ void __launch_bounds__(256) k_raster(PassArgs a, ShadowTarget sh) {
       }
     }
   }
-  const int clog = chunk_log2(units, kMode == RasterMode::Shadow ? kShadowChunkLog2 : kChunkLog2);
+  const int clog = chunk_log2<kMode>(units);
   const uint32_t part_chunks = wave_incl_scan((part_total >> clog) + ((part_total & ((1u << clog) - 1u)) ? 1u : 0u));
   const uint32_t nchunks = wave_total(part_chunks);
   const uint32_t csize = 1u << clog;
