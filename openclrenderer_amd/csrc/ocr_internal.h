@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <atomic>
 #include <memory>
 #include <mutex>
@@ -344,6 +345,7 @@ struct WorkState {
 // An event that outlives whichever of its holders ends first.
 struct Event {
   hipEvent_t ev = nullptr;
+  std::atomic<bool> over{false};   // what recorded it is gone, and its work finished
   Event() = default;
   Event(const Event&) = delete;
   Event& operator=(const Event&) = delete;
@@ -445,6 +447,8 @@ struct Scene {
   std::vector<Reader> map_readers[2];
   hipStream_t sh_stream = nullptr;
   static void note_into(std::vector<Reader>& list, const Reader& ev) {
+    // frames that are gone leave nothing to wait for
+    list.erase(std::remove_if(list.begin(), list.end(), [](const Reader& r) { return r->over.load(); }), list.end());
     // an event recorded again stands for its last recording
     for (const Reader& r : list)
       if (r == ev) return;

@@ -994,6 +994,7 @@ void ocr_frame_destroy(ocr_frame* f) {
   }
   dev_free(f->post_in);
   for (int b = 0; b < Frame::kSets; b++) {
+    if (f->done[b]) f->done[b]->over = true;   // freeing its buffers waited for its renders
     if (f->ss[b]) (void)hipStreamDestroy(f->ss[b]);
     if (f->entry[b]) (void)hipEventDestroy(f->entry[b]);
   }
