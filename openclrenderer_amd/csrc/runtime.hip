@@ -353,15 +353,18 @@ static void pack_obj(const ocr_obj_desc& s, ObjDesc& d) {
 }
 
 constexpr uint32_t kSplitChunk = 400000;   // 57.6 MB of staging
+constexpr uint32_t kSplitLeast = 1024;     // where the device has no room for it
 static_assert(kSplitChunk * sizeof(ocr_triangle) <= Ctx::kStageBytes, "staging");
 
-// The context's staging buffer with room for `bytes` (stage_mu held).
-static int stage_buffer(Ctx* c, size_t bytes, uint8_t** out) {
+// The context's staging buffer with room for `bytes`, or where the device has no
+// such room for as much as there is, at least `least` (stage_mu held); bytes:
+// out, how much it is.
+static int stage_buffer(Ctx* c, size_t& bytes, size_t least, uint8_t** out) {
   if (c->stage_bytes < bytes) {
     dev_free(c->stage);
     c->stage_bytes = 0;
-    const int rc = dev_alloc(&c->stage, bytes, "upload staging");
-    if (rc) return rc;
+    for (int rc; (rc = dev_alloc(&c->stage, bytes, "upload staging")); bytes = std::max(bytes / 2, least))
+      if (bytes <= least) return rc;
     c->stage_bytes = bytes;
   }
   *out = c->stage;
@@ -407,13 +410,15 @@ int ocr_scene_create(ocr_ctx* ctx, const ocr_triangle* tris, uint32_t ntri, cons
   if (ntri) {
     std::lock_guard<std::mutex> lk(ctx->stage_mu);
     uint8_t* stage = nullptr;
-    if ((rc = stage_buffer(ctx, sizeof(ocr_triangle) * (size_t)std::min<uint32_t>(ntri, kSplitChunk), &stage))) {
+    size_t bytes = sizeof(ocr_triangle) * (size_t)std::min<uint32_t>(ntri, kSplitChunk);
+    if ((rc = stage_buffer(ctx, bytes, std::min(bytes, sizeof(ocr_triangle) * (size_t)kSplitLeast), &stage))) {
       ocr_scene_destroy(s);
       return rc;
     }
     ocr_triangle* const staged = reinterpret_cast<ocr_triangle*>(stage);
-    for (uint32_t t = 0; t < ntri && e == hipSuccess; t += kSplitChunk) {
-      const uint32_t n = std::min<uint32_t>(kSplitChunk, ntri - t);
+    const uint32_t chunk = (uint32_t)(bytes / sizeof(ocr_triangle));
+    for (uint32_t t = 0; t < ntri && e == hipSuccess; t += chunk) {
+      const uint32_t n = std::min<uint32_t>(chunk, ntri - t);
       e = hipMemcpy(staged, tris + t, sizeof(ocr_triangle) * (size_t)n, hipMemcpyHostToDevice);
       if (e == hipSuccess) e = launch_split(staged, n, s->tri_pos + t, s->tri_attr + t, nullptr);
     }
@@ -644,24 +649,26 @@ int ocr_atlas_upload(ocr_scene* s, const ocr_tex_src* texs, uint32_t ntex) {
   OCR_HIP_CHECK(hipMemcpy(a.tex, desc.data(), sizeof(TexDesc) * desc.size(), hipMemcpyHostToDevice));
   OCR_HIP_CHECK(hipMemcpy(a.sizes, sizes.data(), sizeof(uint32_t) * a.nsizes, hipMemcpyHostToDevice));
   // texture::update_me_to_gpu + update_gpu_mipmaps (texture.cpp:323-493), in
-  // groups of at most kAtlasGroup textures and kAtlasStage bytes (a texture
-  // has at most 16 MiB).
-  constexpr size_t kAtlasStage = Ctx::kStageBytes;
+  // groups of at most kAtlasGroup textures and `limit` bytes (a texture has at
+  // most 16 MiB).
+  size_t limit = Ctx::kStageBytes;
   auto bytes_of = [&](uint32_t t) { return ((size_t)texs[t].width * texs[t].height * 4 + 255) / 256 * 256; };
   auto group_end = [&](uint32_t t, size_t& bytes) {
     uint32_t e = t;
-    for (bytes = 0; e < ntex && e - t < kAtlasGroup && (e == t || bytes + bytes_of(e) <= kAtlasStage); e++)
+    for (bytes = 0; e < ntex && e - t < kAtlasGroup && (e == t || bytes + bytes_of(e) <= limit); e++)
       bytes += bytes_of(e);
     return e;
   };
-  size_t max_bytes = 0, bytes = 0;
+  size_t max_bytes = 0, one = 0, bytes = 0;
+  for (uint32_t t = 0; t < ntex; t++) one = std::max(one, bytes_of(t));
   for (uint32_t t = 0; t < ntex;) {
     t = group_end(t, bytes);
     max_bytes = std::max(max_bytes, bytes);
   }
   std::lock_guard<std::mutex> stage_lock(s->ctx->stage_mu);
   uint8_t* staging = nullptr;
-  if (ntex && (rc = stage_buffer(s->ctx, max_bytes, &staging))) return rc;
+  if (ntex && (rc = stage_buffer(s->ctx, max_bytes, one, &staging))) return rc;
+  limit = max_bytes;
   hipStream_t st = nullptr;
   int status = OCR_OK;
   for (uint32_t t = 0; t < ntex && status == OCR_OK;) {
@@ -906,11 +913,12 @@ static int read_maps(Scene* s, const uint32_t* maps, uint32_t n, uint32_t* out) 
   }
   constexpr size_t kPart = 16u << 20;
   const size_t strip = (size_t)4 * L, strips = total / strip;   // four rows each
-  const size_t part = std::min(strips, kPart / (strip * 4));
   std::lock_guard<std::mutex> lk(s->ctx->stage_mu);
   uint8_t* stage = nullptr;
-  const int rc = stage_buffer(s->ctx, part * strip * 4, &stage);
+  size_t bytes = std::min(strips, kPart / (strip * 4)) * strip * 4;
+  const int rc = stage_buffer(s->ctx, bytes, strip * 4, &stage);
   if (rc) return rc;
+  const size_t part = bytes / (strip * 4);
   uint32_t* const rows = reinterpret_cast<uint32_t*>(stage);
   for (size_t i = 0; i < strips; i += part) {
     const size_t k = std::min(part, strips - i);

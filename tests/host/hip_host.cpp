@@ -38,7 +38,7 @@ std::map<const void*, void*> g_vars;
 std::map<void*, size_t> g_mem;
 std::string g_log;
 int g_next = 1, g_fail_launch = -1;
-size_t g_largest_malloc = ~(size_t)0, g_bytes = 0;
+size_t g_room = ~(size_t)0, g_bytes = 0;
 hipError_t g_last = hipSuccess;
 struct { dim3 grid, block; size_t shared; hipStream_t st; } g_call;
 
@@ -61,8 +61,8 @@ const char* host_log() { return g_log.c_str(); }
 void host_clear() { LOCK; g_log.clear(); }
 // The n-th launch from now fails (0: the next); -1: none.
 void host_fail_launch(int n) { g_fail_launch = n; }
-// Device allocations above `bytes` fail.
-void host_limit_malloc(size_t bytes) { g_largest_malloc = bytes; }
+// Device allocations that take more than `bytes` from now on fail.
+void host_limit_device(size_t bytes) { g_room = bytes == ~(size_t)0 ? bytes : g_bytes + bytes; }
 size_t host_device_bytes() { return g_bytes; }
 int host_live_events() { return (int)g_events.size(); }
 // A held stream's work is not finished until it is let go.
@@ -120,7 +120,7 @@ hipError_t hipMemGetInfo(size_t* f, size_t* t) { *f = *t = (size_t)288 << 30; re
 
 hipError_t hipMalloc(void** p, size_t n) {
   LOCK;
-  *p = n > g_largest_malloc ? nullptr : reserve(n);
+  *p = g_bytes + n > g_room ? nullptr : reserve(n);
   if (!*p) return bad(hipErrorOutOfMemory);
   g_mem[*p] = n;
   g_bytes += n;

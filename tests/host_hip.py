@@ -15,7 +15,7 @@ import numpy as np
 H = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
 H.host_log.restype = C.c_char_p
 H.host_device_bytes.restype = C.c_size_t
-H.host_limit_malloc.argtypes = [C.c_size_t]
+H.host_limit_device.argtypes = [C.c_size_t]
 for f in ("host_hold", "host_capture"):
     getattr(H, f).argtypes = [C.c_void_p, C.c_int]
 H.host_stream_id.argtypes = [C.c_void_p]
