@@ -75,3 +75,31 @@ def test_noalloc_into_unaligned_buffers(gpu_ctx, shift):
         hip.hipFree(b)
     for x in (fr, g):
         x.close()
+
+
+@pytest.mark.parametrize("tiles", [0, 1])
+def test_empty_scenes_in_a_row(gpu_ctx, tiles):
+    """Scenes without triangles and with none in view, between others."""
+    w, h = 161, 97
+    view = scenes.make_view(w, h, (0.0, 0.0, -10.0), hfov=70.0)
+    away = scenes.make_view(w, h, (0.0, 0.0, -4.0e5), c_rot=(0.0, np.pi, 0.0), hfov=70.0)
+    full, _ = scenes.random_scene(44, n_tris=300)
+    none, _ = scenes.random_scene(45, n_tris=30)
+    none.tris = none.tris[:0]
+    gs = [runtime.GpuScene(gpu_ctx, s) for s in (full, none)]
+    fr = runtime.Frame(gpu_ctx, w, h)
+    if tiles:
+        fr.set_raster(runtime.RASTER_TILES, 4, 4)
+    ref, st = fr.render_read(gs[0], view), fr.stats()
+    assert st["n_cut"] > 0 and np.count_nonzero(ref["tri_id"] != 0xFFFFFFFF) > 0
+    for k in range(9):
+        for g, v in ((gs[1], view), (gs[0], away))[: 1 + k % 2]:
+            out, e = fr.render_read(g, v), fr.stats()
+            assert (e["n_cut"], e["n_frag"]) == (0, 0), k
+            assert (out["tri_id"] == 0xFFFFFFFF).all() and (out["depth"] == 0xFFFFFFFF).all(), k
+        out, e = fr.render_read(gs[0], view), fr.stats()
+        for n in ("depth", "tri_id", "rgba", "normals"):
+            assert np.array_equal(out[n], ref[n]), (k, n)
+        assert (e["n_cut"], e["n_frag"]) == (st["n_cut"], st["n_frag"]), k
+    for x in [fr] + gs:
+        x.close()
