@@ -89,11 +89,12 @@ static PassArgs batch_pass(const ocr_batch* b) {
   a.tiles = b->tiles;
   a.tile_w_log2 = b->tune.shade_tile_w_log2;
   a.unshadowed = 1u;
+  const uint32_t cap = list_used(a.tri_slots, b->cap_cut);
   for (const Scene* s : b->scenes) {
     if (s->n_shadow) a.unshadowed = 0u;
-    if (needs_far(*s, b->cap_cut)) a.far = 1u;
+    if (needs_far(*s, cap)) a.far = 1u;
   }
-  a.lists = make_lists(b->cuts, b->counters, b->cap_cut, b->tune.raster_tile ? 1u : list_parts(b->tri_slots, b->cap_cut),
+  a.lists = make_lists(b->cuts, b->counters, cap, b->tune.raster_tile ? 1u : list_parts(b->tri_slots, cap),
                        b->tune.raster_tile != 0);
   a.lists.ent = b->ent;
   if (b->tune.raster_tile) a.lists.tb = b->tb;

@@ -314,6 +314,13 @@ inline uint64_t list_capacity(uint64_t tri_slots) {
   const uint64_t blocks = (tri_slots + kPreThreads - 1) / kPreThreads;
   return (blocks + (blocks >= 64 ? kListParts : 1)) * 2 * kPreThreads;
 }
+// Records of a list of cap_cut that a render of tri_slots uses: one that is
+// larger, from an earlier render or a server's reservation, does not spread the
+// partitions over all of it, beyond where 32-bit offsets reach (needs_far).
+inline uint32_t list_used(uint32_t tri_slots, uint32_t cap_cut) {
+  const uint64_t most = list_capacity(tri_slots);
+  return most < cap_cut ? (uint32_t)most : cap_cut;
+}
 // Bits of the overflow word: the cut list is full / the sample space is full.
 constexpr uint32_t kOverflowCuts = 1u, kOverflowSamples = 2u, kOverflowBins = 4u;
 // Raster samples per render, and per cut triangle.  Frames and shadow faces

@@ -173,10 +173,10 @@ static PassArgs single_pass(const Scene* s, const ocr_view* view, Frame* f) {
   a.tiles = view_tiles(view->width, view->height, a.tile_w_log2);
   const Frame::OutBuf& ob = f->out[f->cur];
   const bool tiled = f->raster_mode == OCR_RASTER_TILES;
-  a.lists = make_lists(ob.cuts, ob.counters, ob.cap_cut,
-                       tiled || f->want_cut ? 1u : list_parts(a.tri_slots, ob.cap_cut), tiled);
+  const uint32_t cap = f->want_cut ? ob.cap_cut : list_used(a.tri_slots, ob.cap_cut);
+  a.lists = make_lists(ob.cuts, ob.counters, cap, tiled || f->want_cut ? 1u : list_parts(a.tri_slots, cap), tiled);
   a.lists.ent = ob.ent;
-  a.far = needs_far(*s, ob.cap_cut) ? 1u : 0u;
+  a.far = needs_far(*s, cap) ? 1u : 0u;
   if (f->raster_mode == OCR_RASTER_TILES && ob.tb.bin) {
     a.lists.tb = ob.tb;
     a.view0.bin_begin = 0;

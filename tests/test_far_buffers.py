@@ -41,6 +41,23 @@ H.host_clear(); b.launch_graph(); print("graph", *[k for k in kernels(log()) if 
     assert "k_shade_batch_unshadowed" in lines[2] and "k_shade_batch_far" in lines[3], out
 
 
+def test_small_views_in_a_large_list(tmp_path):
+    """A list that grew beyond 4 GiB serves small renders from its front."""
+    out = host_hip.run(tmp_path, GROUND + """
+sc, view = scenes.random_scene(3)
+sc.tris = np.repeat(sc.tris[:1], 1 << 20)
+g = runtime.GpuScene(ctx, sc)
+frames = [runtime.Frame(ctx, 64, 48) for _ in range(64)]
+b = runtime.Batch(ctx, 64)
+for n in (64, 63, 1):
+    b.set_views([g] * n, [view] * n, frames[:n])
+    print(n, *shading(b.render), *[k for k in shading(b.launch_graph) if "shade" in k])
+""")
+    lines = out.split("\n")
+    assert lines[0].count("k_shade_batch_far") == 2, out
+    assert lines[1].count("k_shade_batch_unshadowed") == lines[2].count("k_shade_batch_unshadowed") == 2, out
+
+
 def test_atlas_and_map_variants(tmp_path):
     out = host_hip.run(tmp_path, GROUND + """
 rgba = np.zeros((2048, 2048, 4), np.uint8)
