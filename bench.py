@@ -97,7 +97,7 @@ def profile_entry(kernel, workload):
 
 def calibration():
     """Measured ceilings on this GPU (calib.hip): the VALU issue rate of
-    independent binary32 and binary64 FMA chains at 8 wavefronts per SIMD,
+    independent binary32 multiplies and adds and binary64 fmas at 8 wavefronts per SIMD,
     and the u32 atomicMin rate on a 1080p-sized buffer, uniform random and
     64-address clusters (the depth pass's neighbourhoods)."""
     cal = C.CDLL(os.path.join(ROOT, "openclrenderer_amd", "libocr_calib.so"))
@@ -105,8 +105,8 @@ def calibration():
     cal.ocr_calib_valu.restype = C.c_double
     cal.ocr_calib_atomics.argtypes = [C.c_int, C.c_uint32, C.c_size_t, C.c_uint32, C.c_int]
     cal.ocr_calib_atomics.restype = C.c_double
-    f32 = cal.ocr_calib_valu(0, 4096)
-    f64 = cal.ocr_calib_valu(1, 4096)
+    f32 = cal.ocr_calib_valu(0, 1024)
+    f64 = cal.ocr_calib_valu(1, 1024)
     n = 1 << 26
     words = 1920 * 1080
     us_rand = cal.ocr_calib_atomics(0, words, n, 1, 5)
@@ -435,7 +435,7 @@ def run_plain(args):
         n = float(prof["valu_insts_per_launch"])
         peak = cal["valu_f32_wave_insts_per_s"]
         valu = {"insts_per_launch": n, "peak_insts_per_s": peak,
-                "peak_source": "measured: independent binary32 FMA chains, 8 wavefronts per SIMD (calib.hip)",
+                "peak_source": "measured: independent binary32 multiplies and adds, 8 wavefronts per SIMD (calib.hip)",
                 "frac": n / (st["ms_shade"] * 1e-3) / peak,
                 "frac_isolated": n / (st_iso["ms_shade"] * 1e-3) / peak}
 
