@@ -804,11 +804,12 @@ static int ensure_shadow_lists(ocr_scene* s, uint32_t cap_cut) {
 // A triangle has at most six pieces per light (three cube faces, each cut in
 // two): every list of up to kShadowListFull records (64 MB) holds as many.
 // Beyond, triangles are many and small, or share the faces' texels: few reach
-// over a face's edge, and there are two records per triangle and light, at
-// most kShadowMaxRecords (896 MB).  Rooms of 12,288 triangles and 4 lights,
-// 196,608 and 16, 983,040 and 4 in 20 layers: 474 us, 3.23, 5.53 ms with one
-// record, 249 us, 2.98, 4.47 ms with 1.25, 2 or 6.  A scene of 200,000 triangles
-// with four lights keeps 109 MB.
+// over a face's edge, and there are three records for two triangles and a
+// light, at most kShadowMaxRecords (896 MB).  Rooms of 12,288 triangles and 4
+// lights, 196,608 and 16, 983,040 and 4 in 20 layers: 474 us, 3.23, 5.53 ms with
+// one record, 249 us, 2.98, 4.47 ms with 1.25, 1.5, 2 or 6; the allocation costs
+// a scene's first pass 1.4 us per MB.  A scene of 200,000 triangles with four
+// lights keeps 82 MB.
 constexpr uint32_t kShadowGroup = 16;
 constexpr uint64_t kShadowListFull = 1u << 20;
 static uint32_t shadow_list_cap(uint32_t ntri, uint32_t nlights) {
@@ -817,7 +818,7 @@ static uint32_t shadow_list_cap(uint32_t ntri, uint32_t nlights) {
   // triangles times lights of a partition
   const uint64_t pairs = (blocks + kListParts - 1) / kListParts * std::min(ntri, kBlock) *
                          std::min(std::max(nlights, 1u), kShadowGroup);
-  const uint64_t per_part = std::min(6 * pairs + 64, std::max(kShadowListFull / kListParts, 2 * pairs + 64));
+  const uint64_t per_part = std::min(6 * pairs + 64, std::max(kShadowListFull / kListParts, pairs + pairs / 2 + 64));
   return (uint32_t)std::min<uint64_t>(per_part * kListParts, kShadowMaxRecords);
 }
 

@@ -1,7 +1,7 @@
 """The shadow pass's list (runtime.hip, shadow_list_cap): what does not fit is
 drawn by single wavefronts, so every list of a small scene holds the six pieces
 a triangle can have per light, whichever partition they fall in, and a larger
-one two records per triangle and light.  Allocations over the stand-in for the
+one three for two triangles and a light.  Allocations over the stand-in for the
 HIP runtime; and the maps of a room whose pieces all are large against the
 oracle."""
 import numpy as np
@@ -14,7 +14,7 @@ MB = 1 << 20
 
 @pytest.mark.parametrize("ntri,lights,least,most", [
     (1, 1, 6, 1), (12, 16, 6, 6), (48, 17, 6, 20), (768, 4, 6, 65), (12288, 4, 4, 65), (16384, 16, 3, 65),
-    (200_000, 4, 2, 110), (300_000, 3, 2, 120), (1_000_000, 16, 0.8, 897)])
+    (200_000, 4, 1.5, 83), (300_000, 3, 1.5, 91), (1_000_000, 16, 0.8, 897)])
 def test_room_for_the_pieces(tmp_path, ntri, lights, least, most):
     out = host_hip.run(tmp_path, f"""
 ctx = runtime.Context(0)
