@@ -37,10 +37,11 @@ namespace ocr {
 // Cut records and sample ranges are allocated once per block (one 64-bit
 // atomicAdd on the packed counter (cuts << 32 | samples) of the block's
 // partition).  The next render's prearrange runs beside the current render's
-// shading, whose wavefronts hold 440 of a SIMD's 512 registers: a block of four
-// wavefronts with at most 72 registers finds room on a CU at once, where a
-// block of eight with 90 waited until the CU had drained (prearrange 36 us
-// alone, 200-260 us beside shading).  With the counters zeroed by the clear
+// shading, whose wavefronts fill most of a SIMD's registers (five of 88 when this
+// was measured, six of 80 now): a block of four wavefronts with at most 72
+// finds room on a CU at once or as soon as one of them ends, where a block of
+// eight with 90 waited until the CU had drained (prearrange 36 us alone,
+// 200-260 us beside shading).  With the counters zeroed by the clear
 // and pieces that cover nothing left out: 1280x719, 120,000 triangles
 // 88.8 -> 81.0 us, 1080p, 1 M triangles 194.8 -> 188.2, the 16-light 4K frame
 // 5.00 -> 4.88 ms.

@@ -721,10 +721,10 @@ __global__ void __launch_bounds__(256) k_shade_batch_far(ShadeLaunch sl) {
 }
 
 // Passes whose scenes have no shadow-casting light: without the occlusion
-// code the kernel takes 79 VGPRs, five wavefronts per SIMD instead of the
+// code the kernel takes 79 VGPRs, six wavefronts per SIMD instead of the
 // four of the general kernel's 113, which hides more of its gathers and
 // leaves room for the next render's raster passes (1080p, 1 M triangles,
-// 4 lights, five wavefronts against three: shading alone 124 -> 108 us).
+// 4 lights, when these were five against three: shading alone 124 -> 108 us).
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_shade_unshadowed(ShadeLaunch sl) {
   shade_pixel<false, false, false, false>(sl);
   zero_work(sl.p.lists);
